@@ -342,7 +342,9 @@ bdh_status run_attention_vjp(const VjpArgs& a, hipStream_t st, uint64_t* launche
     g.B = G; g.sBo = H * T * D; g.sBi = T * D; g.sBn = 1; g.sBk = D;
     g.C = gvt; g.sCo = H * gvt_stride; g.sCi = gvt_stride; g.sCm = D; g.sCn = 1;
     g.M = (int)L; g.N = (int)D; g.K = (int)L;
+    g.klow = 1;
     BDH_HIP_TRY(gemm<E_STORE>(g, S, st, part, pe, &n));
+    g.klow = 0;
     if (rho_iv) {
       // IC = (Q rho_iv) * d^t  (the decay gradient's state term)
       g.A = Q; g.sAo = H * T * N; g.sAi = T * N; g.sAm = N; g.sAk = 1;
