@@ -50,14 +50,16 @@ enum Epi {
   E_ROWSCALE,      // C = acc * d^m
   E_ROWSCALE_ACC,  // C += acc * d^m
   E_CARRY,         // C = acc + src * d^kpow (src null: acc)
-  E_ROWREV_ACC     // C += acc * d^(kpow - m)
+  E_ROWREV_ACC,    // C += acc * d^(kpow - m)
+  E_SYM_DECAY      // C(m, n) = C(n, m) = acc * d^(m-n) for n < m, C(m, m) = 0; and the decay gradient's
+                   // terms ((acc * (m-n)) * src(m, n)) / sd of n < m, summed per tile into dpart
 };
 
 struct GemmF32 {
   const float* A;
   const float* B;
   float* C;
-  const float* src;     // E_CARRY: addend with C's strides (may equal C)
+  const float* src;     // E_CARRY: addend with C's strides (may equal C); E_SYM_DECAY: the scores, or null (no terms)
   int64_t sAo, sAi, sAm, sAk;   // sAm or sAk is 1
   int64_t sBo, sBi, sBn, sBk;   // sBn or sBk is 1
   int64_t sCo, sCi, sCm, sCn;
@@ -69,6 +71,9 @@ struct GemmF32 {
   float* part;          // split-K partials [ksplit, batch, M, N] (ksplit > 1)
   int ksplit;
   int64_t batch;
+  double* dpart;        // E_SYM_DECAY: tile sums [batch, dslots]
+  int dslots, dacc;     // (dacc: added to what is there)
+  int recurrent_eps;    // E_SYM_DECAY: the recurrent backward's decay guard
   int tri;              // masked square product: only the 128 x 128 blocks on or below the diagonal are computed
 };
 
@@ -77,6 +82,23 @@ constexpr int TRI = 128;             // edge of the blocks a masked product is c
 constexpr int DSCALE = 1024;         // KSCALE: most k of one workgroup (LDS table of d^(kpow - k))
 
 __device__ __forceinline__ float dpowf(float d, int e) { return powf(d, (float)e); }
+
+// The divisor of the decay gradient: the reference's two guards against 0.
+__device__ __forceinline__ float decay_sd(float d, int recurrent_eps) {
+  if (recurrent_eps) return (d < 1e-8f && d > -1e-8f) ? 1e-8f : d;
+  return d + 1e-12f;
+}
+
+// Sum of a workgroup's 256 values in a fixed order, in thread 0.
+__device__ __forceinline__ double block_sum(double v, double* red) {
+  red[threadIdx.x] = v;
+  __syncthreads();
+  for (int o = 128; o > 0; o >>= 1) {
+    if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
+    __syncthreads();
+  }
+  return red[0];
+}
 
 // The epilogue's addend: C itself (the accumulating kinds), src (E_CARRY),
 // or none.
@@ -215,7 +237,7 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
   // share the longer operand's rows then run together on one L2.
   const int nwg = (int)gridDim.x, id = (int)blockIdx.x;
   int wk = (nwg & 7) ? id : (id & 7) * (nwg >> 3) + (id >> 3);
-  int tx, ty;
+  int tx, ty, slot = 0;
   int64_t z;
   if (g.tri) {
     // TRI-blocks (by, bx <= by) in row order, SUB tiles each.
@@ -223,8 +245,9 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
     const int nbk = (nty + ED - 1) / ED;
     const int per = nbk * (nbk + 1) / 2 * SUB;
     z = wk / per;
-    int r = (wk - (int)z * per) / SUB;
-    const int sub = (wk - (int)z * per) % SUB;
+    slot = wk - (int)z * per;
+    int r = slot / SUB;
+    const int sub = slot % SUB;
     ty = 0;
     while (r > ty) {
       r -= ty + 1;
@@ -232,7 +255,10 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
     }
     ty = ty * ED + sub / ED;
     tx = r * ED + sub % ED;
-    if (ty >= nty || tx >= ntx) return;
+    if (ty >= nty || tx >= ntx) {
+      if (EPI == E_SYM_DECAY && g.src && t == 0 && !g.dacc) g.dpart[z * g.dslots + slot] = 0.0;
+      return;
+    }
   } else if (ntx < nty) {
     tx = wk % ntx;
     wk /= ntx;
@@ -385,6 +411,42 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
   const float carry = (EPI == E_CARRY && g.decay) ? dpowf(d, g.kpow) : 1.0f;
   float* Pp = P > 1 ? g.part + ((int64_t)kp * g.batch + b) * (int64_t)g.M * g.N : nullptr;
   float* C = g.C + bo * g.sCo + bi * g.sCi;
+  if constexpr (EPI == E_SYM_DECAY) {
+    const float* SC = g.src ? g.src + bo * g.sCo + bi * g.sCi : nullptr;
+    const float sd = decay_sd(d, g.recurrent_eps);
+    double sum = 0.0;
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        const int n = nw + 32 * j + acc_col(lane);
+        float x[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int m = mw + 32 * i + acc_row(lane, r);
+          x[r] = SC && m < g.M && n < m ? SC[(int64_t)m * g.sCm + n] : 0.0f;
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int m = mw + 32 * i + acc_row(lane, r);
+          if (m >= g.M || n > m) continue;
+          const float v = n < m ? big[i][j][r] : 0.0f;
+          sum += (double)(((v * (float)(m - n)) * x[r]) / sd);
+          const float o = g.decay ? v * dpowf(d, m - n) : v;
+          C[(int64_t)m * g.sCm + n] = o;
+          C[(int64_t)n * g.sCm + m] = o;
+        }
+      }
+    if (SC) {
+      __syncthreads();
+      const double all = block_sum(sum, reinterpret_cast<double*>(lds));
+      if (t == 0) {
+        double* o = g.dpart + b * g.dslots + slot;
+        *o = g.dacc ? *o + all : all;
+      }
+    }
+    return;
+  }
   const float* X = P > 1 ? nullptr : epi_addend<EPI>(g, bo, bi);
   const bool whole = m0 + BT <= g.M && n0 + BT <= g.N;
 #pragma unroll
@@ -501,6 +563,15 @@ hipError_t launch_gemm(const GemmF32& g, int64_t nwg, hipStream_t st) {
   return hipGetLastError();
 }
 
+// A product runs on 64 x 64 tiles while its 128 x 128 ones leave CUs idle.
+inline bool small_tiles(int64_t tiles, int p) { return tiles * p < (int64_t)device_cus(); }
+
+// Tile sums an unsplit E_SYM_DECAY product of [L, L] writes per batch.
+inline int sym_slots(int64_t batch, int L) {
+  const int64_t tiles = tile_count(L, L, 128, true);
+  return (int)(small_tiles(tiles * batch, 1) ? tile_count(L, L, 64, true) : tiles);
+}
+
 // C = epilogue(A B^T) over `batch` products.  With `part` (part_elems floats)
 // a long K may be split; the partials need ksplit * batch * M * N floats.
 template <int EPI, bool KSCALE = false>
@@ -512,7 +583,8 @@ hipError_t gemm(GemmF32 g, int64_t batch, hipStream_t st, float* part = nullptr,
     if (g.K > DSCALE) return hipErrorInvalidValue;
   }
   g.batch = batch;
-  g.tri = (EPI == E_TRIL || EPI == E_TRIL_DECAY) && g.M == g.N;
+  g.tri = (EPI == E_TRIL || EPI == E_TRIL_DECAY || EPI == E_SYM_DECAY) && g.M == g.N;
+  if (EPI == E_SYM_DECAY && (!g.tri || part)) return hipErrorInvalidValue;
   const size_t per = (size_t)batch * (size_t)g.M * (size_t)g.N;
   const int64_t tiles = tile_count(g.M, g.N, 128, g.tri) * batch;
   int p = part ? split_k_ranges(tiles, g.K) : 1;
@@ -520,11 +592,11 @@ hipError_t gemm(GemmF32 g, int64_t batch, hipStream_t st, float* part = nullptr,
   if (p < 1) p = 1;
   g.ksplit = p;
   g.part = p > 1 ? part : nullptr;
-  const hipError_t e = tiles * p < (int64_t)device_cus()
+  const hipError_t e = small_tiles(tiles, p)
                            ? launch_gemm<EPI, KSCALE, 64>(g, tile_count(g.M, g.N, 64, g.tri) * batch * p, st)
                            : launch_gemm<EPI, KSCALE, 128>(g, tiles * p, st);
   if (e != hipSuccess) return e;
-  if (p > 1) {
+  if (p > 1 && EPI != E_SYM_DECAY) {
     const int n4 = (g.N + 3) / 4;
     hipLaunchKernelGGL(gemm_reduce_kernel<EPI>, dim3((unsigned)(((int64_t)g.M * n4 + 255) / 256), (unsigned)batch),
                        dim3(256), 0, st, g, n4);

@@ -41,10 +41,9 @@ enum ScratchSlot {
   SLOT_DECODE_IDX,   // decode range active lists    [S, N] int32
   SLOT_DECODE_CNT,   // decode range active counts   [S, G] int32
   SLOT_VJP_S,        // VJP scores tril(QQ^T) * D    [S, T, T] f32
-  SLOT_VJP_GS,       // VJP tril(G V^T)              [S, T, T] f32
-  SLOT_VJP_M,        // VJP GS*D + its transpose     [S, T, T] f32
+  SLOT_VJP_M,        // VJP tril(G V^T)*D + its transpose  [S, T, T] f32
   SLOT_VJP_TD,       // VJP per-head grad_v, IC, G*d^t  3 x [S, T, D] f32
-  SLOT_VJP_PART,     // VJP decay partials           [S] f64
+  SLOT_VJP_PART,     // VJP decay partial sums       [S, slots] f64
   SLOT_GEMM_PART,    // fp32 GEMM split-K partials   [P, batch, M, N] f32
   SLOT_VJP_RHO,      // VJP states at interval starts [n_iv - 1, S, N, D] f32
   SLOT_VJP_GAMMA,    // VJP state gradients          2 x [S, N, D] f32

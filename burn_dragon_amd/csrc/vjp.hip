@@ -7,12 +7,12 @@
 // context gradient, D[r, c] = d^(r-c) and gap = r - c below the diagonal, one
 // interval of L tokens starting from the state rho_iv gives
 //   S      = tril(-1)(Q Q^T) * D            [L, L]   gemm, TRIL_DECAY epilogue
-//   GS     = tril(-1)(G V^T)                [L, L]   gemm, TRIL epilogue
-//   M      = GS * D + (GS * D)^T            [L, L]   elementwise
-//   grad_q = M Q  [+ (G rho_iv^T) * d^t]    [L, N]   gemm (+ ROWSCALE_ACC)
-//   grad_v = S^T G                          [L, D]   gemm, heads summed for Hv = 1
+//   GS     = tril(-1)(G V^T),  M = GS * D + (GS * D)^T
+//                                           [L, L]   gemm, SYM_DECAY epilogue: writes M, and sums
 //   grad_d = sum((GS * gap) * S) / sd  [+ sum((G * IC) * t) / sd],
 //            IC = (Q rho_iv) * d^t                    gemm ROWSCALE + reduction
+//   grad_q = M Q  [+ (G rho_iv^T) * d^t]    [L, N]   gemm (+ ROWSCALE_ACC)
+//   grad_v = S^T G                          [L, D]   gemm over k >= m, heads summed for Hv = 1
 // Longer sequences run as intervals of at most 1024 tokens with the state
 // history and a reverse scan (the reference's recurrent backward does the
 // same per token): the states rho_iv are recomputed forward, then, from the
@@ -23,10 +23,10 @@
 //   grad_v += d^(L-t) (Q Gamma_{iv+1})        gemm P, then a scaled add
 //   grad_d += sum (L-t) d^(L-t) P V / sd + L d^L <rho_iv, Gamma_{iv+1}> / sd
 // and grad_rho0 = Gamma_0.
-// Every product is a batched fp32 GEMM on the fp32 MFMAs (exact fp32
-// products, fp32 accumulation; bdh_gemm_f32.h) with generic strides, so
-// transposed operands need no copy.  Reductions are per stream (f64) and then
-// per head in a fixed order: the result is deterministic.
+// Every product is a batched fp32 GEMM (bdh_gemm_f32.h) with generic strides,
+// so transposed operands need no copy.  The decay gradient's terms are summed
+// in f64 by tile or block into slots of their own, then per head in a fixed
+// order: the result is deterministic.
 #include "bdh_gemm_f32.h"
 
 namespace bdh {
@@ -40,88 +40,71 @@ using gf32::E_ROWREV_ACC;
 using gf32::E_ROWSCALE;
 using gf32::E_ROWSCALE_ACC;
 using gf32::E_STORE;
-using gf32::E_TRIL;
+using gf32::E_SYM_DECAY;
 using gf32::E_TRIL_DECAY;
+using gf32::block_sum;
+using gf32::decay_sd;
 
 constexpr int64_t kVjpInterval = 1024;  // tokens per interval of the reverse scan
-constexpr int kCrossBlocks = 64;        // workgroups per stream of the state-term reduction
-
-__device__ __forceinline__ float decay_sd(float d, int recurrent_eps) {
-  if (recurrent_eps) return (d < 1e-8f && d > -1e-8f) ? 1e-8f : d;
-  return d + 1e-12f;
-}
-
-// M[s, r, c] = W[r, c] + W[c, r], W[r, c] = r > c ? GS[r, c] d^(r - c) : 0,
-// over the leading L x L of ld x ld blocks.
-__global__ __launch_bounds__(256) void msym_kernel(const float* __restrict__ gs, float* __restrict__ m,
-                                                   const float* __restrict__ decay, int H, int L, int ld) {
-  const int64_t s = blockIdx.y;
-  const float d = decay ? decay[s % H] : 1.0f;
-  const float* G = gs + s * (int64_t)ld * ld;
-  float* Mo = m + s * (int64_t)ld * ld;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < (int64_t)L * L; i += (int64_t)gridDim.x * 256) {
-    const int r = (int)(i / L), c = (int)(i - (int64_t)r * L);
-    float v = 0.0f;
-    if (r > c) v = G[(int64_t)r * ld + c] * dpowf(d, r - c);
-    else if (c > r) v = G[(int64_t)c * ld + r] * dpowf(d, c - r);
-    Mo[(int64_t)r * ld + c] = v;
-  }
-}
+constexpr int kCrossBlocks = 64;        // workgroups per stream of the next state's decay terms
+constexpr int kStateBlocks = 16;        // and of the carried state's
 
 __global__ __launch_bounds__(256) void zero_f64_kernel(double* __restrict__ p, int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i < n) p[i] = 0.0;
 }
 
-// Adds stream s's decay-gradient terms of one interval to part[s], in the
-// reference's element op order: ((GS * gap) * S) / sd over the lower
-// triangle, plus, with a state, ((G * IC) * t) / sd over [L, D].  f64 sums,
-// fixed order.
-__global__ __launch_bounds__(256) void decay_partial_kernel(const float* __restrict__ gs,
-                                                            const float* __restrict__ sc, int ld,
-                                                            const float* __restrict__ g, int64_t g_stride,
-                                                            const float* __restrict__ ic,
-                                                            const float* __restrict__ decay, int H, int L,
-                                                            int D, int recurrent_eps,
-                                                            double* __restrict__ part) {
-  __shared__ double red[256];
-  const int64_t s = blockIdx.x;
-  const float sd = decay_sd(decay ? decay[s % H] : 1.0f, recurrent_eps);
-  double acc = 0.0;
-  const float* GS = gs + s * (int64_t)ld * ld;
-  const float* SC = sc + s * (int64_t)ld * ld;
-  for (int64_t i = threadIdx.x; i < (int64_t)L * L; i += 256) {
-    const int r = (int)(i / L), c = (int)(i - (int64_t)r * L);
-    if (r > c) acc += (double)(((GS[(int64_t)r * ld + c] * (float)(r - c)) * SC[(int64_t)r * ld + c]) / sd);
-  }
-  if (ic) {
-    const float* Gs = g + s * g_stride;
-    const float* I = ic + s * (int64_t)ld * D;
-    for (int64_t i = threadIdx.x; i < (int64_t)L * D; i += 256) {
-      const int t = (int)(i / D);
-      acc += (double)(((Gs[i] * I[i]) * (float)t) / sd);
+// Calls f(t, e, t * D + e) for this thread's share of tokens [lo, hi) and
+// columns [0, D): flat order, 256 apart, without a division per element.
+template <class F>
+__device__ __forceinline__ void each_te(int lo, int hi, int D, F&& f) {
+  const int dt = 256 / D, de = 256 - dt * D;
+  int t = lo + (int)threadIdx.x / D, e = (int)threadIdx.x % D;
+  while (t < hi) {
+    f(t, e, (int64_t)t * D + e);
+    t += dt;
+    e += de;
+    if (e >= D) {
+      e -= D;
+      ++t;
     }
   }
-  red[threadIdx.x] = acc;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) part[s] += red[0];
 }
 
-// The decay terms through the next state, per stream and block of a fixed
-// split: block j < kCrossBlocks sums L d^L rho_iv * Gamma / sd over its slice
-// of [N, D]; block kCrossBlocks sums (L - t) d^(L - t) P[t, e] V[t, e] / sd.
-// Results go to cpart[s, j] (f64), folded in order by cross_fold_kernel.
+// Adds (dacc) or sets the carried state's decay terms of one interval, in the
+// reference's element op order ((G * IC) * t) / sd over [L, D]: block j of
+// stream s sums its slice of the tokens into part[s * slots + j].
+__global__ __launch_bounds__(256) void decay_state_kernel(const float* __restrict__ g, int64_t g_stride,
+                                                          const float* __restrict__ ic, int ld,
+                                                          const float* __restrict__ decay, int H, int L, int D,
+                                                          int recurrent_eps, double* __restrict__ part,
+                                                          int slots, int dacc) {
+  __shared__ double red[256];
+  const int64_t s = blockIdx.y;
+  const float sd = decay_sd(decay ? decay[s % H] : 1.0f, recurrent_eps);
+  const int per = (L + kStateBlocks - 1) / kStateBlocks;
+  const int lo = blockIdx.x * per, hi = lo + per < L ? lo + per : L;
+  const float* Gs = g + s * g_stride;
+  const float* I = ic + s * (int64_t)ld * D;
+  double acc = 0.0;
+  each_te(lo, hi, D, [&](int t, int, int64_t i) { acc += (double)(((Gs[i] * I[i]) * (float)t) / sd); });
+  const double all = block_sum(acc, red);
+  if (threadIdx.x == 0) {
+    double* o = part + s * slots + blockIdx.x;
+    *o = dacc ? *o + all : all;
+  }
+}
+
+// Adds the decay terms through the next state: block j of stream s sums its
+// slice of L d^L rho_iv * Gamma / sd over [N, D] and of (L - t) d^(L - t)
+// P[t, e] V[t, e] / sd over the tokens into part[s * slots + j].
 __global__ __launch_bounds__(256) void decay_cross_kernel(const float* __restrict__ p, int ld,
                                                           const float* __restrict__ v, int64_t sVo,
                                                           int64_t sVi, const float* __restrict__ rho,
                                                           const float* __restrict__ gamma,
                                                           const float* __restrict__ decay, int H, int L,
                                                           int64_t ND, int D, int recurrent_eps,
-                                                          double* __restrict__ cpart) {
+                                                          double* __restrict__ part, int slots) {
   __shared__ double red[256];
   const int64_t s = blockIdx.y;
   const int j = blockIdx.x;
@@ -129,49 +112,36 @@ __global__ __launch_bounds__(256) void decay_cross_kernel(const float* __restric
   const float d = decay ? decay[h] : 1.0f;
   const float sd = decay_sd(d, recurrent_eps);
   double acc = 0.0;
-  if (j < kCrossBlocks) {
-    if (rho) {
-      const float w = (float)L * dpowf(d, L);
-      const int64_t per = (ND + kCrossBlocks - 1) / kCrossBlocks;
-      const int64_t lo = j * per, hi = lo + per < ND ? lo + per : ND;
-      const float* R = rho + s * ND;
-      const float* Gm = gamma + s * ND;
-      for (int64_t i = lo + threadIdx.x; i < hi; i += 256) acc += (double)((R[i] * Gm[i]) * w / sd);
-    }
-  } else {
-    const float* P = p + s * (int64_t)ld * D;
-    const float* V = v + b * sVo + h * sVi;
-    for (int64_t i = threadIdx.x; i < (int64_t)L * D; i += 256) {
-      const int t = (int)(i / D);
-      acc += (double)(((P[i] * V[i]) * ((float)(L - t) * dpowf(d, L - t))) / sd);
-    }
+  if (rho) {
+    const float w = (float)L * dpowf(d, L);
+    const int64_t per = (ND + kCrossBlocks - 1) / kCrossBlocks;
+    const int64_t lo = j * per, hi = lo + per < ND ? lo + per : ND;
+    const float* R = rho + s * ND;
+    const float* Gm = gamma + s * ND;
+    for (int64_t i = lo + threadIdx.x; i < hi; i += 256) acc += (double)((R[i] * Gm[i]) * w / sd);
   }
-  red[threadIdx.x] = acc;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) cpart[s * (kCrossBlocks + 1) + j] = red[0];
+  const int per = (L + kCrossBlocks - 1) / kCrossBlocks;
+  const int lo = j * per, hi = lo + per < L ? lo + per : L;
+  const float* P = p + s * (int64_t)ld * D;
+  const float* V = v + b * sVo + h * sVi;
+  each_te(lo, hi, D, [&](int t, int, int64_t i) {
+    acc += (double)(((P[i] * V[i]) * ((float)(L - t) * dpowf(d, L - t))) / sd);
+  });
+  const double all = block_sum(acc, red);
+  if (threadIdx.x == 0) part[s * slots + j] += all;
 }
 
-__global__ __launch_bounds__(256) void cross_fold_kernel(const double* __restrict__ cpart,
-                                                         double* __restrict__ part, int64_t S) {
-  const int64_t s = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (s >= S) return;
-  double acc = 0.0;
-  for (int j = 0; j <= kCrossBlocks; ++j) acc += cpart[s * (kCrossBlocks + 1) + j];
-  part[s] += acc;
-}
-
-// grad_decay[h] = sum over batch (in order) of the stream partials.
-__global__ __launch_bounds__(256) void decay_final_kernel(const double* __restrict__ part,
+// grad_decay[h] = sum over batch and slots of the partial sums: one workgroup
+// a head, its threads' and then their sums in a fixed order.
+__global__ __launch_bounds__(256) void decay_final_kernel(const double* __restrict__ part, int slots,
                                                           float* __restrict__ out, int B, int H) {
-  const int h = blockIdx.x * 256 + threadIdx.x;
-  if (h >= H) return;
+  __shared__ double red[256];
+  const int h = blockIdx.x;
   double acc = 0.0;
-  for (int b = 0; b < B; ++b) acc += part[(int64_t)b * H + h];
-  out[h] = (float)acc;
+  for (int b = 0; b < B; ++b)
+    for (int j = threadIdx.x; j < slots; j += 256) acc += part[((int64_t)b * H + h) * slots + j];
+  const double all = block_sum(acc, red);
+  if (threadIdx.x == 0) out[h] = (float)all;
 }
 
 // gv[b, t, e] (one value head, rows of stride gv_stride per batch from the
@@ -229,19 +199,22 @@ bdh_status run_attention_vjp(const VjpArgs& a, hipStream_t st, uint64_t* launche
   const int64_t n_iv = (T + Lv - 1) / Lv;
   const int64_t LL = Lv * Lv, ND = N * D;
   const bool want_d = a.grad_decay != nullptr;
-  void *ps = nullptr, *pgs = nullptr, *pm = nullptr, *ptd = nullptr, *ppart = nullptr;
+  void *ps = nullptr, *pm = nullptr, *ptd = nullptr, *ppart = nullptr;
   void *prho = nullptr, *pgam = nullptr;
   bdh_status s = scratch(st, SLOT_VJP_S, (size_t)(S * LL) * sizeof(float), &ps);
-  if (s != BDH_OK) return s;
-  s = scratch(st, SLOT_VJP_GS, (size_t)(S * LL) * sizeof(float), &pgs);
   if (s != BDH_OK) return s;
   s = scratch(st, SLOT_VJP_M, (size_t)(S * LL) * sizeof(float), &pm);
   if (s != BDH_OK) return s;
   // [S, Lv, D] buffers: per-head grad_v (Hv = 1), IC, G * d^t, P = Q Gamma
   s = scratch(st, SLOT_VJP_TD, (size_t)(4 * S * Lv * D) * sizeof(float), &ptd);
   if (s != BDH_OK) return s;
-  // decay partials [S] and the state-term partials [S, kCrossBlocks + 1], f64
-  s = scratch(st, SLOT_VJP_PART, (size_t)(S * (kCrossBlocks + 2)) * sizeof(double), &ppart);
+  // The decay gradient's partial sums, f64: per stream the score tiles', the
+  // carried state's and the next state's.  (A shorter last interval may take
+  // the smaller tiles: never more slots than the largest interval on them.)
+  const int t_slots = n_iv > 1 ? (int)gf32::tile_count((int)Lv, (int)Lv, 64, true) : gf32::sym_slots(S, (int)Lv);
+  const int st_slots = a.rho0 || n_iv > 1 ? kStateBlocks : 0;
+  const int slots = t_slots + st_slots + (n_iv > 1 ? kCrossBlocks : 0);
+  s = scratch(st, SLOT_VJP_PART, (size_t)(S * slots) * sizeof(double), &ppart);
   if (s != BDH_OK) return s;
   if (n_iv > 1) {
     // states at the interval starts 1 .. n_iv - 1, and two Gamma buffers
@@ -264,14 +237,12 @@ bdh_status run_attention_vjp(const VjpArgs& a, hipStream_t st, uint64_t* launche
     part = (float*)pp;
   }
   float* Sc = (float*)ps;
-  float* GS = (float*)pgs;
   float* Msym = (float*)pm;
   float* gvh = (float*)ptd;
   float* ic = gvh + S * Lv * D;
   float* gp = ic + S * Lv * D;
   float* Pq = gp + S * Lv * D;
   double* dpart = (double*)ppart;
-  double* cpart = dpart + S;
   float* states = (float*)prho;
   float* gam[2] = {(float*)pgam, pgam ? (float*)pgam + S * ND : nullptr};
   uint64_t n = 0;
@@ -279,8 +250,10 @@ bdh_status run_attention_vjp(const VjpArgs& a, hipStream_t st, uint64_t* launche
   // Strides: query / grad_out / grad_q by stream (b*H + h); value by
   // (b, h) with a zero head stride when Hv = 1.
   const int64_t sVo = Hv * T * D, sVi = Hv == 1 ? 0 : T * D;
-  if (want_d) {
-    hipLaunchKernelGGL(zero_f64_kernel, dim3(cdivu(S, 256)), dim3(256), 0, st, dpart, S);
+  // One interval sets every slot, several add to them.
+  const int dacc = n_iv > 1 ? 1 : 0;
+  if (want_d && dacc) {
+    hipLaunchKernelGGL(zero_f64_kernel, dim3(cdivu(S * slots, 256)), dim3(256), 0, st, dpart, S * slots);
     BDH_HIP_TRY(hipGetLastError());
     ++n;
   }
@@ -318,17 +291,16 @@ bdh_status run_attention_vjp(const VjpArgs& a, hipStream_t st, uint64_t* launche
     g.C = Sc; g.sCo = H * LL; g.sCi = LL; g.sCm = Lv; g.sCn = 1;
     g.M = (int)L; g.N = (int)L; g.K = (int)N;
     BDH_HIP_TRY(gemm<E_TRIL_DECAY>(g, S, st, part, pe, &n));
-    // GS = tril(-1)(G V^T)
+    // M = GS * D + (GS * D)^T, GS = tril(-1)(G V^T), and the decay terms of GS and S
     g.A = G; g.sAo = H * T * D; g.sAi = T * D; g.sAm = D; g.sAk = 1;
     g.B = V; g.sBo = sVo; g.sBi = sVi; g.sBn = D; g.sBk = 1;
-    g.C = GS;
+    g.C = Msym;
     g.K = (int)D;
-    BDH_HIP_TRY(gemm<E_TRIL>(g, S, st, part, pe, &n));
-    // M = GS * D + (GS * D)^T
-    hipLaunchKernelGGL(msym_kernel, dim3(cdivu(L * L, 256 * 16), (unsigned)S), dim3(256), 0, st,
-                       (const float*)GS, Msym, a.decay, (int)H, (int)L, (int)Lv);
-    BDH_HIP_TRY(hipGetLastError());
-    ++n;
+    g.src = want_d ? Sc : nullptr;
+    g.dpart = dpart; g.dslots = slots; g.dacc = dacc;
+    g.recurrent_eps = a.recurrent_eps ? 1 : 0;
+    BDH_HIP_TRY(gemm<E_SYM_DECAY>(g, S, st, nullptr, 0, &n));
+    g.src = nullptr;
     // grad_q = M Q
     g.A = Msym; g.sAo = H * LL; g.sAi = LL; g.sAm = Lv; g.sAk = 1;
     g.B = Q; g.sBo = H * T * N; g.sBi = T * N; g.sBn = 1; g.sBk = N;
@@ -386,20 +358,19 @@ bdh_status run_attention_vjp(const VjpArgs& a, hipStream_t st, uint64_t* launche
       ++n;
     }
     if (want_d) {
-      hipLaunchKernelGGL(decay_partial_kernel, dim3((unsigned)S), dim3(256), 0, st, (const float*)GS,
-                         (const float*)Sc, (int)Lv, G, T * D, rho_iv ? (const float*)ic : nullptr, a.decay,
-                         (int)H, (int)L, (int)D, a.recurrent_eps ? 1 : 0, dpart);
-      BDH_HIP_TRY(hipGetLastError());
-      ++n;
+      if (rho_iv) {
+        hipLaunchKernelGGL(decay_state_kernel, dim3(kStateBlocks, (unsigned)S), dim3(256), 0, st, G, T * D,
+                           (const float*)ic, (int)Lv, a.decay, (int)H, (int)L, (int)D, a.recurrent_eps ? 1 : 0,
+                           dpart + t_slots, slots, dacc);
+        BDH_HIP_TRY(hipGetLastError());
+        ++n;
+      }
       if (gam_next) {
-        hipLaunchKernelGGL(decay_cross_kernel, dim3(kCrossBlocks + 1, (unsigned)S), dim3(256), 0, st,
+        hipLaunchKernelGGL(decay_cross_kernel, dim3(kCrossBlocks, (unsigned)S), dim3(256), 0, st,
                            (const float*)Pq, (int)Lv, V, sVo, sVi, rho_iv, gam_next, a.decay, (int)H,
-                           (int)L, ND, (int)D, a.recurrent_eps ? 1 : 0, cpart);
+                           (int)L, ND, (int)D, a.recurrent_eps ? 1 : 0, dpart + t_slots + st_slots, slots);
         BDH_HIP_TRY(hipGetLastError());
-        hipLaunchKernelGGL(cross_fold_kernel, dim3(cdivu(S, 256)), dim3(256), 0, st, (const double*)cpart,
-                           dpart, S);
-        BDH_HIP_TRY(hipGetLastError());
-        n += 2;
+        ++n;
       }
     }
     // Gamma_iv = Q^T (G * d^t) + d^L Gamma_{iv+1}: needed by the interval
@@ -424,7 +395,7 @@ bdh_status run_attention_vjp(const VjpArgs& a, hipStream_t st, uint64_t* launche
     gam_next = gam_out;
   }
   if (want_d) {
-    hipLaunchKernelGGL(decay_final_kernel, dim3(cdivu(H, 256)), dim3(256), 0, st, (const double*)dpart,
+    hipLaunchKernelGGL(decay_final_kernel, dim3((unsigned)H), dim3(256), 0, st, (const double*)dpart, slots,
                        a.grad_decay, (int)B, (int)H);
     BDH_HIP_TRY(hipGetLastError());
     ++n;
