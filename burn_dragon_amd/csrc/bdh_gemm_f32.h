@@ -109,13 +109,14 @@ __device__ __forceinline__ const float* epi_addend(const GemmF32& g, int64_t bo,
   return nullptr;
 }
 
-// Output value of (m, n) from the sum v and the addend x (when the kind has one).
-template <int EPI>
-__device__ __forceinline__ float epi_value(const GemmF32& g, float d, float carry, int m, int n, float v, float x) {
+// Output value of (m, n) from the sum v, the kind's decay power (a function,
+// called only where the kind has one and a decay is set) and the addend x
+// (when the kind has one).
+template <int EPI, class Pow>
+__device__ __forceinline__ float epi_value(const GemmF32& g, Pow&& power, float carry, int m, int n, float v, float x) {
   if (EPI == E_TRIL) v = n < m ? v : 0.0f;
-  if (EPI == E_TRIL_DECAY) v = n < m ? (g.decay ? v * dpowf(d, m - n) : v) : 0.0f;
-  if ((EPI == E_ROWSCALE || EPI == E_ROWSCALE_ACC) && g.decay) v *= dpowf(d, m);
-  if (EPI == E_ROWREV_ACC && g.decay) v *= dpowf(d, g.kpow - m);
+  if (EPI == E_TRIL_DECAY) v = n < m ? (g.decay ? v * power(m, n) : v) : 0.0f;
+  if ((EPI == E_ROWSCALE || EPI == E_ROWSCALE_ACC || EPI == E_ROWREV_ACC) && g.decay) v *= power(m, n);
   if (EPI == E_ROWSCALE_ACC || EPI == E_ROWREV_ACC) v += x;
   if (EPI == E_CARRY && g.src) v += x * carry;
   return v;
@@ -124,83 +125,77 @@ __device__ __forceinline__ float epi_value(const GemmF32& g, float d, float carr
 // A load of four floats at any float's address.
 typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
 
-// One operand's share of a step for thread t of a BT-row tile, E = BT / 16
-// values:
-//   KC (contiguous along k):    4 values at k 4 (t % 4) of rows t / 4 and
-//       t / 4 + 64 (BT = 128): four lanes read a row's 64 bytes;
-//   RC (contiguous along rows): E values at k (t / BT) E .. of row t % BT: a
-//       wave's load of one k reads 64 consecutive rows.
+// One operand's share of a step for thread t of a BT-row tile: E = BT / 16
+// values, in fours contiguous in memory (16-byte loads):
+//   KC (contiguous along k):    k 4 (t % 4) .. + 3 of rows t / 4 and, BT =
+//       128, t / 4 + 64: four lanes read a row's 64 bytes;
+//   RC (contiguous along rows): rows 4 (t % (BT / 4)) .. + 3 of the E / 4
+//       k's from (t / (BT / 4)) E / 4: a wave reads whole rows of the tile.
 // Rows past the operand's end re-read its last row: their sums are never
 // written.  k past Kt reads as 0.
 template <int BT, bool KC>
 struct Loader {
   static constexpr int E = BT / 16;
-  const float* p;   // KC: the thread's first row at its first k; RC: the tile's first row
+  const float* p;   // KC: the thread's first row at its first k; RC: the tile's first row at its first k
   const float* p1;  // KC, BT = 128: its second row
   int64_t sk;
-  uint32_t row;     // RC: the thread's row (clamped)
-  int k0;           // the thread's first k within a step
-  __device__ __forceinline__ void init(const float* X, int64_t sr, int64_t sk_, int R, int t) {
+  int k0, row, R;   // the thread's first k and row within a step's tile; rows of the tile
+  __device__ __forceinline__ void init(const float* X, int64_t sr, int64_t sk_, int R_, int t) {
     sk = sk_;
+    R = R_;
     if (KC) {
       k0 = (t & 3) * 4;
-      p = X + (int64_t)min(t >> 2, R - 1) * sr + k0;
-      p1 = X + (int64_t)min((t >> 2) + 64, R - 1) * sr + k0;
+      row = t >> 2;
+      p = X + (int64_t)min(row, R - 1) * sr + k0;
+      p1 = X + (int64_t)min(row + 64, R - 1) * sr + k0;
     } else {
-      // BT is a multiple of the wave's 64 rows: k0 is the same for the wave.
-      k0 = __builtin_amdgcn_readfirstlane(t / BT) * E;
-      row = (uint32_t)min(t % BT, R - 1);
-      p = X;
+      k0 = t / (BT / 4) * (E / 4);
+      row = t % (BT / 4) * 4;
+      p = X + (int64_t)k0 * sk;
     }
   }
   // k of value e, relative to the step.
-  __device__ __forceinline__ int k_of(int e) const { return k0 + (KC ? e & 3 : e); }
+  __device__ __forceinline__ int k_of(int e) const { return k0 + (KC ? e & 3 : e >> 2); }
   __device__ __forceinline__ void load(int kb, int Kt, float (&v)[E]) const {
-    if (KC) {
+    const bool fast = kb + GK <= Kt && (KC || R >= BT);
 #pragma unroll
-      for (int r = 0; r < E / 4; ++r) {
-        const float* q = r ? p1 : p;
-        if (kb + GK <= Kt) {
-          const floatx4u a = *reinterpret_cast<const floatx4u*>(q + kb);
-          v[4 * r] = a[0]; v[4 * r + 1] = a[1]; v[4 * r + 2] = a[2]; v[4 * r + 3] = a[3];
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float x = q[min(kb + k0 + e, Kt - 1) - k0];
-            v[4 * r + e] = kb + k0 + e < Kt ? x : 0.0f;
-          }
-        }
-      }
-    } else {
-      const float* q = p + (int64_t)(kb + k0) * sk;
-      if (kb + GK <= Kt) {
-#pragma unroll
-        for (int e = 0; e < E; ++e) v[e] = (q + e * sk)[row];
+    for (int r = 0; r < E / 4; ++r) {
+      const float* q = KC ? (r ? p1 : p) + kb : p + (int64_t)(kb + r) * sk + row;
+      if (fast) {
+        const floatx4u a = *reinterpret_cast<const floatx4u*>(q);
+        v[4 * r] = a[0]; v[4 * r + 1] = a[1]; v[4 * r + 2] = a[2]; v[4 * r + 3] = a[3];
       } else {
 #pragma unroll
-        for (int e = 0; e < E; ++e) {
-          const float x = (p + (int64_t)min(kb + k0 + e, Kt - 1) * sk)[row];
-          v[e] = kb + k0 + e < Kt ? x : 0.0f;
+        for (int e = 0; e < 4; ++e) {
+          const int k = kb + k_of(4 * r + e), kc = min(k, Kt - 1);
+          const float x = KC ? (r ? p1 : p)[kc - k0] : p[(int64_t)(kc - k0) * sk + min(row + e, R - 1)];
+          v[4 * r + e] = k < Kt ? x : 0.0f;
         }
       }
     }
   }
 };
 
-// Bytes of one part's tile in LDS: two halves of 8 k, 16 bytes a row, the
-// second half 128 bytes further so that a KC write's 32 lanes (8 rows, both
-// halves) cover every bank once.
+// LDS tile of one part of an operand, every access free of bank conflicts.
+//   KC: two halves of 8 k, 16 bytes a row, the second half 128 bytes further
+//       (a write's 32 lanes, 8 rows of both halves, cover every bank once);
+//       a fragment is one 16-byte read.
+//   RC: k rows of BT values, 64 bytes apart beyond their own (a transposing
+//       read's 32 lanes, 4 k rows of 64 bytes, cover every bank once); a
+//       fragment is two ds_read_b64_tr_b16, 4 k each: lane 4 r + c of 16
+//       names 4 values of k row r, lane i receives value i of the 4 rows.
 template <int BT>
 constexpr int kHalf = BT * 16 + 128;
 template <int BT>
-constexpr int kPart = 2 * kHalf<BT>;
-template <int BT>
-constexpr int kStage = 6 * kPart<BT>;  // A's three parts, then B's
+constexpr int kPitch = BT * 2 + 64;
+template <int BT, bool KC>
+constexpr int kPart = KC ? 2 * kHalf<BT> : GK * kPitch<BT>;
 
 // Splits a loader's values into their three bf16 parts and writes them to the
-// tile at `lds`.
-template <int BT, bool KC, int E>
-__device__ __forceinline__ void split_store(char* lds, int t, int k0, const float (&v)[E]) {
+// tiles at `lds`.
+template <int BT, bool KC>
+__device__ __forceinline__ void split_store(char* lds, const Loader<BT, KC>& l, const float (&v)[BT / 16]) {
+  constexpr int E = BT / 16;
   uint32_t w[3][E / 2];
 #pragma unroll
   for (int i = 0; i < E / 2; ++i) {
@@ -212,16 +207,35 @@ __device__ __forceinline__ void split_store(char* lds, int t, int k0, const floa
     w[1][i] = m;
     w[2][i] = pack_bf16x2(rx - bf16_lo(m), ry - bf16_hi(m));
   }
-  char* o = lds + (k0 >> 3) * kHalf<BT> + (KC ? t >> 2 : t % BT) * 16 + (k0 & 7) * 2;
+  char* o = lds + (KC ? (l.k0 >> 3) * kHalf<BT> + l.row * 16 + (l.k0 & 7) * 2 : l.k0 * kPitch<BT> + l.row * 2);
 #pragma unroll
-  for (int q = 0; q < 3; ++q) {
-    if constexpr (!KC && E == 8) {
-      *reinterpret_cast<uint4*>(o + q * kPart<BT>) = make_uint4(w[q][0], w[q][1], w[q][2], w[q][3]);
-    } else {
+  for (int q = 0; q < 3; ++q)
 #pragma unroll
-      for (int r = 0; r < E / 4; ++r)
-        *reinterpret_cast<uint2*>(o + q * kPart<BT> + r * 64 * 16) = make_uint2(w[q][2 * r], w[q][2 * r + 1]);
-    }
+    for (int r = 0; r < E / 4; ++r)
+      *reinterpret_cast<uint2*>(o + q * kPart<BT, KC> + r * (KC ? 64 * 16 : kPitch<BT>)) =
+          make_uint2(w[q][2 * r], w[q][2 * r + 1]);
+}
+
+typedef short shortx4 __attribute__((ext_vector_type(4)));
+
+// A 32-row fragment (rows row0 ..) of the part at `lds`; base = frag_base.
+template <int BT, bool KC>
+__device__ __forceinline__ int frag_base(int lane) {
+  if (KC) return (lane >> 5) * kHalf<BT> + (lane & 31) * 16;
+  return (8 * (lane >> 5) + ((lane & 15) >> 2)) * kPitch<BT> + (((lane >> 4) & 1) * 16 + (lane & 3) * 4) * 2;
+}
+template <int BT, bool KC>
+__device__ __forceinline__ bf16x8 frag_read(const char* lds, int base, int row0) {
+  if constexpr (KC) {
+    return *reinterpret_cast<const bf16x8*>(lds + base + row0 * 16);
+  } else {
+    typedef __attribute__((address_space(3))) shortx4 lds4;
+    const char* p = lds + base + row0 * 2;
+    struct {
+      shortx4 v[2];
+    } f = {{__builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4*)p),
+            __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4*)(p + 4 * kPitch<BT>))}};
+    return __builtin_bit_cast(bf16x8, f);
   }
 }
 
@@ -229,7 +243,8 @@ __device__ __forceinline__ void split_store(char* lds, int t, int k0, const floa
 template <int EPI, bool KSCALE, bool AKC, bool BKC, int BT>
 __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, int nty) {
   constexpr int E = BT / 16, NB = BT / 64;  // values a thread stages; 32 x 32 blocks a wave, each way
-  __shared__ __attribute__((aligned(16))) char lds[2 * kStage<BT> + (KSCALE ? 4 * (DSCALE + 3 * GK) : 0)];
+  constexpr int PA = kPart<BT, AKC>, PB = kPart<BT, BKC>, STAGE = 3 * (PA + PB);
+  __shared__ __attribute__((aligned(16))) char lds[2 * STAGE + (KSCALE ? 4 * (DSCALE + 3 * GK) : 0)];
   const int t = threadIdx.x, lane = t & 63, w = wave_id();
   const int wm = w >> 1, wn = w & 1;
   // Workgroup ids are remapped so that each XCD (id % 8) takes a contiguous
@@ -288,7 +303,7 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
   la.init(Ag, g.sAm, g.sAk, g.M - m0, t);
   lb.init(Bg, g.sBn, g.sBk, g.N - n0, t);
 
-  float* sct = reinterpret_cast<float*>(lds + 2 * kStage<BT>);
+  float* sct = reinterpret_cast<float*>(lds + 2 * STAGE);
   if (KSCALE) {
     for (int k = t; k < (nks + 2) * GK; k += 256) sct[k] = k < Kt ? dpowf(d, g.kpow - (k_lo + k)) : 0.0f;
     __syncthreads();
@@ -300,13 +315,13 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
     lb.load(s * GK, Kt, bv);
   };
   auto stage = [&](int s, float (&a)[E], float (&bv)[E]) {
-    char* o = lds + (s & 1) * kStage<BT>;
+    char* o = lds + (s & 1) * STAGE;
     if (KSCALE) {
 #pragma unroll
       for (int e = 0; e < E; ++e) a[e] *= sct[s * GK + la.k_of(e)];
     }
-    split_store<BT, AKC>(o, t, la.k0, a);
-    split_store<BT, BKC>(o + 3 * kPart<BT>, t, lb.k0, bv);
+    split_store(o, la, a);
+    split_store(o + 3 * PA, lb, bv);
   };
 
   floatx16 big[NB][NB], small[NB][NB];
@@ -317,15 +332,16 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
       big[i][j] = zero16();
       small[i][j] = zero16();
     }
+  const int fa = frag_base<BT, AKC>(lane), fb = 3 * PA + frag_base<BT, BKC>(lane);
   auto multiply = [&](int s) {
-    const char* o = lds + (s & 1) * kStage<BT> + (lane >> 5) * kHalf<BT> + (lane & 31) * 16;
+    const char* o = lds + (s & 1) * STAGE;
     bf16x8 a[3][NB], c[3][NB];
 #pragma unroll
     for (int q = 0; q < 3; ++q)
 #pragma unroll
       for (int i = 0; i < NB; ++i) {
-        a[q][i] = *reinterpret_cast<const bf16x8*>(o + q * kPart<BT> + (wm * 32 * NB + 32 * i) * 16);
-        c[q][i] = *reinterpret_cast<const bf16x8*>(o + (3 + q) * kPart<BT> + (wn * 32 * NB + 32 * i) * 16);
+        a[q][i] = frag_read<BT, AKC>(o + q * PA, fa, wm * 32 * NB + 32 * i);
+        c[q][i] = frag_read<BT, BKC>(o + q * PB, fb, wn * 32 * NB + 32 * i);
       }
     auto add = [&](int qa, int qb, floatx16 (&acc)[NB][NB]) {
 #pragma unroll
@@ -360,7 +376,7 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
         __syncthreads();
         multiply(s + u);
         stage(s + u + 1, va[u ^ 1], vb[u ^ 1]);
-        __builtin_amdgcn_sched_group_barrier(0x100, 6 * NB, 0);  // fragment reads
+        __builtin_amdgcn_sched_group_barrier(0x100, 3 * NB * ((AKC ? 1 : 2) + (BKC ? 1 : 2)), 0);  // fragment reads
 #pragma unroll
         for (int i = 0; i < 6 * NB * NB; ++i) {
           __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // an MFMA
@@ -409,6 +425,21 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
   }
 
   const float carry = (EPI == E_CARRY && g.decay) ? dpowf(d, g.kpow) : 1.0f;
+  // The decay powers of the epilogue's m - n (or rows), one powf each for the
+  // tile instead of one an element (which took 8 of a C1 product's 16 us).
+  constexpr bool DIFF = EPI == E_TRIL_DECAY || EPI == E_SYM_DECAY;
+  constexpr bool ROWS = EPI == E_ROWSCALE || EPI == E_ROWSCALE_ACC || EPI == E_ROWREV_ACC;
+  float* pw = reinterpret_cast<float*>(lds);
+  if ((DIFF || ROWS) && P == 1 && g.decay) {
+    __syncthreads();  // every wave has read its last fragments
+    if (DIFF && t < 2 * BT) pw[t] = dpowf(d, max(0, m0 - n0 - BT + 1 + t));
+    if (ROWS && t < BT) pw[t] = dpowf(d, EPI == E_ROWREV_ACC ? g.kpow - (m0 + t) : m0 + t);
+    __syncthreads();
+  }
+  auto power = [&](int m, int n) {
+    if (!(DIFF || ROWS) || !g.decay) return 1.0f;
+    return DIFF ? pw[m - n - (m0 - n0 - BT + 1)] : pw[m - m0];
+  };
   float* Pp = P > 1 ? g.part + ((int64_t)kp * g.batch + b) * (int64_t)g.M * g.N : nullptr;
   float* C = g.C + bo * g.sCo + bi * g.sCi;
   if constexpr (EPI == E_SYM_DECAY) {
@@ -432,7 +463,7 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
           if (m >= g.M || n > m) continue;
           const float v = n < m ? big[i][j][r] : 0.0f;
           sum += (double)(((v * (float)(m - n)) * x[r]) / sd);
-          const float o = g.decay ? v * dpowf(d, m - n) : v;
+          const float o = g.decay ? v * power(m, n) : v;
           C[(int64_t)m * g.sCm + n] = o;
           C[(int64_t)n * g.sCm + m] = o;
         }
@@ -470,7 +501,7 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
         if (P > 1) Pp[(int64_t)m * g.N + n] = big[i][j][r];
         else
           C[(int64_t)m * g.sCm + (int64_t)n * g.sCn] =
-              epi_value<EPI>(g, d, carry, m, n, big[i][j][r], X != nullptr ? x[r] : 0.0f);
+              epi_value<EPI>(g, power, carry, m, n, big[i][j][r], X != nullptr ? x[r] : 0.0f);
       }
     }
 }
@@ -490,6 +521,9 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmF32 g, int n4) {
   const int64_t b = blockIdx.y, bo = b / g.H, bi = b - bo * g.H;
   const float d = g.decay ? g.decay[bi] : 1.0f;
   const float carry = (EPI == E_CARRY && g.decay) ? dpowf(d, g.kpow) : 1.0f;
+  auto power = [&](int m, int n) {
+    return dpowf(d, EPI == E_TRIL_DECAY ? m - n : EPI == E_ROWREV_ACC ? g.kpow - m : m);
+  };
   const int64_t MN = (int64_t)g.M * g.N, total = g.batch * MN;
   const float* P = g.part + b * MN + (int64_t)m * g.N + n;
   const float* X = epi_addend<EPI>(g, bo, bi);
@@ -501,14 +535,14 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmF32 g, int n4) {
     if (X) x = *reinterpret_cast<const floatx4u*>(X + o);
     floatx4u w;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) w[e] = epi_value<EPI>(g, d, carry, m, n + e, v[e], x[e]);
+    for (int e = 0; e < 4; ++e) w[e] = epi_value<EPI>(g, power, carry, m, n + e, v[e], x[e]);
     *reinterpret_cast<floatx4u*>(C) = w;
     return;
   }
   for (int e = 0; e < 4 && n + e < g.N; ++e) {
     float v = 0.0f;
     for (int kp = 0; kp < g.ksplit; ++kp) v += P[kp * total + e];
-    C[e * g.sCn] = epi_value<EPI>(g, d, carry, m, n + e, v, X ? X[o + e * g.sCn] : 0.0f);
+    C[e * g.sCn] = epi_value<EPI>(g, power, carry, m, n + e, v, X ? X[o + e * g.sCn] : 0.0f);
   }
 }
 
