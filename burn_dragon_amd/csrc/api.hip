@@ -383,18 +383,20 @@ bdh_status forward_common(const bdh_recurrent_plan* plan, int32_t dtype, const v
       ++prof.launches;
       qr = (const float*)rot;
     }
-    const int64_t Lmax = want_rho ? (T < 256 ? T : 256) : T;
-    void* scores = nullptr;
-    st = scratch(hs, SLOT_SCORES, (size_t)(B * H * Lmax * Lmax) * sizeof(float), &scores);
-    if (st != BDH_OK) return st;
-    F32Args a{qr, (const float*)v, want_rho ? rho_in : nullptr, decay, ctx, rho_out,
-              (float*)scores, nullptr, B, H, Hv, T, N, D, Lmax, want_rho};
-    const size_t pe = f32_path_part_elems(a);
-    if (pe) {
-      void* part = nullptr;
-      st = scratch(hs, SLOT_GEMM_PART, pe * sizeof(float), &part);
+    F32Args a{qr, (const float*)v, want_rho ? rho_in : nullptr, decay, ctx, rho_out, B, H, Hv, T, N, D, want_rho};
+    const F32Scratch need = f32_path_scratch(a);
+    const struct {
+      int slot;
+      size_t elems;
+      float** out;
+    } bufs[] = {{SLOT_SCORES, need.scores, &a.scores}, {SLOT_SNAP, need.states, &a.states},
+                {SLOT_GEMM_PART, need.part, &a.part}};
+    for (const auto& buf : bufs) {
+      if (!buf.elems) continue;
+      void* p = nullptr;
+      st = scratch(hs, buf.slot, buf.elems * sizeof(float), &p);
       if (st != BDH_OK) return st;
-      a.part = (float*)part;
+      *buf.out = (float*)p;
     }
     hipError_t e = run_f32_path(a, hs, &prof.launches);
     if (e != hipSuccess) return hip_fail(e, "fp32 path launch");

@@ -50,6 +50,8 @@ enum Epi {
   E_ROWSCALE,      // C = acc * d^m
   E_ROWSCALE_ACC,  // C += acc * d^m
   E_CARRY,         // C = acc + src * d^kpow (src null: acc)
+  E_CARRY_SNAP,    // E_CARRY over a K of several intervals of `len`, the last perhaps shorter, one after
+                   // the other; the value at each interval's start but the first goes to snap
   E_ROWREV_ACC,    // C += acc * d^(kpow - m)
   E_SYM_DECAY      // C(m, n) = C(n, m) = acc * d^(m-n) for n < m, C(m, m) = 0; and the decay gradient's
                    // terms ((acc * (m-n)) * src(m, n)) / sd of n < m, summed per tile into dpart
@@ -64,13 +66,20 @@ struct GemmF32 {
   int64_t sBo, sBi, sBn, sBk;   // sBn or sBk is 1
   int64_t sCo, sCi, sCm, sCn;
   int M, N, K, H;
-  int kpow;             // E_CARRY: carry power; KSCALE (decay set): A(m, k) *= d^(kpow - k)
+  int kpow;             // E_CARRY: carry power; KSCALE (decay set): A(m, k) *= d^(kpow - k) (E_CARRY_SNAP: kpow is the end of k's interval)
   int kcausal;          // operand A lower triangular: K of the tile at row m0 limited to m0 + tile
   int klow;             // operand A upper triangular: K of the tile at row m0 from m0's TRI-block on
   const float* decay;   // [H] or null (ones)
   float* part;          // split-K partials [ksplit, batch, M, N] (ksplit > 1)
   int ksplit;
-  int64_t batch;
+  int64_t batch;        // products of an interval
+  // A launch over several intervals (0 and 1: one): interval iv's operands are
+  // sA3, sB3, sC3 further each, and the last one's sizes are M1, N1, K1.
+  int niv, M1, N1, K1;
+  int64_t sA3, sB3, sC3;
+  float* snap;          // E_CARRY_SNAP: [intervals - 1] of C's layout, sSnap apart
+  int64_t sSnap;
+  int len;              // E_CARRY_SNAP: tokens of an interval (a multiple of 2 GK)
   double* dpart;        // E_SYM_DECAY: tile sums [batch, dslots]
   int dslots, dacc;     // (dacc: added to what is there)
   int recurrent_eps;    // E_SYM_DECAY: the recurrent backward's decay guard
@@ -103,9 +112,9 @@ __device__ __forceinline__ double block_sum(double v, double* red) {
 // The epilogue's addend: C itself (the accumulating kinds), src (E_CARRY),
 // or none.
 template <int EPI>
-__device__ __forceinline__ const float* epi_addend(const GemmF32& g, int64_t bo, int64_t bi) {
-  if (EPI == E_ROWSCALE_ACC || EPI == E_ROWREV_ACC) return g.C + bo * g.sCo + bi * g.sCi;
-  if (EPI == E_CARRY && g.src) return g.src + bo * g.sCo + bi * g.sCi;
+__device__ __forceinline__ const float* epi_addend(const GemmF32& g, int64_t c0) {
+  if (EPI == E_ROWSCALE_ACC || EPI == E_ROWREV_ACC) return g.C + c0;
+  if ((EPI == E_CARRY || EPI == E_CARRY_SNAP) && g.src) return g.src + c0;
   return nullptr;
 }
 
@@ -119,6 +128,7 @@ __device__ __forceinline__ float epi_value(const GemmF32& g, Pow&& power, float 
   if ((EPI == E_ROWSCALE || EPI == E_ROWSCALE_ACC || EPI == E_ROWREV_ACC) && g.decay) v *= power(m, n);
   if (EPI == E_ROWSCALE_ACC || EPI == E_ROWREV_ACC) v += x;
   if (EPI == E_CARRY && g.src) v += x * carry;
+  if (EPI == E_CARRY_SNAP) v += x * carry;
   return v;
 }
 
@@ -287,27 +297,39 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
   }
   const int P = g.ksplit > 1 ? g.ksplit : 1;
   const int kp = (int)(z % P);
-  const int64_t b = z / P, bo = b / g.H, bi = b - bo * g.H;
+  const int64_t bz = z / P, iv = g.niv > 1 ? bz / g.batch : 0, b = bz - iv * g.batch, bo = b / g.H, bi = b - bo * g.H;
   const int m0 = ty * BT, n0 = tx * BT;
+  const bool lastiv = g.niv > 1 && iv == g.niv - 1;
+  const int M = lastiv ? g.M1 : g.M, N = lastiv ? g.N1 : g.N, K = lastiv ? g.K1 : g.K;
+  if (m0 >= M || n0 >= N) return;  // a shorter last interval
   const float d = g.decay ? g.decay[bi] : 1.0f;
-  const int Kfull = g.kcausal ? min(g.K, m0 + BT) : g.K;
+  const int Kfull = g.kcausal ? min(K, m0 + BT) : K;
   const int kbase = g.klow ? m0 / TRI * TRI : 0;
   const int chunk = ((Kfull - kbase + P - 1) / P + GK - 1) / GK * GK;
   const int k_lo = min(Kfull, kbase + kp * chunk);
   const int Kt = min(Kfull, k_lo + chunk) - k_lo;  // this workgroup's depth, from k_lo
   const int nks = (Kt + GK - 1) / GK;
-  const float* Ag = g.A + bo * g.sAo + bi * g.sAi + (int64_t)m0 * g.sAm + (int64_t)k_lo * g.sAk;
-  const float* Bg = g.B + bo * g.sBo + bi * g.sBi + (int64_t)n0 * g.sBn + (int64_t)k_lo * g.sBk;
+  const float* A0 = g.A + iv * g.sA3 + bo * g.sAo + bi * g.sAi;
+  const float* B0 = g.B + iv * g.sB3 + bo * g.sBo + bi * g.sBi;
+  const int64_t c0 = iv * g.sC3 + bo * g.sCo + bi * g.sCi;
   Loader<BT, AKC> la;
   Loader<BT, BKC> lb;
-  la.init(Ag, g.sAm, g.sAk, g.M - m0, t);
-  lb.init(Bg, g.sBn, g.sBk, g.N - n0, t);
+  la.init(A0 + (int64_t)m0 * g.sAm + (int64_t)k_lo * g.sAk, g.sAm, g.sAk, M - m0, t);
+  lb.init(B0 + (int64_t)n0 * g.sBn + (int64_t)k_lo * g.sBk, g.sBn, g.sBk, N - n0, t);
 
   float* sct = reinterpret_cast<float*>(lds + 2 * STAGE);
+  constexpr bool SNAP = EPI == E_CARRY_SNAP;
   if (KSCALE) {
-    for (int k = t; k < (nks + 2) * GK; k += 256) sct[k] = k < Kt ? dpowf(d, g.kpow - (k_lo + k)) : 0.0f;
+    if (SNAP) {
+      for (int k = t; k <= g.len; k += 256) sct[k] = dpowf(d, k);
+    } else {
+      for (int k = t; k < (nks + 2) * GK; k += 256) sct[k] = k < Kt ? dpowf(d, g.kpow - (k_lo + k)) : 0.0f;
+    }
     __syncthreads();
   }
+  // SNAP: tokens of interval i, and a power of its token k's weight (0 past K).
+  auto len_of = [&](int i) { return min(g.len, Kt - i * g.len); };
+  int siv = 0, soff = 0;  // the interval and offset of the step staged next
 
   float va[2][E], vb[2][E];
   auto load = [&](int s, float (&a)[E], float (&bv)[E]) {
@@ -318,7 +340,14 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
     char* o = lds + (s & 1) * STAGE;
     if (KSCALE) {
 #pragma unroll
-      for (int e = 0; e < E; ++e) a[e] *= sct[s * GK + la.k_of(e)];
+      for (int e = 0; e < E; ++e) a[e] *= sct[SNAP ? max(0, len_of(siv) - soff - la.k_of(e)) : s * GK + la.k_of(e)];
+      if (SNAP) {
+        soff += GK;
+        if (soff == g.len) {
+          soff = 0;
+          ++siv;
+        }
+      }
     }
     split_store(o, la, a);
     split_store(o + 3 * PA, lb, bv);
@@ -357,6 +386,46 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
     add(2, 0, small);
   };
 
+  const int mw = m0 + wm * 32 * NB, nw = n0 + wn * 32 * NB;  // the wave's block
+  // SNAP, at the end of interval i, another one following: the state there is
+  // written, and the next interval's sum starts from 0 and is added to it (as
+  // an interval's sum always was: one sum over all of them would round to the
+  // growing state's last bit).
+  const float* X = P > 1 ? nullptr : epi_addend<EPI>(g, c0);
+  bool bad = false;  // a sum is not finite
+  auto snapshot = [&](int i) {
+    float* o = g.snap + i * g.sSnap + c0;
+    // (The block's addresses are not kept through the step loop: 64 of them
+    // would not fit beside the accumulators.)
+    int mo = mw + acc_row(lane, 0);
+    asm volatile("" : "+v"(mo));
+    const float dl = g.decay ? dpowf(d, len_of(i)) : 1.0f;
+#pragma unroll
+    for (int i2 = 0; i2 < NB; ++i2)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        const int n = nw + 32 * j + acc_col(lane);
+        const int64_t off = (int64_t)(mo + 32 * i2) * g.sCm + (int64_t)n * g.sCn;
+        float x[16];
+        if (X != nullptr) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            x[r] = mo + 32 * i2 + acc_row(0, r) < M && n < N ? X[off + acc_row(0, r) * g.sCm] : 0.0f;
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const float v = big[i2][j][r] + small[i2][j][r];
+          bad |= !__builtin_isfinite(v);
+          if (mo + 32 * i2 + acc_row(0, r) < M && n < N)
+            o[off + acc_row(0, r) * g.sCm] = X != nullptr ? v + x[r] * dl : v;
+        }
+        big[i2][j] = zero16();
+        small[i2][j] = zero16();
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    X = o;
+  };
+
   // Step s: its parts are in LDS buffer s & 1, step s + 1's values in
   // register set (s + 1) & 1; the loads of step s + 2 go to the other set.
   // One barrier a step: it ends the writes of step s's buffer and the reads
@@ -368,26 +437,30 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
     load(0, va[0], vb[0]);
     load(1, va[1], vb[1]);
     stage(0, va[0], vb[0]);
-    int s = 0;
-    do {
+    int s = 0, end = SNAP ? min(nks, g.len / GK) : nks, i = 0;
+    while (true) {
+      do {
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        load(s + u + 2, va[u], vb[u]);
-        __syncthreads();
-        multiply(s + u);
-        stage(s + u + 1, va[u ^ 1], vb[u ^ 1]);
-        __builtin_amdgcn_sched_group_barrier(0x100, 3 * NB * ((AKC ? 1 : 2) + (BKC ? 1 : 2)), 0);  // fragment reads
+        for (int u = 0; u < 2; ++u) {
+          load(s + u + 2, va[u], vb[u]);
+          __syncthreads();
+          multiply(s + u);
+          stage(s + u + 1, va[u ^ 1], vb[u ^ 1]);
+          __builtin_amdgcn_sched_group_barrier(0x100, 3 * NB * ((AKC ? 1 : 2) + (BKC ? 1 : 2)), 0);  // fragment reads
 #pragma unroll
-        for (int i = 0; i < 6 * NB * NB; ++i) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // an MFMA
-          __builtin_amdgcn_sched_group_barrier(0x002, NB == 2 ? 4 : 8, 0);  // VALU
+          for (int k = 0; k < 6 * NB * NB; ++k) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // an MFMA
+            __builtin_amdgcn_sched_group_barrier(0x002, NB == 2 ? 4 : 8, 0);  // VALU
+          }
         }
-      }
-      s += 2;
-    } while (s < nks);
+        s += 2;
+      } while (s < end);
+      if (!SNAP || end >= nks) break;
+      snapshot(i++);
+      end = min(nks, end + g.len / GK);
+    }
   }
 
-  bool bad = false;
 #pragma unroll
   for (int i = 0; i < NB; ++i)
 #pragma unroll
@@ -395,25 +468,26 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         big[i][j][r] += small[i][j][r];
+        small[i][j][r] = 0.0f;
         bad |= !__builtin_isfinite(big[i][j][r]);
       }
-  const int mw = m0 + wm * 32 * NB, nw = n0 + wn * 32 * NB;  // the wave's block
   if (__any(bad)) {
     // Not finite: the block again on v_mfma_f32_32x32x2_f32, straight from memory.
-    const float* A0 = g.A + bo * g.sAo + bi * g.sAi;
-    const float* B0 = g.B + bo * g.sBo + bi * g.sBi;
+    if (SNAP) X = epi_addend<EPI>(g, c0);
 #pragma unroll
     for (int i = 0; i < NB; ++i)
 #pragma unroll
       for (int j = 0; j < NB; ++j) big[i][j] = zero16();
+    int i0 = 0;  // SNAP: the interval
     for (int k = 0; k < Kt; k += 2) {
+      if (SNAP && k == (i0 + 1) * g.len) snapshot(i0++);
       const int kk = k + (lane >> 5), ka = k_lo + min(kk, Kt - 1);
       float av[NB], bv[NB];
 #pragma unroll
       for (int i = 0; i < NB; ++i) {
-        av[i] = A0[(int64_t)min(mw + 32 * i + (lane & 31), g.M - 1) * g.sAm + (int64_t)ka * g.sAk];
-        if (KSCALE) av[i] *= sct[min(kk, Kt - 1)];
-        bv[i] = B0[(int64_t)min(nw + 32 * i + (lane & 31), g.N - 1) * g.sBn + (int64_t)ka * g.sBk];
+        av[i] = A0[(int64_t)min(mw + 32 * i + (lane & 31), M - 1) * g.sAm + (int64_t)ka * g.sAk];
+        if (KSCALE) av[i] *= sct[SNAP ? max(0, len_of(i0) - (kk - i0 * g.len)) : min(kk, Kt - 1)];
+        bv[i] = B0[(int64_t)min(nw + 32 * i + (lane & 31), N - 1) * g.sBn + (int64_t)ka * g.sBk];
         if (kk >= Kt) av[i] = bv[i] = 0.0f;
       }
 #pragma unroll
@@ -424,7 +498,9 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
     }
   }
 
-  const float carry = (EPI == E_CARRY && g.decay) ? dpowf(d, g.kpow) : 1.0f;
+  const float carry = !g.decay ? 1.0f
+                      : SNAP   ? dpowf(d, len_of((nks - 1) * GK / g.len))
+                      : EPI == E_CARRY ? dpowf(d, g.kpow) : 1.0f;
   // The decay powers of the epilogue's m - n (or rows), one powf each for the
   // tile instead of one an element (which took 8 of a C1 product's 16 us).
   constexpr bool DIFF = EPI == E_TRIL_DECAY || EPI == E_SYM_DECAY;
@@ -440,10 +516,11 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
     if (!(DIFF || ROWS) || !g.decay) return 1.0f;
     return DIFF ? pw[m - n - (m0 - n0 - BT + 1)] : pw[m - m0];
   };
-  float* Pp = P > 1 ? g.part + ((int64_t)kp * g.batch + b) * (int64_t)g.M * g.N : nullptr;
-  float* C = g.C + bo * g.sCo + bi * g.sCi;
+  const int64_t batches = g.batch * (g.niv > 1 ? g.niv : 1);
+  float* Pp = P > 1 ? g.part + ((int64_t)kp * batches + bz) * (int64_t)g.M * g.N : nullptr;
+  float* C = g.C + c0;
   if constexpr (EPI == E_SYM_DECAY) {
-    const float* SC = g.src ? g.src + bo * g.sCo + bi * g.sCi : nullptr;
+    const float* SC = g.src ? g.src + c0 : nullptr;
     const float sd = decay_sd(d, g.recurrent_eps);
     double sum = 0.0;
 #pragma unroll
@@ -455,12 +532,12 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int m = mw + 32 * i + acc_row(lane, r);
-          x[r] = SC && m < g.M && n < m ? SC[(int64_t)m * g.sCm + n] : 0.0f;
+          x[r] = SC && m < M && n < m ? SC[(int64_t)m * g.sCm + n] : 0.0f;
         }
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int m = mw + 32 * i + acc_row(lane, r);
-          if (m >= g.M || n > m) continue;
+          if (m >= M || n > m) continue;
           const float v = n < m ? big[i][j][r] : 0.0f;
           sum += (double)(((v * (float)(m - n)) * x[r]) / sd);
           const float o = g.decay ? v * power(m, n) : v;
@@ -478,8 +555,7 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
     }
     return;
   }
-  const float* X = P > 1 ? nullptr : epi_addend<EPI>(g, bo, bi);
-  const bool whole = m0 + BT <= g.M && n0 + BT <= g.N;
+  const bool whole = m0 + BT <= M && n0 + BT <= N;
 #pragma unroll
   for (int i = 0; i < NB; ++i)
 #pragma unroll
@@ -491,13 +567,13 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int m = mw + 32 * i + acc_row(lane, r);
-          x[r] = whole || (m < g.M && n < g.N) ? X[(int64_t)m * g.sCm + (int64_t)n * g.sCn] : 0.0f;
+          x[r] = whole || (m < M && n < N) ? X[(int64_t)m * g.sCm + (int64_t)n * g.sCn] : 0.0f;
         }
       }
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int m = mw + 32 * i + acc_row(lane, r);
-        if (!whole && (m >= g.M || n >= g.N)) continue;
+        if (!whole && (m >= M || n >= N)) continue;
         if (P > 1) Pp[(int64_t)m * g.N + n] = big[i][j][r];
         else
           C[(int64_t)m * g.sCm + (int64_t)n * g.sCn] =
@@ -508,7 +584,7 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
 
 // Split-K: sums the P partials of each (b, m, n) in range order and applies
 // the epilogue, four columns a thread (the last thread of a row that is not a
-// multiple of four: the rest).  Batch blockIdx.y.  A masked
+// multiple of four: the rest).  Product blockIdx.y.  A masked
 // product's blocks above the diagonal are left out: their partials were not
 // written, and their outputs are never read.
 template <int EPI>
@@ -518,18 +594,23 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmF32 g, int n4) {
   if (mi >= g.M) return;
   const int m = (int)mi, n = (int)(i - mi * n4) * 4;
   if (g.tri && n / TRI > m / TRI) return;
-  const int64_t b = blockIdx.y, bo = b / g.H, bi = b - bo * g.H;
+  const int64_t bz = blockIdx.y, iv = g.niv > 1 ? bz / g.batch : 0, b = bz - iv * g.batch, bo = b / g.H,
+                bi = b - bo * g.H;
+  const bool lastiv = g.niv > 1 && iv == g.niv - 1;
+  const int M = lastiv ? g.M1 : g.M, N = lastiv ? g.N1 : g.N;
+  if (m >= M || n >= N) return;
   const float d = g.decay ? g.decay[bi] : 1.0f;
   const float carry = (EPI == E_CARRY && g.decay) ? dpowf(d, g.kpow) : 1.0f;
   auto power = [&](int m, int n) {
     return dpowf(d, EPI == E_TRIL_DECAY ? m - n : EPI == E_ROWREV_ACC ? g.kpow - m : m);
   };
-  const int64_t MN = (int64_t)g.M * g.N, total = g.batch * MN;
-  const float* P = g.part + b * MN + (int64_t)m * g.N + n;
-  const float* X = epi_addend<EPI>(g, bo, bi);
+  const int64_t MN = (int64_t)g.M * g.N, total = (int64_t)gridDim.y * MN;
+  const float* P = g.part + bz * MN + (int64_t)m * g.N + n;
+  const int64_t c0 = iv * g.sC3 + bo * g.sCo + bi * g.sCi;
+  const float* X = epi_addend<EPI>(g, c0);
   const int64_t o = (int64_t)m * g.sCm + (int64_t)n * g.sCn;
-  float* C = g.C + bo * g.sCo + bi * g.sCi + o;
-  if (g.sCn == 1 && n + 4 <= g.N) {
+  float* C = g.C + c0 + o;
+  if (g.sCn == 1 && n + 4 <= N) {
     floatx4 v = zero4(), x = zero4();
     for (int kp = 0; kp < g.ksplit; ++kp) v += *reinterpret_cast<const floatx4u*>(P + kp * total);
     if (X) x = *reinterpret_cast<const floatx4u*>(X + o);
@@ -539,7 +620,7 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmF32 g, int n4) {
     *reinterpret_cast<floatx4u*>(C) = w;
     return;
   }
-  for (int e = 0; e < 4 && n + e < g.N; ++e) {
+  for (int e = 0; e < 4 && n + e < N; ++e) {
     float v = 0.0f;
     for (int kp = 0; kp < g.ksplit; ++kp) v += P[kp * total + e];
     C[e * g.sCn] = epi_value<EPI>(g, power, carry, m, n + e, v, X ? X[o + e * g.sCn] : 0.0f);
@@ -586,7 +667,10 @@ hipError_t launch_gemm(const GemmF32& g, int64_t nwg, hipStream_t st) {
   const bool akc = g.sAk == 1, bkc = g.sBk == 1;
   if ((!akc && g.sAm != 1) || (!bkc && g.sBn != 1) || nwg > INT32_MAX) return hipErrorInvalidValue;
   const dim3 grid((unsigned)nwg);
-  if (akc && bkc)
+  if constexpr (EPI == E_CARRY_SNAP) {  // the state's operands are both contiguous along their rows
+    if (akc || bkc) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((gemm_split_kernel<EPI, KSCALE, false, false, BT>), grid, dim3(256), 0, st, g, ntx, nty);
+  } else if (akc && bkc)
     hipLaunchKernelGGL((gemm_split_kernel<EPI, KSCALE, true, true, BT>), grid, dim3(256), 0, st, g, ntx, nty);
   else if (akc)
     hipLaunchKernelGGL((gemm_split_kernel<EPI, KSCALE, true, false, BT>), grid, dim3(256), 0, st, g, ntx, nty);
@@ -597,6 +681,8 @@ hipError_t launch_gemm(const GemmF32& g, int64_t nwg, hipStream_t st) {
   return hipGetLastError();
 }
 
+constexpr int64_t kMaxBatch = 65535;  // products of a launch (the reduce's grid)
+
 // A product runs on 64 x 64 tiles while its 128 x 128 ones leave CUs idle.
 inline bool small_tiles(int64_t tiles, int p) { return tiles * p < (int64_t)device_cus(); }
 
@@ -606,7 +692,7 @@ inline int sym_slots(int64_t batch, int L) {
   return (int)(small_tiles(tiles * batch, 1) ? tile_count(L, L, 64, true) : tiles);
 }
 
-// C = epilogue(A B^T) over `batch` products.  With `part` (part_elems floats)
+// C = epilogue(A B^T) over `batch` products (of each of g.niv intervals).  With `part` (part_elems floats)
 // a long K may be split; the partials need ksplit * batch * M * N floats.
 template <int EPI, bool KSCALE = false>
 hipError_t gemm(GemmF32 g, int64_t batch, hipStream_t st, float* part = nullptr, size_t part_elems = 0,
@@ -614,9 +700,12 @@ hipError_t gemm(GemmF32 g, int64_t batch, hipStream_t st, float* part = nullptr,
   if (g.M <= 0 || g.N <= 0 || batch <= 0) return hipSuccess;
   if constexpr (KSCALE) {
     if (!g.decay) return gemm<EPI, false>(g, batch, st, part, part_elems, launches);
-    if (g.K > DSCALE) return hipErrorInvalidValue;
+    if ((EPI == E_CARRY_SNAP ? g.len : g.K) > DSCALE) return hipErrorInvalidValue;
   }
+  if (EPI == E_CARRY_SNAP && (part || g.len <= 0 || g.len % (2 * GK) != 0)) return hipErrorInvalidValue;
   g.batch = batch;
+  if (g.niv > 1) batch *= g.niv;
+  if (batch > kMaxBatch) return hipErrorInvalidValue;
   g.tri = (EPI == E_TRIL || EPI == E_TRIL_DECAY || EPI == E_SYM_DECAY) && g.M == g.N;
   if (EPI == E_SYM_DECAY && (!g.tri || part)) return hipErrorInvalidValue;
   const size_t per = (size_t)batch * (size_t)g.M * (size_t)g.N;

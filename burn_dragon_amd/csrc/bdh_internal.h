@@ -47,7 +47,7 @@ enum ScratchSlot {
   SLOT_GEMM_PART,    // fp32 GEMM split-K partials   [P, batch, M, N] f32
   SLOT_VJP_RHO,      // VJP states at interval starts [n_iv - 1, S, N, D] f32
   SLOT_VJP_GAMMA,    // VJP state gradients          2 x [S, N, D] f32
-  SLOT_SNAP,         // states at interval starts (bf16 path) [n_iv, S, D, N] bf16
+  SLOT_SNAP,         // states at interval starts: bf16 path [n_iv, S, D, N] bf16, fp32 path [n_iv - 1, S, N, D] f32
   SLOT_COUNT
 };
 // Scratch of the calling stream (see api.hip): grows on first use of a
@@ -80,6 +80,7 @@ hipError_t launch_rope_rotate_f32(const float* x, const float* freqs, float* out
                                   int64_t T, int64_t N, int64_t pos0, int fixed, hipStream_t st);
 
 // --- fp32 path (prefill_f32.hip) -------------------------------------------
+constexpr int64_t kF32Interval = 512;  // tokens of its state-carry intervals
 struct F32Args {
   const float* q;       // rotated queries [S, T, N]
   const float* v;       // [B, Hv, T, D]
@@ -87,15 +88,19 @@ struct F32Args {
   const float* decay;   // [H] or null
   float* ctx;           // [S, T, D]
   float* rho_out;       // [S, N, D]
-  float* scores;        // scratch [S, Lmax, Lmax]
-  float* part;          // scratch for the GEMMs' split-K partials (f32_path_part_elems floats)
-  int64_t B, H, Hv, T, N, D, Lmax;
+  int64_t B, H, Hv, T, N, D;
   bool state;           // false: context only (single interval, no rho)
-  // Context-only calls on pre-rotated queries: gram partials in bf16 (half
-  // the partial traffic; the scores then carry ~9 significant bits).
-  bool part16 = false;
+  // Scratch (f32_path_scratch).
+  float* scores = nullptr;
+  float* states = nullptr;
+  float* part = nullptr;
 };
-size_t f32_path_part_elems(const F32Args& a);
+struct F32Scratch {
+  size_t scores;  // floats: scores of a group of intervals [intervals, S, L, L]
+  size_t states;  // states at its interval starts but the first [intervals - 1, S, N, D]
+  size_t part;    // the GEMMs' split-K partials
+};
+F32Scratch f32_path_scratch(const F32Args& a);
 hipError_t run_f32_path(const F32Args& a, hipStream_t st, uint64_t* launches);
 
 // --- bf16 MFMA path (prefill_bf16.hip) --------------------------------------

@@ -99,8 +99,8 @@ int32_t bdh_supports_backend(void);
  * through causal score blocks of 128 tokens.  0 = auto: 512 (the
  * reference's default, config.rs:10), with or without decay; otherwise a
  * multiple of 128 up to 4096 (BDH_UNSUPPORTED otherwise).  The result does
- * not depend on it beyond rounding; the fp32 path materialises rho every 256
- * tokens whatever it is.
+ * not depend on it beyond rounding; the fp32 path materialises rho at least
+ * every 512 tokens whatever it is.
  * time == 1 with BDH_F32 (the reference's decode call, sequence_dispatch.rs
  * :109-124; it selects kernels by T, forward_runtime.rs:235-256) runs the
  * one-token step of bdh_decode_step: with rho_out == rho_in and no decay

@@ -22,7 +22,9 @@ TOL = 3e-6
     (1, 2, 2, 129, 48, 129, True, [0.99, 0.98]),   # one row and column past a 128 tile
     (1, 1, 1, 257, 1026, 33, False, None),         # masked blocks, split k with a ragged range
     (16, 4, 1, 160, 64, 200, True, None),          # 128 tiles (over one a CU), ragged in both
-    (1, 1, 1, 1030, 36, 12, True, [0.999]),        # the backward's second interval
+    (1, 1, 1, 1030, 36, 12, True, [0.999]),        # the backward's second interval, three of the forward
+    (2, 2, 1, 513, 130, 70, True, [0.99, 0.999]),  # two state intervals, the last short
+    (16, 1, 1, 700, 1030, 72, False, None),        # two intervals, 128-row tiles, split k over both
 ])
 def test_edges_match_oracle(oracle, B, H, Hv, T, N, D, rho, decay):
     torch = need_gpu()
@@ -59,7 +61,7 @@ def test_edges_match_oracle(oracle, B, H, Hv, T, N, D, rho, decay):
     assert (np.abs(host(grads.grad_decay) - ref[2]) <= TOL * size).all()
 
 
-@pytest.mark.parametrize("T,N,D", [(40, 32, 24), (200, 96, 160)])
+@pytest.mark.parametrize("T,N,D", [(40, 32, 24), (200, 96, 160), (600, 32, 24)])
 def test_values_without_bf16_parts(T, N, D):
     # An infinity, a NaN and a finite value above bf16's largest: every output
     # is what fp32 products give, infinite and NaN in the same places.
