@@ -115,7 +115,11 @@ __device__ __forceinline__ void carry_loader(const CarryArgs& a, char* lds, int6
   // (cos, sin) of the lane's 4 pairs at its two tokens of the step rotated
   // next: from frac(pos f) for step 0 (positions clamped to T - 1 as the
   // rows are), then advanced by e(32 f) a step, one complex multiply a pair
-  // instead of a phase, a cosine and a sine (the steps run in order).
+  // instead of a phase, a cosine and a sine (the steps run in order).  A call
+  // of one interval computes every step's words from their phases, as the
+  // state units of a call without a carried state do: a sequence split in
+  // such calls then carries the state of the whole.
+  const bool direct = a.T <= a.L;
   float ca[4], sa[4], cb[4], sb[4], ec[4], es[4];
   if (ROPE) {
     const int64_t ta = 2 * tp < a.T ? 2 * tp : a.T - 1, tb = 2 * tp + 1 < a.T ? 2 * tp + 1 : a.T - 1;
@@ -161,8 +165,17 @@ __device__ __forceinline__ void carry_loader(const CarryArgs& a, char* lds, int6
                       pack_bf16x2(ca[3], sa[3]));
       c1 = make_uint4(pack_bf16x2(cb[0], sb[0]), pack_bf16x2(cb[1], sb[1]), pack_bf16x2(cb[2], sb[2]),
                       pack_bf16x2(cb[3], sb[3]));
+      const float pn = (float)(a.fixed ? a.pos0 : a.pos0 + t + BK);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
+        if (direct) {
+          const float fa = rope_frac(pn, fq[j]), fb = rope_frac(a.fixed ? pn : pn + 1.0f, fq[j]);
+          ca[j] = __builtin_amdgcn_cosf(fa);
+          sa[j] = __builtin_amdgcn_sinf(fa);
+          cb[j] = __builtin_amdgcn_cosf(fb);
+          sb[j] = __builtin_amdgcn_sinf(fb);
+          continue;
+        }
         const float na = ca[j] * ec[j] - sa[j] * es[j], ma = sa[j] * ec[j] + ca[j] * es[j];
         const float nb = cb[j] * ec[j] - sb[j] * es[j], mb = sb[j] * ec[j] + cb[j] * es[j];
         ca[j] = na;

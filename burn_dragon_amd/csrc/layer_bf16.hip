@@ -296,9 +296,10 @@ __global__ __launch_bounds__(NT, 2) void layer_gemm_kernel(LayerGemmArgs g) {
 // register of a lane holds 4 consecutive latents of one token.  The
 // workgroup owns one column tile (latent chunk) and walks the row tiles in
 // order, so at any time the workgroups write neighbouring 256-byte pieces of
-// the same rows.  Needs T % 128 == 0, N % 128 == 0, 64 <= D <= 256 with
-// D % 32 == 0, and at most one column tile per CU (C5: 256 column tiles on
-// 256 CUs).  Measured at C5 (GEMM X of layer_gemm_kernel: 688 us): 766 us
+// the same rows.  A row tile is 128 tokens of one sequence, its last one
+// perhaps fewer (the rows past it are fetched, multiplied and not stored).
+// Needs N % 128 == 0, 64 <= D <= 256 with D % 32 == 0, and at most one column
+// tile per CU (C5: 256 column tiles on 256 CUs).  Measured at C5 (GEMM X of layer_gemm_kernel: 688 us): 766 us
 // with 4 MFMA waves that also issued the DMAs, 4 store waves and a barrier
 // per K step (the store waves held the barriers); 620 us with 8 store waves
 // and no 64-bit divisions in the loops; 601 us with 8 MFMA waves meeting
@@ -320,6 +321,15 @@ __global__ __launch_bounds__(NT, 2) void layer_gemm_kernel(LayerGemmArgs g) {
 // among them fragment registers stored to scratch before their read had
 // completed (tests/asm_waits.py reports exactly that); not run.
 constexpr int XR_T = 128;                      // tile edge (tokens and latents)
+// Row tiles of a sequence of T tokens: of 128 tokens, the last perhaps fewer.
+__host__ __device__ inline int tiles_of(int64_t T) { return (int)((T + XR_T - 1) / XR_T); }
+// The wave-role GEMM X and the fused Y + Z launch fetch, multiply and do not
+// store a sequence's last tile's missing rows, which the 256-row tiles of the
+// separate GEMMs pack away; they still win while at least half of their rows
+// are tokens (B2 T777 N8192 D256: X 76 -> 60 us, Y and Z 147 -> 110).
+bool tiles_filled(int64_t T) { return (int64_t)tiles_of(T) * XR_T <= 2 * T; }
+// Rows past a buffer's last that those tiles may fetch.
+constexpr int64_t kTilePad = XR_T;
 constexpr int XR_EBLK = XR_T * BK * 2;         // bytes of one 32-deep block of 128 rows
 constexpr int XR_EMAX = (T256 / BK) * XR_EBLK; // encoder chunk, D <= 256
 constexpr int XR_RING = 3;
@@ -376,7 +386,8 @@ __global__ __launch_bounds__(64 * (XR_MW + XR_DW + XR_SW), 1) void layer_x_roles
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   if (tid < 20) counts[tid] = 0;
   __syncthreads();
-  const int ct = (int)(g.H * g.N / XR_T), mt = (int)(g.M / XR_T);
+  const int tps = tiles_of(g.T);  // row tiles of a sequence
+  const int ct = (int)(g.H * g.N / XR_T), mt = (int)g.B * tps;
   const int ctile = (int)blockIdx.x % ct, rg = (int)blockIdx.x / ct;
   const int ntile = (mt - rg + rg_count - 1) / rg_count;  // row tiles rg, rg + rg_count, ...
   const int nk = (int)(g.D / BK);
@@ -464,9 +475,11 @@ __global__ __launch_bounds__(64 * (XR_MW + XR_DW + XR_SW), 1) void layer_x_roles
       dma16(Eg, src(i) + (uint32_t)(sblk * 64), lE + (uint32_t)(sblk * XR_EBLK + i * 1024));
     }
     const uint32_t cs0 = src(dw), cs1 = src(dw + XR_DW);
-    const bf16_t* cg = g.a + (int64_t)rg * XR_T * g.D;
-    const int64_t cstep = (int64_t)rg_count * XR_T * g.D;
-    int sk = 0, slot = 0;
+    auto tile_rows = [&](int tile) {
+      return g.a + ((int64_t)(tile / tps) * g.T + (int64_t)(tile % tps) * XR_T) * g.D;
+    };
+    int sk = 0, slot = 0, tile = rg;
+    const bf16_t* cg = tile_rows(tile);
     uint32_t seen = 0;
     for (int j = 0; j < J; ++j) {
       // Slot j % 3 held step j - 3: free once every MFMA wave has read it.
@@ -477,7 +490,8 @@ __global__ __launch_bounds__(64 * (XR_MW + XR_DW + XR_SW), 1) void layer_x_roles
       slot = slot == XR_RING - 1 ? 0 : slot + 1;
       if (++sk == nk) {
         sk = 0;
-        cg += cstep;
+        tile += rg_count;
+        cg = tile_rows(tile < mt ? tile : rg);
       }
       // Step j - 1 (this wave's part; with step 0 the encoder chunk) has
       // landed once only step j's 2 DMAs are in flight.
@@ -500,11 +514,12 @@ __global__ __launch_bounds__(64 * (XR_MW + XR_DW + XR_SW), 1) void layer_x_roles
 #pragma unroll
     for (int j = 0; j < 4; ++j) fq[j] = g.freqs[n0 + 8 * li + 2 * j];
   }
-  int64_t obase = 0, pbase = 0;  // of the staged tile: offset of its token 0, that token's position
+  int64_t obase = 0, pbase = 0;  // of the staged tile: offset of its token 0, that token in its sequence
   auto store_piece = [&](int u) {
     const int tl = (XR_T / XR_SW) * sw + 4 * u + gq;
     const int64_t o = obase + (int64_t)tl * g.N;
     const int64_t t = pbase + tl;
+    if (t >= g.T) return;
     const float4 lo = *reinterpret_cast<const float4*>(stg + xr_stg(tl, 8 * li));
     const float4 hi = *reinterpret_cast<const float4*>(stg + xr_stg(tl, 8 * li + 4));
     const float r[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
@@ -530,15 +545,12 @@ __global__ __launch_bounds__(64 * (XR_MW + XR_DW + XR_SW), 1) void layer_x_roles
   };
   // Per tile: once every MFMA wave has staged it, the tile's pieces are read
   // from staging, formed and stored; then this wave's freed counter says so.
-  int64_t row0 = (int64_t)rg * XR_T;  // first token row (b * T + t) of the tile
   uint32_t seen = 0;
   for (int i = 0; i < ntile; ++i) {
     wave_wait_min<4>(staged, (uint32_t)(i + 1), seen);
-    // A tile lies inside one sequence (T % 128 == 0).
-    const int64_t bb = row0 / g.T, t0 = row0 - bb * g.T;
-    obase = ((bb * g.H + h) * g.T + t0) * g.N + n0 + 8 * li;
-    pbase = t0;
-    row0 += (int64_t)rg_count * XR_T;
+    const int tile = rg + i * rg_count, bb = tile / tps;
+    pbase = (int64_t)(tile - bb * tps) * XR_T;
+    obase = (((int64_t)bb * g.H + h) * g.T + pbase) * g.N + n0 + 8 * li;
 #pragma unroll
     for (int u = 0; u < XR_PC; ++u) store_piece(u);
     // The pieces' staging reads are complete (their values went into the
@@ -548,8 +560,9 @@ __global__ __launch_bounds__(64 * (XR_MW + XR_DW + XR_SW), 1) void layer_x_roles
 }
 
 // ---- GEMM Y fused into GEMM Z --------------------------------------------
-// With T a multiple of 256 and D <= 256 the layer never writes y.  One
-// workgroup (8 waves, one per CU) owns a 256-token tile (one sequence) and a
+// With D <= 256 the layer never writes y.  One workgroup (4 waves, two per
+// CU) owns a 128-token tile of one sequence (the last one's missing rows are
+// fetched and multiplied, not stored) and a
 // range of 128-latent chunks of H N, and per chunk
 //   Y^T  = Ev_chunk a_h^T        [128 latents x 256 tokens], K = D
 //   y    = act(Y) * x            bf16, into LDS as the next product's A operand
@@ -632,7 +645,8 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void layer_yz_kernel(LayerGemmArgs
   const int nc = (int)(HN / YZ_C), cpn = (int)(g.N / YZ_C);  // chunks, chunks per head
   const int jb = (int)((int64_t)nc * kp / g.ks), je = (int)((int64_t)nc * (kp + 1) / g.ks);
   const int ny = (int)(g.D / BK), per = ny + 4;  // Y steps, then 4 z steps, per chunk
-  const int64_t m0 = (int64_t)mtile * TM, bb = m0 / g.T, t0 = m0 - bb * g.T;
+  const int tps = tiles_of(g.T);
+  const int64_t bb = mtile / tps, t0 = (int64_t)(mtile - (int)bb * tps) * TM;
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_addr(lds));
   // DMA lanes (16 rows of 64 bytes per instruction): the lane writing slot
   // c of row r fetches chunk c ^ ((r >> 1) & 3), the swizzle of lds_off.
@@ -816,8 +830,8 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void layer_yz_kernel(LayerGemmArgs
   }
   dma_wait_barrier<0>();  // the epilogue reuses the ring
   epilogue_64x128(accz, reinterpret_cast<bf16_t*>(lds), w, lane, [&](int row, int col, float4 v) {
-    const int64_t m = m0 + 64 * zm + row, d = 128 * zd + col;
-    if (d < g.D) *reinterpret_cast<float4*>(&g.zpart[((int64_t)kp * g.M + m) * g.D + d]) = v;
+    const int64_t t = t0 + 64 * zm + row, m = bb * g.T + t, d = 128 * zd + col;
+    if (t < g.T && d < g.D) *reinterpret_cast<float4*>(&g.zpart[((int64_t)kp * g.M + m) * g.D + d]) = v;
   });
 }
 
@@ -1006,25 +1020,28 @@ __global__ __launch_bounds__(256) void residual_kernel(const float* __restrict__
   const float* z = zpart + m * D + lane;
 #pragma unroll
   for (int i = 0; i < PER; ++i) v[i] = z[64 * i];
-  // Partials in order kp = 1, 2, ...; the loads of U splits are issued
-  // before their adds.
-  constexpr int U = PER <= 8 ? 4 : 1;
+  // Partials in order kp = 1, 2, ...; the loads of a group of splits are
+  // issued before their adds (groups of 16, then 4: with 4 alone the 31
+  // partials of a few-row decoder were 8 memory round trips).
   const int64_t zs = M * D;
   int kp = 1;
-  for (; kp + U <= ks; kp += U) {
-    float t[U][PER];
+  auto add = [&](auto count) {
+    constexpr int U = decltype(count)::value;
+    for (; kp + U <= ks; kp += U) {
+      float t[U][PER];
 #pragma unroll
-    for (int j = 0; j < U; ++j)
+      for (int j = 0; j < U; ++j)
 #pragma unroll
-      for (int i = 0; i < PER; ++i) t[j][i] = z[(kp + j) * zs + 64 * i];
+        for (int i = 0; i < PER; ++i) t[j][i] = z[(kp + j) * zs + 64 * i];
 #pragma unroll
-    for (int j = 0; j < U; ++j)
+      for (int j = 0; j < U; ++j)
 #pragma unroll
-      for (int i = 0; i < PER; ++i) v[i] += t[j][i];
-  }
-  for (; kp < ks; ++kp)
-#pragma unroll
-    for (int i = 0; i < PER; ++i) v[i] += z[kp * zs + 64 * i];
+        for (int i = 0; i < PER; ++i) v[i] += t[j][i];
+    }
+  };
+  if constexpr (PER <= 4) add(std::integral_constant<int, 16>{});
+  if constexpr (PER <= 8) add(std::integral_constant<int, 4>{});
+  add(std::integral_constant<int, 1>{});
   ln_wave<PER>(v, D);
 #pragma unroll
   for (int i = 0; i < PER; ++i) v[i] += cur[m * D + lane + 64 * i];
@@ -1113,14 +1130,14 @@ hipError_t launch_gemm(const LayerGemmArgs& g, hipStream_t st) {
 
 // Row-tile groups of the two-role GEMM X (layer_x_roles_kernel), or 0 where
 // the shape needs layer_gemm_kernel<G_X>: x wanted in f32 (the decode step),
-// few rows, T or N not a multiple of 128, D not a multiple of 32, under 64
-// or above 256, or more 128-latent column tiles than CUs.  A workgroup per column
+// few rows, mostly empty row tiles, N not a multiple of 128, D not a multiple
+// of 32, under 64 or above 256, or more 128-latent column tiles than CUs.  A workgroup per column
 // tile and group; the groups split the row tiles.
 int x_roles_groups(const LayerGemmArgs& g) {
-  if (g.xf || g.M <= SK_MAXM || g.T % XR_T != 0 || g.N % XR_T != 0 || g.D % BK != 0 || g.D < 2 * BK ||
+  if (g.xf || g.M <= SK_MAXM || !tiles_filled(g.T) || g.N % XR_T != 0 || g.D % BK != 0 || g.D < 2 * BK ||
       g.D > T256)
     return 0;
-  const int64_t ct = g.H * g.N / XR_T, mt = g.M / XR_T, cus = device_cus();
+  const int64_t ct = g.H * g.N / XR_T, mt = g.B * tiles_of(g.T), cus = device_cus();
   if (ct > cus) return 0;
   const int64_t r = cus / ct;
   return (int)(r < mt ? r : mt);
@@ -1138,21 +1155,26 @@ hipError_t launch_x(const LayerGemmArgs& g, hipStream_t st) {
 }
 
 // Split count of the fused Y + Z launch over the 128-latent chunks, or 0
-// where the shape needs GEMM Y and GEMM Z apart: T a multiple of 256 (a
-// token tile inside one sequence), D a multiple of 64 up to 256 (the z tile),
-// DMA offsets within 32 bits.  About one workgroup per CU, with at least 4
-// chunks each where the chunks allow (C5: 64 token tiles x 4 splits of 64).
+// where the shape needs GEMM Y and GEMM Z apart: few rows or mostly empty
+// token tiles, D not a multiple of 64 or above 256 (the z tile), DMA offsets
+// past 32 bits.  As many as fill two workgroups a CU, with at least 4 chunks
+// each where the chunks allow, and no more than needed for the same longest
+// range (C5: 128 token tiles x 4 splits of 64 chunks; 14 tiles and 256
+// chunks: 32 of 8, not 36: every split writes one more set of partials).
 constexpr int YZ_NW = 4;  // waves of the fused launch: 128-token tiles, two workgroups a CU
 constexpr int YZ_TM = YZGeom<YZ_NW>::TM;
+static_assert(YZ_TM == XR_T, "one tiling of the sequences");
 
 int yz_splits(int64_t M, int64_t H, int64_t T, int64_t N, int64_t D) {
-  if (M <= SK_MAXM || T % YZ_TM != 0 || D % 64 != 0 || D > T256) return 0;
+  if (M <= SK_MAXM || !tiles_filled(T) || D % 64 != 0 || D > T256) return 0;
   const int64_t HN = H * N;
   if (HN % YZ_C != 0 || (int64_t)YZ_TM * N * 2 >= ((int64_t)1 << 32)) return 0;
-  const int64_t tiles = M / YZ_TM, nc = HN / YZ_C;
+  const int64_t tiles = M / T * tiles_of(T), nc = HN / YZ_C;
   int64_t ks = (int64_t)device_cus() * (8 / YZ_NW) / tiles;
   if (ks > nc / 4) ks = nc / 4;
-  return (int)(ks < 1 ? 1 : ks);
+  if (ks < 1) ks = 1;
+  const int64_t longest = (nc + ks - 1) / ks;
+  return (int)((nc + longest - 1) / longest);
 }
 
 hipError_t launch_yz(const LayerGemmArgs& g, hipStream_t st) {
@@ -1299,9 +1321,9 @@ bdh_status run_layer(const LayerArgs& a, hipStream_t st, uint64_t* launches) {
       if (tiles_z * cand >= 512) break;
     }
   }
-  bdh_status s = scratch(st, SLOT_LAYER_CUR, (size_t)(M * a.D) * sizeof(bf16_t), &curb);
+  bdh_status s = scratch(st, SLOT_LAYER_CUR, (size_t)((M + kTilePad) * a.D) * sizeof(bf16_t), &curb);
   if (s != BDH_OK) return s;
-  s = scratch(st, SLOT_LAYER_XY, (size_t)(S * a.T * a.N) * sizeof(bf16_t), &xy);
+  s = scratch(st, SLOT_LAYER_XY, (size_t)((S * a.T + kTilePad) * a.N) * sizeof(bf16_t), &xy);
   if (s != BDH_OK) return s;
   // q: rope(x) in bf16 for the MFMA attention, or x in f32 for the decode
   // step (which rotates as it gathers).
@@ -1315,7 +1337,7 @@ bdh_status run_layer(const LayerArgs& a, hipStream_t st, uint64_t* launches) {
   }
   s = scratch(st, SLOT_LAYER_ATTN, (size_t)(S * a.T * a.D) * sizeof(float), &attn);
   if (s != BDH_OK) return s;
-  s = scratch(st, SLOT_LAYER_AN, (size_t)(S * a.T * a.D) * sizeof(bf16_t), &an);
+  s = scratch(st, SLOT_LAYER_AN, (size_t)((S * a.T + kTilePad) * a.D) * sizeof(bf16_t), &an);
   if (s != BDH_OK) return s;
   s = scratch(st, SLOT_LAYER_Z, (size_t)(ks * M * a.D) * sizeof(float), &zp);
   if (s != BDH_OK) return s;
@@ -1395,7 +1417,7 @@ bdh_status run_layer(const LayerArgs& a, hipStream_t st, uint64_t* launches) {
   g.b = a.encv;
   if (ks_yz > 0) {
     g.dec = a.dec;
-    g.mt = (int)(M / YZ_TM);
+    g.mt = (int)a.B * tiles_of(a.T);
     g.ks = ks;
     g.zpart = (float*)zp;
     BDH_HIP_TRY(launch_yz(g, st));

@@ -18,6 +18,7 @@
 // RoPE is applied to Q tiles between HBM and LDS, each lane computing the
 // (cos, sin) of its pairs from the f32 phase; with one interval rotated
 // queries are never written to memory.
+#include <algorithm>
 #include <cstdlib>
 #include <type_traits>
 
@@ -237,6 +238,7 @@ hipError_t launch_ctx_wc(const CtxArgs& c, int ks, hipStream_t st) {
   switch (ks) {
     case 1: hipLaunchKernelGGL((ctx_kernel<1, WC, P16>), grid, dim3(256), 0, st, c); break;
     case 2: hipLaunchKernelGGL((ctx_kernel<2, WC, P16>), grid, dim3(256), 0, st, c); break;
+    case 3: hipLaunchKernelGGL((ctx_kernel<3, WC, P16>), grid, dim3(256), 0, st, c); break;
     case 4: hipLaunchKernelGGL((ctx_kernel<4, WC, P16>), grid, dim3(256), 0, st, c); break;
     case 8: hipLaunchKernelGGL((ctx_kernel<8, WC, P16>), grid, dim3(256), 0, st, c); break;
     default: return hipErrorInvalidValue;
@@ -413,6 +415,28 @@ int device_cus() {
 constexpr size_t kCarrySnapMax = (size_t)8 << 30;
 
 namespace {
+// Time model (us) of the 8-wave gram and readout tiles (snap_wide.hip, one
+// workgroup a CU) over `units` tiles of nk steps split in k N ranges: a step
+// 0.75 us, a unit's prologue and epilogue 8 us; `mb` MB of partials a range,
+// each written and read at 4.5 MB/us.  (C4, chunk 512: 1, 2 and 4 ranges 463,
+// 406 and 446 us; measured 2 fastest.  Few tiles leave CUs idle until the
+// ranges fill them: 80 tiles of 256 steps, layer B2 T777 N8192: 1 range 205,
+// 2 104, 3 72 + partials.)
+double snap_time(int64_t units, int nk, int k, double mb) {
+  const int64_t slots = device_cus();
+  return (double)((units * k + slots - 1) / slots) * (0.75 * nk / k + 8.0) + 2.0 * k * mb / 4.5;
+}
+// The fastest count of N ranges by that model; at least 8 steps a range, and
+// with `even` an even number of them.
+int snap_ranges(int64_t units, int nk, double mb, bool even) {
+  int best = 1;
+  for (const int k : {2, 3, 4, 8}) {
+    if (nk / k < 8 || (even && nk % (2 * k) != 0)) continue;
+    if (snap_time(units, nk, k, mb) < snap_time(units, nk, best, mb)) best = k;
+  }
+  return best;
+}
+
 // Two or more intervals, no decay: v^T, the state-carry kernel (which also
 // rotates x once and writes q), one launch of every interval's gram tiles
 // and readouts (from the bf16 snapshots), then the context kernel, which
@@ -424,21 +448,14 @@ bdh_status run_carry_path(const Bf16Args& a, hipStream_t st, uint64_t* launches,
   const int64_t rd_iv0 = a.rho_in ? 0 : 1;
   // Gram and readout tiles run in 8-wave workgroups (snap_wide.hip, one per
   // CU); an interval's readout tiles join its gram group (same N range, same
-  // XCD, dispatched together): they read the same q rows.  N splits: 1 or 2,
-  // whichever gives the fewer steps in rounds of units over the CUs, 1 on a
-  // tie (every split writes, and the context kernel re-reads, one more set
-  // of partials).  Measured at C4: chunk 1024 (a tie) 0.83 ms with 1 split,
-  // 0.88 with 2; chunk 512 0.875 with 2, 0.889 with 1; 4 splits (the fewest
-  // rounds at 512 and 1024) made the context kernel read twice as much
-  // (chunk 512: 157 against 58 us) and the call 0.93-0.98 ms; 3 splits at
-  // chunk 512 (4 rounds of 86 steps against 3 of 128) took the gram/readout
-  // and carry launches 0.614 -> 0.602 ms but the call 0.745 -> 0.777 ms.
+  // XCD, dispatched together): they read the same q rows.  N ranges by
+  // snap_ranges (every range writes, and the context kernel re-reads, one
+  // more set of partials).
   const int ndb256 = (int)cdiv(a.D, T256);
   const int rd_pg = nb * ndb256;
-  const int64_t slots = device_cus();
-  const int64_t upg = (int64_t)nb * (nb - 1) / 2 + nb + rd_pg;
-  auto rounds = [&](int k) { return (S * n_iv * k * upg + slots - 1) / slots * (nk / k); };
-  const int ks = (nk % 2 == 0 && rounds(2) < rounds(1)) ? 2 : 1;
+  const int64_t upg = (int64_t)nb * (nb + 1) / 2;
+  const int ks = snap_ranges(S * n_iv * (upg + rd_pg), nk,
+                             ((double)S * n_iv * upg * T256 * T256 + (double)S * a.T * a.D) * 4e-6, false);
   const int kr = ks;
 
   void *vt = nullptr, *part = nullptr, *snap = nullptr, *rdp = nullptr, *q = nullptr;
@@ -502,7 +519,7 @@ bdh_status run_carry_path(const Bf16Args& a, hipStream_t st, uint64_t* launches,
   ktime_end(kt, st);
 
   CtxArgs cx{(const bf16_t*)vt, (const float*)part, a.ctx, a.H, a.Hv, a.T, a.D, L, Lp, Tp, Dp, S,
-             n_iv, 0, (int)n_iv, (int)cdiv(L, CTX_ROWS), (const float*)rdp, kr, rd_iv0};
+             n_iv, 0, (int)n_iv, (int)cdiv(std::min(L, a.T), CTX_ROWS), (const float*)rdp, kr, rd_iv0};
   BDH_HIP_TRY(launch_ctx(cx, ks, st));
   if (launches) *launches += 4;
   return BDH_OK;
@@ -514,19 +531,13 @@ bdh_status run_carry_path(const Bf16Args& a, hipStream_t st, uint64_t* launches,
 // suits them (whole 256-row blocks, an even step count per N range), else in
 // 8-wave workgroups (snap_wide.hip, the tiles of the state-carry form without
 // readouts).  Measured at C5 (same box): 4-wave tiles 10.97-11.06 ms a
-// forward against 11.18-11.22 ms.  N splits:
-// the fewest of 1, 2 or 4 with the fewest steps in rounds of units over the
-// CUs.  (The layer's attention runs here: the layer rotates q in its GEMM
+// forward against 11.18-11.22 ms.  N ranges by snap_ranges.  (The layer's attention runs here: the layer rotates q in its GEMM
 // epilogue.)
 bdh_status run_gram_path(const Bf16Args& a, hipStream_t st, uint64_t* launches, int64_t S, int64_t Tp,
                          int64_t Dp, int64_t Lp, int nb, int nk) {
   const int64_t L = a.L;
-  const int64_t slots = device_cus();
-  const int64_t upg = (int64_t)nb * (nb - 1) / 2 + nb;
-  auto rounds = [&](int k) { return (S * k * upg + slots - 1) / slots * (nk / k); };
-  int ks = 1;
-  for (int cand = 2; cand <= 4 && nk % (2 * cand) == 0; cand *= 2)
-    if (rounds(cand) < rounds(ks)) ks = cand;
+  const int64_t upg = (int64_t)nb * (nb + 1) / 2;
+  const int ks = snap_ranges(S * upg, nk, (double)S * upg * T256 * T256 * (a.part16 ? 2e-6 : 4e-6), true);
 
   void *vt = nullptr, *part = nullptr;
   bdh_status stt = scratch(st, SLOT_VT, (size_t)(a.B * a.Hv * Dp * Tp) * sizeof(bf16_t), &vt);
@@ -655,7 +666,13 @@ bdh_status run_bf16_path(const Bf16Args& a, hipStream_t st, uint64_t* launches) 
   const int nk = (int)(a.N / 32);  // 32-deep gram steps
   const int state_units = prefill_state_units(S, a.N, a.D);
   // (The readout units address a snapshot's rows with 32-bit offsets.)
-  if (a.state && n_iv >= 2 && a.D * a.N * 2 < ((int64_t)1 << 31) &&
+  // One interval with a carried state takes the state-carry form (which reads
+  // rho once, for its snapshot and its successor) from 24 M elements of x on:
+  // B8 nh4 T300 N8192 D256 422 against 365 us, T512 498 against 457, B8 T400
+  // N2048 in place 235 against 224; below, its launches cost more (B1 T512
+  // N8192 104 against 121 us, B4 T256 N4096 95 against 112).
+  const bool carried1 = a.rho_in != nullptr && S * a.T * a.N >= ((int64_t)24 << 20);
+  if (a.state && (n_iv >= 2 || carried1) && a.D * a.N * 2 < ((int64_t)1 << 31) &&
       (size_t)(n_iv * S * a.N * a.D) * sizeof(bf16_t) <= kCarrySnapMax)
     return run_carry_path(a, st, launches, S, Tp, Dp, n_iv, Lp, nb, nk);
   if (!a.state && a.rho_in == nullptr && a.freqs == nullptr && a.decay == nullptr && n_iv == 1)
@@ -816,7 +833,9 @@ bdh_status run_bf16_path(const Bf16Args& a, hipStream_t st, uint64_t* launches) 
     }
     if (iv == 0) {
       // tril(S) V of every interval: the gram partials are all written by
-      // the first launch.
+      // the first launch.  (Adding one interval's readout partials here too
+      // was slower than their own launch: few workgroups, 16 partials after
+      // one another: B1 T512 N8192 104 -> 116 us.)
       CtxArgs c{(const bf16_t*)vt, (const float*)part, a.ctx, a.H, a.Hv, a.T, a.D, L, Lp, Tp, Dp, S,
                 n_iv, 0, (int)(a.state ? n_iv : 1), (int)cdiv(Lc0, CTX_ROWS), nullptr, 0, 0};
       BDH_HIP_TRY(launch_ctx(c, ks, st));

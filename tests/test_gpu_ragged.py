@@ -1,0 +1,73 @@
+"""Sequences whose length is no multiple of a tile: the layer's 128-token
+tiles with missing rows (bdh_lowrank_layer_fwd), and a call of one interval
+that continues a state, on both of its routes."""
+import numpy as np
+import pytest
+
+from tests.gpu_util import TOL_BF16, announce, dev, host, need_gpu, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("B,H,T,N,D,carried", [
+    (2, 2, 65, 256, 64, False),    # one tile a sequence, just over half filled
+    (2, 2, 63, 256, 64, True),     # under half: the separate GEMMs
+    (3, 1, 129, 256, 128, True),   # a second tile of one row
+    (1, 2, 255, 512, 256, False),  # one row short of two tiles
+    (5, 2, 200, 256, 192, True),   # ten tiles, splits of unequal chunk counts
+])
+def test_layer_tiles_match_oracle(oracle, B, H, T, N, D, carried):
+    torch = need_gpu()
+    import burn_dragon_amd as bd
+    rng = np.random.default_rng(T * 3 + N)
+    cur = oracle.layer_norm_f64(rng.standard_normal((B, T, D))).astype(np.float32)
+    enc, encv = ((rng.standard_normal((H, D, N)) * 0.05).astype(np.float32) for _ in range(2))
+    dec = (rng.standard_normal((H * N, D)) * 0.05).astype(np.float32)
+    rho0 = (rng.standard_normal((B, H, N, D)) * 0.05).astype(np.float32) if carried else None
+    w = bd.LowRankWeights.pack(dev(torch, enc[None]), dev(torch, encv[None]), dev(torch, dec))
+    announce("layer tiles", B, H, T, N, D, carried)
+    # Scratch rows past the last token hold whatever was there: make it NaN.
+    big = torch.full((B, T + 200, D), float("nan"), device="cuda")
+    bd.lowrank_layer_forward(big, w, position=0)
+    out = bd.lowrank_layer_forward(dev(torch, cur), w, position=7, rho=dev(torch, rho0) if carried else None,
+                                   want_rho=carried)
+    torch.cuda.synchronize()
+    nref, rref = oracle.lowrank_layer_f64(cur, oracle.round_bf16(enc), oracle.round_bf16(encv),
+                                          oracle.round_bf16(dec), pos0=7, rho0=rho0)
+    assert rel_l2(host(out.next), nref) <= TOL_BF16
+    if carried:
+        assert rel_l2(host(out.rho), rref) <= TOL_BF16
+
+
+@pytest.mark.parametrize("B,T,N,D,rope,decay,inplace", [
+    (1, 130, 512, 96, 5, None, False),                          # few elements: gram, readout and state units
+    (1, 130, 512, 96, None, [0.99, 0.98, 0.97, 0.96], True),
+    (2, 390, 8192, 64, 5, None, False),                         # many: the state-carry form
+    (2, 390, 8192, 64, 5, None, True),
+    (2, 390, 8192, 64, None, [0.99, 0.98, 0.97, 0.96], False),
+])
+def test_one_interval_onto_a_state(oracle, B, T, N, D, rope, decay, inplace):
+    torch = need_gpu()
+    import burn_dragon_amd as bd
+    H = 4
+    rng = np.random.default_rng(N + T)
+    x = oracle.round_bf16(np.maximum(rng.standard_normal((B, H, T, N), dtype=np.float32) - 1.645, 0))
+    v = oracle.round_bf16(rng.standard_normal((B, 1, T, D), dtype=np.float32) / 16)
+    rho0 = (rng.standard_normal((B, H, N, D)) * 0.2).astype(np.float32)
+    d = np.array(decay, np.float32) if decay else None
+    announce("one interval onto a state", B, T, N, D, rope, decay, inplace)
+    tx, tv = dev(torch, x, torch.bfloat16), dev(torch, v, torch.bfloat16)
+    tr, td = dev(torch, rho0), dev(torch, d) if decay else None
+    kw = dict(inplace=inplace)
+    out = (bd.try_fused_recurrent_attention(tx, tv, tr, td, **kw) if rope is None else
+           bd.try_fused_recurrent_attention_rope(tx, tv, tr, td, position=rope, **kw))
+    torch.cuda.synchronize()
+    assert (out.rho.data_ptr() == tr.data_ptr()) == inplace
+    if not inplace:
+        assert np.array_equal(host(tr), rho0)
+    for b, h in ((0, 0), (B - 1, 3)):
+        q = x[b:b + 1, h:h + 1]
+        q = q if rope is None else oracle.rope_rotate(q, pos0=rope)
+        ctx, rho = oracle.recurrent_f64(q, v[b:b + 1], rho0[b:b + 1, h:h + 1], d[h:h + 1] if decay else None)
+        assert rel_l2(host(out.context[b, h]), ctx[0, 0]) <= TOL_BF16
+        assert rel_l2(host(out.rho[b, h]), rho[0, 0]) <= TOL_BF16
