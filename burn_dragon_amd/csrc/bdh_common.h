@@ -91,4 +91,32 @@ __device__ __forceinline__ floatx16 zero16() {
   return z;
 }
 
+// Wave-wide sum (fixed butterfly order: the same result in every lane).
+__device__ __forceinline__ float wave_sum(float v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  return v;
+}
+
+constexpr int LN_MAX = 32;  // D / 64 values per lane (D <= 2048)
+
+// LayerNorm of one D-row held 64-strided across the wave's lanes, in place:
+// (v - mean) / sqrt(var + eps), biased variance, two passes.
+template <int PER>
+__device__ __forceinline__ void ln_wave(float (&v)[LN_MAX], int D) {
+  float s = 0.0f;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) s += v[i];
+  const float mean = wave_sum(s) / (float)D;
+  float q = 0.0f;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    v[i] -= mean;
+    q += v[i] * v[i];
+  }
+  const float den = sqrtf(wave_sum(q) / (float)D + 1e-5f);
+#pragma unroll
+  for (int i = 0; i < PER; ++i) v[i] /= den;
+}
+
 }  // namespace bdh

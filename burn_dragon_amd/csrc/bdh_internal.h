@@ -37,9 +37,8 @@ enum ScratchSlot {
   SLOT_LAYER_AN,     // its LayerNorm (bf16)         [B, H, T, D]
   SLOT_LAYER_Z,      // decoder split-K partials     [ks, B*T, D] f32
   SLOT_LAYER_RHO,    // a successor state not kept   [B, H, N, D] f32
-  SLOT_DECODE_PART,  // decode range readouts        [S, G, D] f32
-  SLOT_DECODE_IDX,   // decode range active lists    [S, N] int32
-  SLOT_DECODE_CNT,   // decode range active counts   [S, G] int32
+  SLOT_DECODE_PART,  // decode range readouts [S, G, D] f32, lists and counts (decode_part_bytes)
+  SLOT_DECODE_CTR,   // decode: ranges of a stream that have finished  [CUs] uint32, 0 between launches
   SLOT_VJP_S,        // VJP scores tril(QQ^T) * D    [S, T, T] f32
   SLOT_VJP_M,        // VJP tril(G V^T)*D + its transpose  [S, T, T] f32
   SLOT_VJP_TD,       // VJP per-head grad_v, IC, G*d^t  3 x [S, T, D] f32
@@ -157,6 +156,7 @@ bdh_status lm_logits(const float* hidden, int64_t M, int64_t D, const bf16_t* he
 // the sparse step (only the active rows are read and written).  Otherwise
 // the dense step: every row of rho_in (zeros when null) is read and written
 // to rho, rho = (rho_in + rot(x)^T v) * decay, in place or not.
+constexpr int64_t kDecodeNormMaxD = 256;
 struct DecodeArgs {
   const float* x;       // [S, N]
   const float* v;       // [B, Hv, D]
@@ -169,6 +169,9 @@ struct DecodeArgs {
   int32_t* idx_out;     // [S, N] or null
   int32_t* cnt_out;     // [S] or null
   int64_t B, H, Hv, N, D;
+  // LayerNorm of a (gamma 1, beta 0) in bf16 [S, D] in place of a_out, or
+  // null; the sparse step, D % 64 == 0 and at most kDecodeNormMaxD.
+  bf16_t* an = nullptr;
   // Buffers for the range readouts and lists of a split stream; null: the
   // stream's scratch.
   void* part_buf = nullptr;

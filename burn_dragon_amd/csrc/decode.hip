@@ -21,9 +21,14 @@
 // (recurrent.rs:259) and its per-row update (recurrent.rs:415) in one pass.
 //
 // Readouts are reduced across waves in LDS in a fixed order; with G > 1 the
-// range partials (and range lists) go to a range buffer and a finalize kernel
-// sums them (and concatenates the lists) in range order, so results are
-// deterministic and no atomics or cross-workgroup fences are needed.
+// range partials go to a range buffer, and the last of a stream's workgroups
+// to finish sums them in range order, so the result is deterministic.  Where
+// the active lists are asked for, the step is dense, or the buffers are a
+// caller's (which overlapping calls may share), a finalize kernel sums the
+// partials (and concatenates the lists) instead.  At C3's shape with B = 1
+// (4 streams of 16 ranges) the finalize launch was 4.4 of 14.3 us.
+#include <type_traits>
+
 #include "bdh_internal.h"
 
 namespace bdh {
@@ -33,6 +38,7 @@ constexpr int DR_THREADS = 1024;
 constexpr int DR_WAVES = DR_THREADS / 64;
 constexpr int DR_SEG = 8192;       // rows compacted per pass (LDS list capacity)
 constexpr int DR_UNROLL = 8;
+constexpr int DR_MAXG = 16;        // row ranges of a stream
 constexpr int ROWS_PER_THREAD = 8;  // 4 whole (even, odd) RoPE pairs
 constexpr int DD_THREADS = 256;     // dense step
 constexpr int DD_WAVES = DD_THREADS / 64;
@@ -52,6 +58,9 @@ struct DecodeKernelArgs {
   int H, Hv, N, D;
   int G, rows;        // ranges per stream, rows per range (a multiple of 8)
   float pos;
+  uint32_t* ctr;      // sparse step, G > 1: ranges of each stream done [S] (0 before and after), or null: finalize launch
+  float* a_final;     // with ctr: [S, D]
+  bf16_t* an;         // LayerNorm of the readout [S, D] in its place, or null (D <= 256)
 };
 
 template <bool VEC4>
@@ -141,6 +150,8 @@ __global__ __launch_bounds__(DR_THREADS) void decode_kernel(DecodeKernelArgs p) 
   __shared__ float lval[DR_SEG];
   __shared__ __attribute__((aligned(16))) float red[DR_WAVES * CB];
   __shared__ int32_t wtot[DR_WAVES];
+  __shared__ float whole[kDecodeNormMaxD];  // the readout, for its LayerNorm
+  __shared__ uint32_t arrived;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t s = blockIdx.x / p.G;
@@ -234,9 +245,63 @@ __global__ __launch_bounds__(DR_THREADS) void decode_kernel(DecodeKernelArgs p) 
       float sum = red[cc];
 #pragma unroll
       for (int w = 1; w < DR_WAVES; ++w) sum += red[w * CB + cc];
-      if (cb + cc < p.D) a_s[cb + cc] = sum;
+      if (cb + cc >= p.D) continue;
+      if (p.ctr) __hip_atomic_store(a_s + cb + cc, sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      else if (p.an && p.G == 1) whole[cb + cc] = sum;
+      else a_s[cb + cc] = sum;
     }
     __syncthreads();
+  }
+  if (p.ctr) {
+    // The last range of the stream to get here sums all of them.  Every value
+    // that crosses workgroups is stored and loaded by device-scope atomic
+    // accesses, which go past the XCDs' own L2 caches: once a wave's stores
+    // have been acknowledged (vmcnt 0) they are where the other XCDs' loads
+    // look, so counting after that wait and the barrier orders them, without
+    // a release fence's write-back of the whole L2 (394 us a step at C3).
+    // (Only the waves that stored partials have anything to wait for: the
+    // others' rho rows are read by later launches alone.)
+    if (wave * 64 < CB) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (tid == 0) {
+      arrived = __hip_atomic_fetch_add(p.ctr + s, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (arrived == (uint32_t)p.G - 1)
+        __hip_atomic_store(p.ctr + s, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (arrived != (uint32_t)p.G - 1) return;
+    const float* part = p.a_out + s * p.G * p.D;
+    for (int d = tid; d < p.D; d += DR_THREADS) {
+      float v[DR_MAXG];
+#pragma unroll
+      for (int k = 0; k < DR_MAXG; ++k)
+        v[k] = k < p.G ? __hip_atomic_load(part + k * p.D + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.0f;
+      float sum = v[0];
+#pragma unroll
+      for (int k = 1; k < DR_MAXG; ++k)
+        if (k < p.G) sum += v[k];
+      if (p.an) whole[d] = sum;
+      else p.a_final[s * p.D + d] = sum;
+    }
+    __syncthreads();
+  }
+  if (p.an && wave == 0) {
+    // LayerNorm of the whole readout (D = 64, 128, 192 or 256) by one wave.
+    float v[LN_MAX];
+    auto norm = [&](auto per) {
+      constexpr int PER = decltype(per)::value;
+#pragma unroll
+      for (int i = 0; i < PER; ++i) v[i] = whole[lane + 64 * i];
+      ln_wave<PER>(v, p.D);
+#pragma unroll
+      for (int i = 0; i < PER; ++i) p.an[s * p.D + lane + 64 * i] = (bf16_t)v[i];
+    };
+    switch (p.D / 64) {
+      case 1: norm(std::integral_constant<int, 1>{}); break;
+      case 2: norm(std::integral_constant<int, 2>{}); break;
+      case 3: norm(std::integral_constant<int, 3>{}); break;
+      case 4: norm(std::integral_constant<int, 4>{}); break;
+    }
   }
   if (p.G == 1 && idx_s)
     for (int k = done + tid; k < p.N; k += DR_THREADS) idx_s[k] = -1;
@@ -387,7 +452,7 @@ void decode_ranges(const DecodeArgs& a, int* G, int* rows) {
     // splitting further costs more in partials than it gains.)
     int g = 1;
     const int64_t S = a.B * a.H;
-    while (g < 16 && S * 2 * g <= (int64_t)device_cus() && a.N / (2 * g) >= 256) g *= 2;
+    while (g < DR_MAXG && S * 2 * g <= (int64_t)device_cus() && a.N / (2 * g) >= 256) g *= 2;
     *G = g;
     *rows = (int)(((a.N + g - 1) / g + 7) / 8 * 8);
   } else {
@@ -436,6 +501,11 @@ bdh_status run_decode(const DecodeArgs& a, hipStream_t st, uint64_t* launches) {
   p.G = G;
   p.rows = rows;
   p.pos = a.pos;
+  p.ctr = nullptr;
+  p.a_final = a.a_out;
+  p.an = a.an;
+  if (a.an && (!sparse || a.D % 64 != 0 || a.D > kDecodeNormMaxD || a.idx_out || a.cnt_out || a.part_buf))
+    return fail(BDH_EINVAL, "a normalised readout needs the sparse step and whole rows");
   if (G > 1) {
     const size_t need = decode_part_bytes(a);
     char* buf = (char*)a.part_buf;
@@ -454,6 +524,14 @@ bdh_status run_decode(const DecodeArgs& a, hipStream_t st, uint64_t* launches) {
       buf += align256((size_t)(S * a.N) * sizeof(int32_t));
     }
     if (a.idx_out || a.cnt_out) p.cnt_out = (int32_t*)buf;
+    if (!a.part_buf) {
+      // (S < CUs wherever a sparse step is split.  Kept by every split step on
+      // the stream, so that a later capture of another form finds it.)
+      void* c = nullptr;
+      const bdh_status s = scratch(st, SLOT_DECODE_CTR, (size_t)device_cus() * sizeof(uint32_t), &c, true);
+      if (s != BDH_OK) return s;
+      if (sparse && !a.idx_out && !a.cnt_out) p.ctr = (uint32_t*)c;
+    }
   }
   // Float4 columns need D % 4 == 0 and 16-byte aligned rows.
   const bool vec4 = (a.D % 4) == 0 &&
@@ -499,7 +577,7 @@ bdh_status run_decode(const DecodeArgs& a, hipStream_t st, uint64_t* launches) {
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return hip_fail(e, "decode step launch");
   if (launches) *launches += 1;
-  if (G > 1) {
+  if (G > 1 && !p.ctr) {
     hipLaunchKernelGGL(decode_finalize_kernel, dim3((unsigned)S), dim3(256), 0, st, p.a_out,
                        p.idx_out, p.cnt_out, a.a_out, a.idx_out, a.cnt_out, G, rows, p.N, p.D);
     e = hipGetLastError();

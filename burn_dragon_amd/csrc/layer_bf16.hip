@@ -46,6 +46,7 @@ struct LayerGemmArgs {
   bf16_t* xy;         // X: x out; Y: x in, y out (same place); [B, H, T, N]
   bf16_t* q;          // X: rope(x) out [B, H, T, N], or null (no rotation)
   float* xf;          // X: x out in f32 [B, H, T, N], or null
+  const float* af;    // few rows, X and L: the rows of a in f32 (a unused)
   const float* freqs; // X: RoPE frequencies [N] (with q)
   int64_t pos0;       // X: position of token 0
   int fixed;          // X: every token at pos0
@@ -853,6 +854,10 @@ __global__ __launch_bounds__(256) void skinny_gemm_kernel(LayerGemmArgs g) {
   // column block and a K range, which its 4 waves split and sum through LDS
   // in wave order.  (X, Y: 13 and 15 -> 11 us at C5 decode.)
   constexpr bool WAVECOL = KIND == G_X || KIND == G_Y;
+  // X and the logits take their rows in f32 and round them here (as
+  // to_bf16_kernel does, which was a launch of its own).
+  constexpr bool F32 = KIND == G_X || KIND == G_L;
+  constexpr int CH = F32 ? SK_CHUNK / MB : SK_CHUNK;  // steps loaded at once
   __shared__ floatx4 red[WAVECOL ? 1 : 4][MB][64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int64_t ncols = KIND == G_Z ? g.D : KIND == G_L ? g.V : g.H * g.N;
@@ -871,37 +876,52 @@ __global__ __launch_bounds__(256) void skinny_gemm_kernel(LayerGemmArgs g) {
   int64_t cb = c0 + (lane & 15);
   cb = cb < ncols ? cb : ncols - 1;
   const bf16_t* brow = g.b + (KIND == G_Z ? cb * 128 : cb * K) + kl;
-  const bf16_t* arow[MB];
+  typedef typename std::conditional<F32, float, bf16_t>::type elem;
+  const elem* arow[MB];
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) {
     int64_t m = 16 * mb + (lane & 15);
     m = m < g.M ? m : g.M - 1;
     const int64_t bb = m / g.T, t = m - bb * g.T;
-    if (KIND == G_X || KIND == G_L) arow[mb] = g.a + m * g.D + kl;
+    if constexpr (F32) arow[mb] = g.af + m * g.D + kl;
     else if (KIND == G_Y) arow[mb] = g.a + ((bb * g.H + h) * g.T + t) * g.D + kl;
     else arow[mb] = g.a + (bb * g.H * g.T + t) * g.N + kl;
   }
   floatx4 acc[MB];
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) acc[mb] = zero4();
-  for (int k0 = kb; k0 < ke; k0 += SK_CHUNK) {
-    const int n = ke - k0 < SK_CHUNK ? ke - k0 : SK_CHUNK;
-    bf16x8 bq[SK_CHUNK], aq[SK_CHUNK][MB];
+  for (int k0 = kb; k0 < ke; k0 += CH) {
+    const int n = ke - k0 < CH ? ke - k0 : CH;
+    struct Raw {
+      float4 v[2];
+    };
+    bf16x8 bq[CH];
+    typename std::conditional<F32, Raw, bf16x8>::type aq[CH][MB];
 #pragma unroll
-    for (int s = 0; s < SK_CHUNK; ++s) {
+    for (int s = 0; s < CH; ++s) {
       if (s >= n) break;
       const int64_t k = (int64_t)(k0 + s) * 32;
       // Z: k runs over (head, neuron); a 32-deep step stays inside one head.
       const int64_t aoff = KIND == G_Z ? (k / g.N) * g.T * g.N + k % g.N : k;
       bq[s] = *reinterpret_cast<const bf16x8*>(brow + (KIND == G_Z ? dec_off(0, k, g.D) : k));
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb) aq[s][mb] = *reinterpret_cast<const bf16x8*>(arow[mb] + aoff);
+      for (int mb = 0; mb < MB; ++mb)
+        aq[s][mb] = *reinterpret_cast<const typename std::conditional<F32, Raw, bf16x8>::type*>(arow[mb] + aoff);
     }
 #pragma unroll
-    for (int s = 0; s < SK_CHUNK; ++s) {
+    for (int s = 0; s < CH; ++s) {
       if (s >= n) break;
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb) acc[mb] = mfma16(aq[s][mb], bq[s], acc[mb]);
+      for (int mb = 0; mb < MB; ++mb) {
+        if constexpr (F32) {
+          const Raw& r = aq[s][mb];
+          const uint4 w = make_uint4(pack_bf16x2(r.v[0].x, r.v[0].y), pack_bf16x2(r.v[0].z, r.v[0].w),
+                                     pack_bf16x2(r.v[1].x, r.v[1].y), pack_bf16x2(r.v[1].z, r.v[1].w));
+          acc[mb] = mfma16(__builtin_bit_cast(bf16x8, w), bq[s], acc[mb]);
+        } else {
+          acc[mb] = mfma16(aq[s][mb], bq[s], acc[mb]);
+        }
+      }
     }
   }
   const int64_t c = c0 + (lane & 15);
@@ -960,34 +980,6 @@ __global__ __launch_bounds__(256) void skinny_gemm_kernel(LayerGemmArgs g) {
 #pragma unroll
   for (int ww = 1; ww < 4; ++ww) v = v + red[ww][w][lane];
   emit(w, v);
-}
-
-// Wave-wide sum (fixed butterfly order: the same result in every lane).
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
-
-constexpr int LN_MAX = 32;  // D / 64 values per lane (D <= 2048)
-
-// LayerNorm of one D-row held 64-strided across the wave's lanes, in place:
-// (v - mean) / sqrt(var + eps), biased variance, two passes.
-template <int PER>
-__device__ __forceinline__ void ln_wave(float (&v)[LN_MAX], int D) {
-  float s = 0.0f;
-#pragma unroll
-  for (int i = 0; i < PER; ++i) s += v[i];
-  const float mean = wave_sum(s) / (float)D;
-  float q = 0.0f;
-#pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    v[i] -= mean;
-    q += v[i] * v[i];
-  }
-  const float den = sqrtf(wave_sum(q) / (float)D + 1e-5f);
-#pragma unroll
-  for (int i = 0; i < PER; ++i) v[i] /= den;
 }
 
 // out_bf16[r, :] = LN(in[r, :]) for `rows` rows of D (one wave per row).
@@ -1279,13 +1271,16 @@ bdh_status pack_lm_head(int64_t D, int64_t V, const float* head, bf16_t* packed,
 bdh_status lm_logits(const float* hidden, int64_t M, int64_t D, const bf16_t* head, int64_t V,
                      float* logits, hipStream_t st) {
   void* hb = nullptr;
-  bdh_status s = scratch(st, SLOT_LAYER_CUR, (size_t)(M * D) * sizeof(bf16_t), &hb);
-  if (s != BDH_OK) return s;
-  hipLaunchKernelGGL(to_bf16_kernel, dim3(cdiv(M * D, 1024)), dim3(256), 0, st, hidden,
-                     (bf16_t*)hb, M * D);
-  BDH_HIP_TRY(hipGetLastError());
+  if (M > SK_MAXM) {
+    const bdh_status s = scratch(st, SLOT_LAYER_CUR, (size_t)(M * D) * sizeof(bf16_t), &hb);
+    if (s != BDH_OK) return s;
+    hipLaunchKernelGGL(to_bf16_kernel, dim3(cdiv(M * D, 1024)), dim3(256), 0, st, hidden,
+                       (bf16_t*)hb, M * D);
+    BDH_HIP_TRY(hipGetLastError());
+  }
   LayerGemmArgs g{};
   g.a = (const bf16_t*)hb;
+  g.af = hidden;
   g.b = head;
   g.zpart = logits;
   g.B = 1; g.H = 1; g.T = M; g.N = 1; g.D = D; g.M = M; g.V = V;
@@ -1351,10 +1346,15 @@ bdh_status run_layer(const LayerArgs& a, hipStream_t st, uint64_t* launches) {
     rho_out = (float*)r;
   }
 
-  hipLaunchKernelGGL(to_bf16_kernel, dim3(cdiv(M * a.D, 1024)), dim3(256), 0, st, a.cur,
-                     (bf16_t*)curb, M * a.D);
-  BDH_HIP_TRY(hipGetLastError());
+  // The layer input in bf16: the GEMMs' operand (few rows take the f32 one)
+  // and the attention's value (the decode step takes the f32 one).
+  if (!decode || M > SK_MAXM) {
+    hipLaunchKernelGGL(to_bf16_kernel, dim3(cdiv(M * a.D, 1024)), dim3(256), 0, st, a.cur,
+                       (bf16_t*)curb, M * a.D);
+    BDH_HIP_TRY(hipGetLastError());
+  }
   LayerGemmArgs g{};
+  g.af = a.cur;
   g.B = a.B; g.H = a.H; g.T = a.T; g.N = a.N; g.D = a.D; g.M = M;
   g.mt = (int)cdiv(M, T256);
   g.ct = (int)(HN / (T256 / 2));
@@ -1386,6 +1386,8 @@ bdh_status run_layer(const LayerArgs& a, hipStream_t st, uint64_t* launches) {
     d.freqs = a.freqs;
     d.pos = (float)a.pos0;
     d.a_out = (float*)attn;
+    // (The step normalises its readout itself where it holds whole rows.)
+    d.an = a.D <= kDecodeNormMaxD ? (bf16_t*)an : nullptr;
     d.idx_out = nullptr;
     d.cnt_out = nullptr;
     d.B = a.B; d.H = a.H; d.Hv = 1; d.N = a.N; d.D = a.D;
@@ -1412,7 +1414,9 @@ bdh_status run_layer(const LayerArgs& a, hipStream_t st, uint64_t* launches) {
     if (s != BDH_OK) return s;
   }
 
-  BDH_HIP_TRY(dispatch_per<LnF>((int)a.D, (const float*)attn, (bf16_t*)an, S * a.T, (int)a.D, st));
+  const bool normed = decode && a.D <= kDecodeNormMaxD;
+  if (!normed)
+    BDH_HIP_TRY(dispatch_per<LnF>((int)a.D, (const float*)attn, (bf16_t*)an, S * a.T, (int)a.D, st));
   g.a = (const bf16_t*)an;
   g.b = a.encv;
   if (ks_yz > 0) {
@@ -1431,7 +1435,8 @@ bdh_status run_layer(const LayerArgs& a, hipStream_t st, uint64_t* launches) {
     BDH_HIP_TRY(launch_gemm<G_Z>(g, st));
   }
   BDH_HIP_TRY(dispatch_per<ResF>((int)a.D, (const float*)zp, a.cur, a.next, M, (int)a.D, ks, st));
-  if (launches) *launches += (ks_yz > 0 ? 5 : 6) + n_attn;
+  if (launches)
+    *launches += (ks_yz > 0 ? 5 : 6) - (normed ? 1 : 0) - (decode && M <= SK_MAXM ? 1 : 0) + n_attn;
   return BDH_OK;
 }
 

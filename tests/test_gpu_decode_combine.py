@@ -1,0 +1,65 @@
+"""A decode step whose streams are split into row ranges: the last range to
+finish sums the partial readouts, in range order (the same bits as the
+finalize launch of a step that also returns its active rows), step after
+step, and in graph replays with other work between them."""
+import numpy as np
+import pytest
+
+from tests.gpu_util import announce, dev, need_gpu
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(torch, B, H, N, D, seed):
+    rng = np.random.default_rng(seed)
+    x = np.maximum(rng.standard_normal((B, H, N)) - 1.645, 0).astype(np.float32)
+    v = (rng.standard_normal((B, 1, D)) / 16).astype(np.float32)
+    rho = (rng.standard_normal((B, H, N, D)) * 0.2).astype(np.float32)
+    return dev(torch, x), dev(torch, v), dev(torch, rho)
+
+
+@pytest.mark.parametrize("B,H,N,D", [
+    (1, 4, 8192, 256),   # 16 ranges
+    (1, 1, 514, 96),     # 2 ranges, the last ragged
+    (3, 4, 2050, 65),    # scalar columns, ranges not a multiple of 8 rows apart from the last
+    (1, 2, 4096, 600),   # three column blocks
+    (32, 4, 1024, 64),   # 2 ranges on 128 streams, the most that are split
+])
+def test_combined_readout_is_the_finalized_one(B, H, N, D):
+    torch = need_gpu()
+    import burn_dragon_amd as bd
+    announce("decode combine", B, H, N, D)
+    x, v, rho = _inputs(torch, B, H, N, D, N)
+    r1, r2 = rho.clone(), rho.clone()
+    for step in range(6):
+        a = bd.decode_step(x, v, r1, position=step).readout
+        b = bd.decode_step(x, v, r2, position=step, want_active=True).readout
+        torch.cuda.synchronize()
+        assert torch.equal(a, b) and torch.equal(r1, r2), step
+
+
+def test_replays_with_other_steps_between_them():
+    torch = need_gpu()
+    import burn_dragon_amd as bd
+    announce("decode combine in a graph")
+    x, v, rho = _inputs(torch, 1, 4, 8192, 256, 3)
+    x2, v2, rho2 = _inputs(torch, 2, 4, 4096, 128, 4)
+    out = torch.empty(1, 4, 256, device="cuda")
+    st = torch.cuda.Stream()
+    with torch.cuda.stream(st):
+        r = rho.clone()
+        # The lists' form warms the stream; the form captured is the other one.
+        bd.decode_step(x, v, r, position=0, want_active=True)
+        r.copy_(rho)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=st):
+            bd.decode_step(x, v, r, position=9, out=out)
+        ref = rho.clone()
+        for i in range(4):
+            graph.replay()
+            bd.decode_step(x2, v2, rho2, position=i)
+            want = bd.decode_step(x, v, ref, position=9).readout
+            torch.cuda.synchronize()
+            assert torch.equal(out, want) and torch.equal(r, ref), i
+        del graph
+    bd.release_stream_scratch(st)
