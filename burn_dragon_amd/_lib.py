@@ -121,6 +121,8 @@ class BdhError(RuntimeError):
 def load() -> ctypes.CDLL:
     """Loads the in-tree library (raises if it has not been built)."""
     global _lib
+    if _lib is not None:
+        return _lib
     with _lock:
         if _lib is None:
             if not os.path.exists(LIB_PATH):

@@ -57,7 +57,7 @@ def try_fused_dense_causal_attention_with_plan(query, value, decay, plan=None
     ctx = torch.empty((B, H, T, D), device=q.device, dtype=torch.float32)
     st = _lib.load().bdh_dense_causal_attention_fwd(
         ctypes.byref(cplan), code, _ptr(q), _ptr(v), _ptr(d), _ptr(ctx),
-        ctypes.c_void_p(_stream_ptr(q.device)))
+        _stream_ptr(q.device))
     return ctx if _lib.check(st) else None
 
 

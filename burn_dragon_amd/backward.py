@@ -84,7 +84,7 @@ def dense_causal_attention_vjp_with_initial_rho(grad_output, query, value, decay
     gr = torch.empty((B, H, N, D), device=dev, dtype=torch.float32) if r is not None else None
     st = _lib.load().bdh_dense_causal_attention_vjp(
         ctypes.byref(plan), _ptr(q), _ptr(v), _ptr(d), _ptr(r), _ptr(g), _ptr(gq), _ptr(gv), _ptr(gd),
-        _ptr(gr), ctypes.c_void_p(_stream_ptr(dev)))
+        _ptr(gr), _stream_ptr(dev))
     if not _lib.check(st):
         return None
     return DenseCausalAttentionVjp(gq, gv, gd, gr)
@@ -113,7 +113,7 @@ def recurrent_attention_vjp(grad_context, query, value, rho=None, decay=None
     gr = torch.empty((B, H, N, D), device=dev, dtype=torch.float32) if r is not None else None
     st = _lib.load().bdh_recurrent_attention_vjp(
         ctypes.byref(plan), _ptr(q), _ptr(v), _ptr(r), _ptr(d), _ptr(g), _ptr(gq), _ptr(gv), _ptr(gr),
-        _ptr(gd), ctypes.c_void_p(_stream_ptr(dev)))
+        _ptr(gd), _stream_ptr(dev))
     if not _lib.check(st):
         return None
     return RecurrentAttentionGrads(gq, gv, gr, gd)

@@ -34,11 +34,14 @@
 namespace bdh {
 namespace {
 
+// Threads of a sparse step's workgroup: 1024, or 512 over ranges of at most
+// DR_SMALL rows (few streams, many ranges: fewer waves to start and to meet).
 constexpr int DR_THREADS = 1024;
-constexpr int DR_WAVES = DR_THREADS / 64;
+constexpr int DR_SMALL_THREADS = 512;
+constexpr int DR_SMALL = 256;
 constexpr int DR_SEG = 8192;       // rows compacted per pass (LDS list capacity)
 constexpr int DR_UNROLL = 8;
-constexpr int DR_MAXG = 16;        // row ranges of a stream
+constexpr int DR_MAXG = 32;        // row ranges of a stream
 constexpr int ROWS_PER_THREAD = 8;  // 4 whole (even, odd) RoPE pairs
 constexpr int DD_THREADS = 256;     // dense step
 constexpr int DD_WAVES = DD_THREADS / 64;
@@ -143,13 +146,14 @@ __device__ __forceinline__ int block_prefix(int cnt, int lane, int wave, int32_t
   return off + incl - cnt;
 }
 
-template <bool ROPE, bool VEC4>
-__global__ __launch_bounds__(DR_THREADS) void decode_kernel(DecodeKernelArgs p) {
-  constexpr int CB = ColBlock<VEC4>::W;
-  __shared__ int32_t lidx[DR_SEG];
-  __shared__ float lval[DR_SEG];
-  __shared__ __attribute__((aligned(16))) float red[DR_WAVES * CB];
-  __shared__ int32_t wtot[DR_WAVES];
+template <bool ROPE, bool VEC4, int THREADS>
+__global__ __launch_bounds__(THREADS) void decode_kernel(DecodeKernelArgs p) {
+  constexpr int CB = ColBlock<VEC4>::W, WAVES = THREADS / 64;
+  constexpr int SEG = THREADS == DR_THREADS ? DR_SEG : DR_SMALL;  // rows listed per pass
+  __shared__ int32_t lidx[SEG];
+  __shared__ float lval[SEG];
+  __shared__ __attribute__((aligned(16))) float red[WAVES * CB];
+  __shared__ int32_t wtot[WAVES];
   __shared__ float whole[kDecodeNormMaxD];  // the readout, for its LayerNorm
   __shared__ uint32_t arrived;
 
@@ -177,14 +181,14 @@ __global__ __launch_bounds__(DR_THREADS) void decode_kernel(DecodeKernelArgs p) 
       else vv.x = vs[c];
     }
 
-    for (int seg0 = r0; seg0 < r1; seg0 += DR_SEG) {
-      const int seg_end = min(r1, seg0 + DR_SEG);
+    for (int seg0 = r0; seg0 < r1; seg0 += SEG) {
+      const int seg_end = min(r1, seg0 + SEG);
       // ---- compaction of rows [seg0, seg_end) ----
       const int base = seg0 + tid * ROWS_PER_THREAD;
       float r[ROWS_PER_THREAD];
       const unsigned m = rows8<ROPE>(xs, p.freqs, p.pos, base, seg_end, aligned && base < seg_end, r);
       int seg_total = 0;
-      int pos = block_prefix<DR_WAVES>(__popc(m), lane, wave, wtot, seg_total);
+      int pos = block_prefix<WAVES>(__popc(m), lane, wave, wtot, seg_total);
 #pragma unroll
       for (int e = 0; e < ROWS_PER_THREAD; ++e)
         if ((m >> e) & 1u) {
@@ -195,18 +199,18 @@ __global__ __launch_bounds__(DR_THREADS) void decode_kernel(DecodeKernelArgs p) 
       __syncthreads();
       if (first) {
         if (idx_s)
-          for (int k = tid; k < seg_total; k += DR_THREADS) idx_s[done + k] = lidx[k];
+          for (int k = tid; k < seg_total; k += THREADS) idx_s[done + k] = lidx[k];
         done += seg_total;
       }
 
       // ---- stream the active rows: a += r rho_row ; rho_row += r v ----
-      for (int k0 = wave; k0 < seg_total; k0 += DR_WAVES * DR_UNROLL) {
+      for (int k0 = wave; k0 < seg_total; k0 += WAVES * DR_UNROLL) {
         float4 row[DR_UNROLL];
         float rv[DR_UNROLL];
         float* ptr[DR_UNROLL];
 #pragma unroll
         for (int u = 0; u < DR_UNROLL; ++u) {
-          const int k = k0 + u * DR_WAVES;
+          const int k = k0 + u * WAVES;
           const bool ok = k < seg_total && cv;
           rv[u] = k < seg_total ? lval[k] : 0.0f;
           ptr[u] = rho_s + (int64_t)(k < seg_total ? lidx[k] : 0) * p.D + c;
@@ -215,7 +219,7 @@ __global__ __launch_bounds__(DR_THREADS) void decode_kernel(DecodeKernelArgs p) 
         }
 #pragma unroll
         for (int u = 0; u < DR_UNROLL; ++u) {
-          const int k = k0 + u * DR_WAVES;
+          const int k = k0 + u * WAVES;
           acc.x = fmaf(row[u].x, rv[u], acc.x);
           float4 nr;
           nr.x = fmaf(rv[u], vv.x, row[u].x);
@@ -241,10 +245,10 @@ __global__ __launch_bounds__(DR_THREADS) void decode_kernel(DecodeKernelArgs p) 
     if (VEC4) *reinterpret_cast<float4*>(&red[wave * CB + lane * 4]) = acc;
     else red[wave * CB + lane] = acc.x;
     __syncthreads();
-    for (int cc = tid; cc < CB; cc += DR_THREADS) {
+    for (int cc = tid; cc < CB; cc += THREADS) {
       float sum = red[cc];
 #pragma unroll
-      for (int w = 1; w < DR_WAVES; ++w) sum += red[w * CB + cc];
+      for (int w = 1; w < WAVES; ++w) sum += red[w * CB + cc];
       if (cb + cc >= p.D) continue;
       if (p.ctr) __hip_atomic_store(a_s + cb + cc, sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       else if (p.an && p.G == 1) whole[cb + cc] = sum;
@@ -271,7 +275,7 @@ __global__ __launch_bounds__(DR_THREADS) void decode_kernel(DecodeKernelArgs p) 
     __syncthreads();
     if (arrived != (uint32_t)p.G - 1) return;
     const float* part = p.a_out + s * p.G * p.D;
-    for (int d = tid; d < p.D; d += DR_THREADS) {
+    for (int d = tid; d < p.D; d += THREADS) {
       float v[DR_MAXG];
 #pragma unroll
       for (int k = 0; k < DR_MAXG; ++k)
@@ -304,7 +308,7 @@ __global__ __launch_bounds__(DR_THREADS) void decode_kernel(DecodeKernelArgs p) 
     }
   }
   if (p.G == 1 && idx_s)
-    for (int k = done + tid; k < p.N; k += DR_THREADS) idx_s[k] = -1;
+    for (int k = done + tid; k < p.N; k += THREADS) idx_s[k] = -1;
   if (p.cnt_out && tid == 0) p.cnt_out[s * p.G + g] = done;
 }
 
@@ -448,11 +452,16 @@ bool sparse_step(const DecodeArgs& a) { return a.decay == nullptr && a.rho_in !=
 void decode_ranges(const DecodeArgs& a, int* G, int* rows) {
   if (sparse_step(a)) {
     // Double while the grid stays within one workgroup per CU and a range
-    // keeps at least 256 rows.  (Measured: with a stream per CU already,
-    // splitting further costs more in partials than it gains.)
+    // keeps at least 256 rows, up to 16 ranges; at ordinary sizes on to 32
+    // ranges of 128 rows (B1 nh4 N8192 D256: 16 ranges of 512 rows in 1024
+    // threads xx us, 32 of 256 in 512 threads xx).  (Measured: with a stream
+    // per CU already, splitting further costs more in partials than it gains.)
     int g = 1;
     const int64_t S = a.B * a.H;
-    while (g < DR_MAXG && S * 2 * g <= (int64_t)device_cus() && a.N / (2 * g) >= 256) g *= 2;
+    const bool ordinary = a.N <= 65536 && a.D <= 2048;
+    while (S * 2 * g <= (int64_t)device_cus() &&
+           (ordinary ? g < DR_MAXG && a.N / (2 * g) >= 128 : g < 16 && a.N / (2 * g) >= 256))
+      g *= 2;
     *G = g;
     *rows = (int)(((a.N + g - 1) / g + 7) / 8 * 8);
   } else {
@@ -540,14 +549,19 @@ bdh_status run_decode(const DecodeArgs& a, hipStream_t st, uint64_t* launches) {
   const bool rope = a.freqs != nullptr;
   const int kt = ktime_begin(BDH_KERNEL_DECODE, st);
   if (sparse) {
-    const dim3 grid((unsigned)(S * G)), blk(DR_THREADS);
-    if (rope) {
-      if (vec4) hipLaunchKernelGGL((decode_kernel<true, true>), grid, blk, 0, st, p);
-      else hipLaunchKernelGGL((decode_kernel<true, false>), grid, blk, 0, st, p);
-    } else {
-      if (vec4) hipLaunchKernelGGL((decode_kernel<false, true>), grid, blk, 0, st, p);
-      else hipLaunchKernelGGL((decode_kernel<false, false>), grid, blk, 0, st, p);
-    }
+    const dim3 grid((unsigned)(S * G));
+    auto launch = [&](auto threads) {
+      constexpr int TH = decltype(threads)::value;
+      if (rope) {
+        if (vec4) hipLaunchKernelGGL((decode_kernel<true, true, TH>), grid, dim3(TH), 0, st, p);
+        else hipLaunchKernelGGL((decode_kernel<true, false, TH>), grid, dim3(TH), 0, st, p);
+      } else {
+        if (vec4) hipLaunchKernelGGL((decode_kernel<false, true, TH>), grid, dim3(TH), 0, st, p);
+        else hipLaunchKernelGGL((decode_kernel<false, false, TH>), grid, dim3(TH), 0, st, p);
+      }
+    };
+    if (rows <= DR_SMALL) launch(std::integral_constant<int, DR_SMALL_THREADS>{});
+    else launch(std::integral_constant<int, DR_THREADS>{});
   } else {
     const dim3 grid((unsigned)(S * G)), blk(DD_THREADS);
     const int key = (rope ? 8 : 0) | (vec4 ? 4 : 0) | (a.decay ? 2 : 0) | (a.rho_in ? 1 : 0);

@@ -65,7 +65,7 @@ def decode_step(x: torch.Tensor, value: torch.Tensor, rho: torch.Tensor, *,
     st = _lib.load().bdh_decode_step(
         B, H, Hv, N, D, _ptr(xc), _ptr(vc), _ptr(rho), _ptr(decay),
         ctypes.byref(rope) if rope else None,
-        _ptr(a), _ptr(idx), _ptr(cnt), ctypes.c_void_p(_stream_ptr(x.device)))
+        _ptr(a), _ptr(idx), _ptr(cnt), _stream_ptr(x.device))
     if not _lib.check(st):
         return None
     return DecodeOutput(a, idx, cnt)

@@ -58,7 +58,7 @@ class LowRankWeights(NamedTuple):
         enc_c, encv_c, dec_c = enc.contiguous(), encv.contiguous(), decoder.contiguous()
         st = _lib.load().bdh_lowrank_pack_weights(
             H, N, D, _ptr(enc_c), _ptr(encv_c), _ptr(dec_c), _ptr(ep), _ptr(evp), _ptr(dp),
-            ctypes.c_void_p(_stream_ptr(dev)))
+            _stream_ptr(dev))
         if not _lib.check(st):
             return None
         return LowRankWeights(ep, evp, dp, H, N, D)
@@ -126,7 +126,7 @@ def lowrank_layer_forward(current: torch.Tensor, weights: LowRankWeights, *,
     st = _lib.load().bdh_lowrank_layer_fwd_ex(
         ctypes.byref(plan), _ptr(cur), _ptr(weights.encoder), _ptr(weights.encoder_v),
         _ptr(weights.decoder), ctypes.byref(rope) if rope else None, _ptr(rho_in), _ptr(nxt),
-        _ptr(rho_out), ctypes.byref(opts), ctypes.c_void_p(_stream_ptr(cur.device)))
+        _ptr(rho_out), ctypes.byref(opts), _stream_ptr(cur.device))
     if not _lib.check(st):
         return None
     return LowRankLayerOutput(nxt, rho_out)

@@ -67,7 +67,7 @@ def pack_model(embed: torch.Tensor, encoder: torch.Tensor, encoder_v: torch.Tens
     head_c = lm_head.contiguous()
     packed = torch.empty((Vh, D), device=embed.device, dtype=torch.bfloat16)
     st = _lib.load().bdh_lm_head_pack(D, Vh, _ptr(head_c), _ptr(packed),
-                                      ctypes.c_void_p(_stream_ptr(embed.device)))
+                                      _stream_ptr(embed.device))
     if not _lib.check(st):
         return None
     return BdhModelWeights(embed.contiguous(), layer, packed, Vh, int(n_layer))
@@ -99,7 +99,7 @@ def model_forward_logits(tokens: torch.Tensor, weights: BdhModelWeights, *,
     B, T = tokens.shape
     D = weights.layer.embd
     dev = tokens.device
-    stream = ctypes.c_void_p(_stream_ptr(dev))
+    stream = _stream_ptr(dev)
     lib = _lib.load()
     tok = tokens.contiguous()
     cur = torch.empty((B, T, D), device=dev, dtype=torch.float32)
@@ -145,7 +145,7 @@ def save_model_state(path: str, state: BdhModelState, persist_sequence_state: bo
             dev = r.device
         descs[i].persist_sequence_state = int(persist_sequence_state)
         descs[i].retain_terminal_sequence_state = int(retain_terminal_sequence_state)
-    stream = ctypes.c_void_p(_stream_ptr(dev)) if dev is not None else None
+    stream = _stream_ptr(dev) if dev is not None else None
     st = _lib.load().bdh_state_record_save(str(path).encode(), int(state.position), n, descs, ptrs,
                                            stream)
     if st != _lib.BDH_OK:
@@ -178,7 +178,7 @@ def load_model_state(path: str, device: torch.device) -> BdhModelState:
         ptrs[i] = r.data_ptr()
         state.rho.append(r)
     st = lib.bdh_state_record_load(str(path).encode(), n.value, descs, ptrs,
-                                   ctypes.c_void_p(_stream_ptr(device)))
+                                   _stream_ptr(device))
     if st != _lib.BDH_OK:
         raise _lib.BdhError(f"bdh_state_record_load: {_lib.last_error()}")
     return state

@@ -89,7 +89,9 @@ def _dtype_code(t: torch.Tensor) -> Optional[int]:
 
 
 def _stream_ptr(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The current stream's handle, without building a Stream object."""
+    index = device.index if device.index is not None else torch.cuda.current_device()
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 def _on_device(*ts) -> bool:
@@ -135,7 +137,8 @@ def _prepare(query, value, rho, decay, plan):
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+    """A tensor's address (the signatures' pointer arguments take integers)."""
+    return t.data_ptr() if t is not None else None
 
 
 def try_fused_recurrent_attention_with_plan(query, value, rho=None, decay=None, plan=None,
@@ -159,7 +162,7 @@ def try_fused_recurrent_attention_with_plan(query, value, rho=None, decay=None, 
         rho_out = torch.empty((B, H, N, D), device=q.device, dtype=torch.float32)
     st = _lib.load().bdh_recurrent_attention_fwd(
         ctypes.byref(cplan), code, _ptr(q), _ptr(v), _ptr(r), _ptr(d), _ptr(ctx), _ptr(rho_out),
-        chunk, ctypes.c_void_p(_stream_ptr(q.device)))
+        chunk, _stream_ptr(q.device))
     if not _lib.check(st):
         return None
     return RecurrentAttentionOutput(ctx, rho_out)
@@ -200,7 +203,7 @@ def try_fused_recurrent_attention_rope(x, value, rho=None, decay=None, *, positi
         rho_out = torch.empty((B, H, N, D), device=q.device, dtype=torch.float32)
     st = _lib.load().bdh_recurrent_attention_rope_fwd(
         ctypes.byref(cplan), code, _ptr(q), _ptr(v), _ptr(r), _ptr(d), ctypes.byref(rope),
-        _ptr(ctx), _ptr(rho_out), chunk, ctypes.c_void_p(_stream_ptr(q.device)))
+        _ptr(ctx), _ptr(rho_out), chunk, _stream_ptr(q.device))
     if not _lib.check(st):
         return None
     return RecurrentAttentionOutput(ctx, rho_out)
