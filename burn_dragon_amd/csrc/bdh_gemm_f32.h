@@ -555,31 +555,63 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
     }
     return;
   }
-  const bool whole = m0 + BT <= M && n0 + BT <= N;
+  // Out through LDS (free once every wave has read its last fragments), 32
+  // rows of the wave's block at a time in a region of its own, so that a lane
+  // stores 16 bytes and a wave whole 256-byte pieces of rows (from the
+  // accumulators' layout, 4 bytes a lane in 128-byte pieces, the 268 MB state
+  // of the f32 C2 shape left at 1.6 TB/s).
+  constexpr int EP = 32 * NB + 4, LPR = 8 * NB, RPI = 64 / LPR;  // row pitch; lanes a row; rows an access
+  float* eb = reinterpret_cast<float*>(lds + 1024) + w * 32 * EP;  // past the power table
+  static_assert(1024 + 4 * 32 * EP * 4 <= 2 * STAGE && 2 * BT * 4 <= 1024, "the epilogue's LDS");
+  __syncthreads();
+  const int er = lane / LPR, n = nw + (lane % LPR) * 4;
+  const bool quad = g.sCn == 1 && n + 4 <= N;
 #pragma unroll
-  for (int i = 0; i < NB; ++i)
+  for (int i = 0; i < NB; ++i) {
 #pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      const int n = nw + 32 * j + acc_col(lane);
-      float x[16];
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) eb[acc_row(lane, r) * EP + 32 * j + acc_col(lane)] = big[i][j][r];
+    floatx4 v[32 / RPI], x[32 / RPI];
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wave's lanes have written
+#pragma unroll
+    for (int q = 0; q < 32 / RPI; ++q) {
+      const int m = mw + 32 * i + q * RPI + er;
+      v[q] = *reinterpret_cast<const floatx4*>(&eb[(q * RPI + er) * EP + (lane % LPR) * 4]);
+      x[q] = zero4();
       // A block's addends are all loaded before its first store.
-      if (X != nullptr) {
+      if (X == nullptr || m >= M || n >= N) continue;
+      const float* xp = X + (int64_t)m * g.sCm + (int64_t)n * g.sCn;
+      if (quad) {
+        x[q] = *reinterpret_cast<const floatx4u*>(xp);
+      } else {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int m = mw + 32 * i + acc_row(lane, r);
-          x[r] = whole || (m < M && n < N) ? X[(int64_t)m * g.sCm + (int64_t)n * g.sCn] : 0.0f;
-        }
-      }
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int m = mw + 32 * i + acc_row(lane, r);
-        if (!whole && (m >= M || n >= N)) continue;
-        if (P > 1) Pp[(int64_t)m * g.N + n] = big[i][j][r];
-        else
-          C[(int64_t)m * g.sCm + (int64_t)n * g.sCn] =
-              epi_value<EPI>(g, power, carry, m, n, big[i][j][r], X != nullptr ? x[r] : 0.0f);
+        for (int e = 0; e < 4; ++e)
+          if (n + e < N) x[q][e] = xp[e * g.sCn];
       }
     }
+#pragma unroll
+    for (int q = 0; q < 32 / RPI; ++q) {
+      const int m = mw + 32 * i + q * RPI + er;
+      if (m >= M || n >= N) continue;
+      float* o = P > 1 ? Pp + (int64_t)m * g.N + n : C + (int64_t)m * g.sCm + (int64_t)n * g.sCn;
+      floatx4u y;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        y[e] = P > 1 ? v[q][e] : epi_value<EPI>(g, power, carry, m, n + e, v[q][e], x[q][e]);
+      if (P > 1 ? n + 4 <= N : quad) {
+        if (EPI == E_CARRY || EPI == E_CARRY_SNAP || EPI == E_STORE)
+          __builtin_nontemporal_store(y, reinterpret_cast<floatx4u*>(o));
+        else
+          *reinterpret_cast<floatx4u*>(o) = y;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n + e < N) o[P > 1 ? e : e * g.sCn] = y[e];
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read before the next 32 rows are written
+  }
 }
 
 // Split-K: sums the P partials of each (b, m, n) in range order and applies
