@@ -683,24 +683,10 @@ bdh_status run_bf16_path(const Bf16Args& a, hipStream_t st, uint64_t* launches) 
     if (r != BDH_UNSUPPORTED) return r;
   }
 
-  // N splits of the gram: the fewest for which the longest gram unit stays
-  // within ~85% of the first launch's average work per workgroup slot (two
-  // per CU; every split writes, and the context kernel re-reads, one more
-  // partial score buffer).  Work is counted in 32-deep steps of one 256x128
-  // tile; a state unit costs its token steps plus ~4 for its rho write.
-  const double gram_work = (double)S * n_iv * nb * (nb + 1) * nk;
-  const double state_work = a.state ? state_units * (((Lc0 + 63) / 64) * 2 + 4.0) : 0.0;
-  const double per_slot = (gram_work + state_work) / (2.0 * device_cus());
-  // Every N range must be an even number of steps (nk is a multiple of 8, so
-  // ks = 1, 2 and 4 always qualify).
-  int ks = 1;
-  for (int cand = 1; cand <= 8 && nk % (2 * cand) == 0; cand *= 2) {
-    ks = cand;
-    if ((double)nk / cand <= 0.85 * per_slot) break;
-  }
-
   // Readout splits: the fewest for which one readout unit stays within the
   // average work per workgroup slot of its launch (readout + state units).
+  // Work is counted in 32-deep steps of one 256x128 tile; a state unit costs
+  // its token steps plus ~4 for its rho write.
   const bool carried = a.rho_in != nullptr || n_iv > 1;
   int rd_kr = 1;
   if (carried) {
@@ -711,6 +697,25 @@ bdh_status run_bf16_path(const Bf16Args& a, hipStream_t st, uint64_t* launches) 
       rd_kr = cand;
       if ((double)nk / cand <= 1.25 * slot) break;
     }
+  }
+
+  // N splits of the gram: the fewest for which the longest gram unit stays
+  // within 1.2 times the first launch's average work per workgroup slot (two
+  // per CU), every unit's prologue and epilogue counted as 8 more steps; each
+  // split writes, and the context kernel re-reads, one more partial score
+  // buffer.  (Without the readout units and the units' own cost in the sum, at
+  // 0.85: B2 nh4 T333 N8192 onto a state 8 splits, 143 us, 4: 132 us; B8 T60
+  // N2048 8 splits, 62 us, 2: 52 us.)
+  constexpr double kUnit = 8.0;
+  const double rd_work = carried ? prefill_readout_units(S, Lc0, a.D, rd_kr) * ((double)nk / rd_kr + kUnit) : 0.0;
+  const double state_work = a.state ? state_units * (((Lc0 + 63) / 64) * 2 + kUnit) : 0.0;
+  // Every N range must be an even number of steps (nk is a multiple of 8, so
+  // ks = 1, 2 and 4 always qualify).
+  int ks = 1;
+  for (int cand = 1; cand <= 8 && nk % (2 * cand) == 0; cand *= 2) {
+    ks = cand;
+    const double gram_work = (double)S * n_iv * cand * (nb * nb + (nb + 1) / 2) * ((double)nk / cand + kUnit);
+    if ((double)nk / cand <= 1.2 * (gram_work + state_work + rd_work) / (2.0 * device_cus())) break;
   }
 
   void *vt = nullptr, *part = nullptr, *rdp = nullptr, *rho_a = nullptr, *rho_b = nullptr;
