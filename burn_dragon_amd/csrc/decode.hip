@@ -1,15 +1,16 @@
 // One-token (T = 1) steps of the recurrence on gfx950 (fp32), one launch per
-// token (plus a finalize launch when streams are split into row ranges):
+// token (plus, in the cases named below, a finalize launch when streams are
+// split into row ranges):
 //   A = active rows of rot(x)   (x_i != 0, or x_{i^1} != 0 and frac(p f_i) != 0)
 //   a = rot(x)[A] . rho[A, :]   (read before the update)
 //   rho' = (rho + rot(x)^T v) * d
 //
 // Sparse step (rho updated in place, no decay): only the rows in A change,
-// so only they are read and written.  G 1024-thread workgroups per (batch,
-// head) stream each own a range of N / G rows (G grows while the grid stays
-// within one workgroup per CU).  A workgroup compacts its range's active rows
+// so only they are read and written.  G workgroups per (batch, head) stream
+// (1024 threads, 512 for ranges of up to 256 rows) each own a range of N / G
+// rows (G grows while the grid stays within one workgroup per CU).  A workgroup compacts its range's active rows
 // (8 rows per thread, wavefront prefix scan, workgroup offsets through LDS)
-// into an LDS list (ascending), then its 16 waves stream exactly those rho
+// into an LDS list (ascending), then its waves stream exactly those rho
 // rows: a whole 1 KiB row per wave per load at D = 256 (float4 per lane), 8
 // rows in flight per wave.
 //
@@ -26,7 +27,8 @@
 // the active lists are asked for, the step is dense, or the buffers are a
 // caller's (which overlapping calls may share), a finalize kernel sums the
 // partials (and concatenates the lists) instead.  At C3's shape with B = 1
-// (4 streams of 16 ranges) the finalize launch was 4.4 of 14.3 us.
+// (4 streams of 32 ranges) a kernel of 8.1 us and a finalize launch of 4.4 are
+// one of 11.2.
 #include <type_traits>
 
 #include "bdh_internal.h"
@@ -454,12 +456,14 @@ void decode_ranges(const DecodeArgs& a, int* G, int* rows) {
     // Double while the grid stays within one workgroup per CU and a range
     // keeps at least 256 rows, up to 16 ranges; at ordinary sizes on to 32
     // ranges of 128 rows (B1 nh4 N8192 D256: 16 ranges of 512 rows in 1024
-    // threads xx us, 32 of 256 in 512 threads xx).  (Measured: with a stream
+    // threads 11.6 us, 32 of 256 in 512 threads 11.2).  (Measured: with a stream
     // per CU already, splitting further costs more in partials than it gains.)
     int g = 1;
     const int64_t S = a.B * a.H;
     const bool ordinary = a.N <= 65536 && a.D <= 2048;
-    while (S * 2 * g <= (int64_t)device_cus() &&
+    // (Streams of fewer than 512 rows stay whole: they need no scratch, so
+    // they can be captured before an eager call.)
+    while (S * 2 * g <= (int64_t)device_cus() && a.N >= 512 &&
            (ordinary ? g < DR_MAXG && a.N / (2 * g) >= 128 : g < 16 && a.N / (2 * g) >= 256))
       g *= 2;
     *G = g;

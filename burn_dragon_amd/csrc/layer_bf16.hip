@@ -327,7 +327,7 @@ __host__ __device__ inline int tiles_of(int64_t T) { return (int)((T + XR_T - 1)
 // The wave-role GEMM X and the fused Y + Z launch fetch, multiply and do not
 // store a sequence's last tile's missing rows, which the 256-row tiles of the
 // separate GEMMs pack away; they still win while at least half of their rows
-// are tokens (B2 T777 N8192 D256: X 76 -> 60 us, Y and Z 147 -> 110).
+// are tokens (B2 T777 N8192 D256: X 76 -> 60 us, Y and Z 147 -> 110 us).
 bool tiles_filled(int64_t T) { return (int64_t)tiles_of(T) * XR_T <= 2 * T; }
 // Rows past a buffer's last that those tiles may fetch.
 constexpr int64_t kTilePad = XR_T;

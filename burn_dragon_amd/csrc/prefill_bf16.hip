@@ -437,7 +437,7 @@ int snap_ranges(int64_t units, int nk, double mb, bool even) {
   return best;
 }
 
-// Two or more intervals, no decay: v^T, the state-carry kernel (which also
+// Two or more intervals, or one onto a large carried state: v^T, the state-carry kernel (which also
 // rotates x once and writes q), one launch of every interval's gram tiles
 // and readouts (from the bf16 snapshots), then the context kernel, which
 // adds the readout partials.  Four launches whatever the interval count.
@@ -667,11 +667,15 @@ bdh_status run_bf16_path(const Bf16Args& a, hipStream_t st, uint64_t* launches) 
   const int state_units = prefill_state_units(S, a.N, a.D);
   // (The readout units address a snapshot's rows with 32-bit offsets.)
   // One interval with a carried state takes the state-carry form (which reads
-  // rho once, for its snapshot and its successor) from 24 M elements of x on:
-  // B8 nh4 T300 N8192 D256 422 against 365 us, T512 498 against 457, B8 T400
-  // N2048 in place 235 against 224; below, its launches cost more (B1 T512
-  // N8192 104 against 121 us, B4 T256 N4096 95 against 112).
-  const bool carried1 = a.rho_in != nullptr && S * a.T * a.N >= ((int64_t)24 << 20);
+  // rho once, for its snapshot and its successor) where its gram has more than
+  // one block of 256 tokens, its columns fill the carry kernel's 256-column
+  // block and x has 48 M elements: B8 nh4 T300 N8192 D256 418 -> 380 us, T512
+  // 494 -> 467, B24 T512 N2048 438 -> 374, B3 T512 N8192 205 -> 201.  Elsewhere
+  // its extra launches and the q stream cost more: B8 T400 N2048 (25 M) 138
+  // against 144 us, B8 T256 N8192 310 against 334, B16 T512 N4096 D64 378
+  // against 396, B16 T400 N4096 D128 with decay 330 against 392.
+  const bool carried1 =
+      a.rho_in != nullptr && a.T > T256 && a.D > T256 / 2 && S * a.T * a.N >= ((int64_t)48 << 20);
   if (a.state && (n_iv >= 2 || carried1) && a.D * a.N * 2 < ((int64_t)1 << 31) &&
       (size_t)(n_iv * S * a.N * a.D) * sizeof(bf16_t) <= kCarrySnapMax)
     return run_carry_path(a, st, launches, S, Tp, Dp, n_iv, Lp, nb, nk);
@@ -700,12 +704,15 @@ bdh_status run_bf16_path(const Bf16Args& a, hipStream_t st, uint64_t* launches) 
   }
 
   // N splits of the gram: the fewest for which the longest gram unit stays
-  // within 1.2 times the first launch's average work per workgroup slot (two
-  // per CU), every unit's prologue and epilogue counted as 8 more steps; each
+  // within 1.2 times (unsplit: 0.95) the first launch's average work per
+  // workgroup slot (two per CU), every unit's prologue and epilogue counted as
+  // 8 more steps; each
   // split writes, and the context kernel re-reads, one more partial score
   // buffer.  (Without the readout units and the units' own cost in the sum, at
   // 0.85: B2 nh4 T333 N8192 onto a state 8 splits, 143 us, 4: 132 us; B8 T60
-  // N2048 8 splits, 62 us, 2: 52 us.)
+  // N2048 8 splits, 62 us, 2: 52 us.  With 0.95 throughout, B8 nh4 T256 N8192
+  // onto a state is 332 against 310 us; with 1.2 throughout, a layer of B16 T256
+  // N8192 989 against 968.)
   constexpr double kUnit = 8.0;
   const double rd_work = carried ? prefill_readout_units(S, Lc0, a.D, rd_kr) * ((double)nk / rd_kr + kUnit) : 0.0;
   const double state_work = a.state ? state_units * (((Lc0 + 63) / 64) * 2 + kUnit) : 0.0;
@@ -715,7 +722,8 @@ bdh_status run_bf16_path(const Bf16Args& a, hipStream_t st, uint64_t* launches) 
   for (int cand = 1; cand <= 8 && nk % (2 * cand) == 0; cand *= 2) {
     ks = cand;
     const double gram_work = (double)S * n_iv * cand * (nb * nb + (nb + 1) / 2) * ((double)nk / cand + kUnit);
-    if ((double)nk / cand <= 1.2 * (gram_work + state_work + rd_work) / (2.0 * device_cus())) break;
+    const double slot_work = (gram_work + state_work + rd_work) / (2.0 * device_cus());
+    if ((double)nk / cand <= (cand == 1 ? 0.95 : 1.2) * slot_work) break;
   }
 
   void *vt = nullptr, *part = nullptr, *rdp = nullptr, *rho_a = nullptr, *rho_b = nullptr;

@@ -19,8 +19,8 @@ def _inputs(torch, B, H, N, D, seed):
 
 
 @pytest.mark.parametrize("B,H,N,D", [
-    (1, 4, 8192, 256),   # 16 ranges
-    (1, 1, 514, 96),     # 2 ranges, the last ragged
+    (1, 4, 8192, 256),   # 32 ranges
+    (1, 1, 514, 96),     # 4 ranges, the last ragged
     (3, 4, 2050, 65),    # scalar columns, ranges not a multiple of 8 rows apart from the last
     (1, 2, 4096, 600),   # three column blocks
     (32, 4, 1024, 64),   # 2 ranges on 128 streams, the most that are split
@@ -59,6 +59,31 @@ def test_replays_with_other_steps_between_them():
             graph.replay()
             bd.decode_step(x2, v2, rho2, position=i)
             want = bd.decode_step(x, v, ref, position=9).readout
+            torch.cuda.synchronize()
+            assert torch.equal(out, want) and torch.equal(r, ref), i
+        del graph
+    bd.release_stream_scratch(st)
+
+
+def test_short_streams_are_captured_without_an_eager_call():
+    # Fewer than 512 rows: the step takes no scratch, so a stream's first call may be a captured one.
+    torch = need_gpu()
+    import burn_dragon_amd as bd
+    announce("decode of short streams captured cold")
+    x, v, rho = _inputs(torch, 2, 4, 510, 64, 5)
+    ref = rho.clone()
+    want = bd.decode_step(x, v, ref, position=9).readout  # frequency table resident
+    out = torch.empty(2, 4, 64, device="cuda")
+    torch.cuda.synchronize()
+    st = torch.cuda.Stream()
+    with torch.cuda.stream(st):
+        r = rho.clone()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=st):
+            bd.decode_step(x, v, r, position=9, out=out)
+        for i in range(3):
+            r.copy_(rho)
+            graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(out, want) and torch.equal(r, ref), i
         del graph
