@@ -46,7 +46,7 @@ struct LayerGemmArgs {
   bf16_t* xy;         // X: x out; Y: x in, y out (same place); [B, H, T, N]
   bf16_t* q;          // X: rope(x) out [B, H, T, N], or null (no rotation)
   float* xf;          // X: x out in f32 [B, H, T, N], or null
-  const float* af;    // few rows, X and L: the rows of a in f32 (a unused)
+  const float* af;    // few rows, L and the decode step's X: the rows of a in f32 (a unused), else null
   const float* freqs; // X: RoPE frequencies [N] (with q)
   int64_t pos0;       // X: position of token 0
   int fixed;          // X: every token at pos0
@@ -847,16 +847,18 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void layer_yz_kernel(LayerGemmArgs
 constexpr int SK_MAXM = 64;
 constexpr int SK_CHUNK = 8;  // 32-deep steps loaded at once per wave
 
-template <int KIND, int MB>  // MB = 16-row blocks: 1, 2 or 4
+// MB = 16-row blocks: 1, 2 or 4.  F32 (X, logits): the rows are f32 and
+// rounded here, as to_bf16_kernel does, where that would be a launch for this
+// product alone (the decode step and the logits); its loads are half as many
+// steps deep, so X of a B1 T47 prompt, whose attention needs the bf16 rows
+// anyway, takes 12.2 us from those and 14.4 from the f32 ones.
+template <int KIND, int MB, bool F32>
 __global__ __launch_bounds__(256) void skinny_gemm_kernel(LayerGemmArgs g) {
   // X, Y (K = D, H N columns): each wave owns a 16-column block and all of
   // K.  Z (K = H N) and the logits (few columns): the workgroup owns one
   // column block and a K range, which its 4 waves split and sum through LDS
   // in wave order.  (X, Y: 13 and 15 -> 11 us at C5 decode.)
   constexpr bool WAVECOL = KIND == G_X || KIND == G_Y;
-  // X and the logits take their rows in f32 and round them here (as
-  // to_bf16_kernel does, which was a launch of its own).
-  constexpr bool F32 = KIND == G_X || KIND == G_L;
   constexpr int CH = F32 ? SK_CHUNK / MB : SK_CHUNK;  // steps loaded at once
   __shared__ floatx4 red[WAVECOL ? 1 : 4][MB][64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -884,6 +886,7 @@ __global__ __launch_bounds__(256) void skinny_gemm_kernel(LayerGemmArgs g) {
     m = m < g.M ? m : g.M - 1;
     const int64_t bb = m / g.T, t = m - bb * g.T;
     if constexpr (F32) arow[mb] = g.af + m * g.D + kl;
+    else if (KIND == G_X) arow[mb] = g.a + m * g.D + kl;
     else if (KIND == G_Y) arow[mb] = g.a + ((bb * g.H + h) * g.T + t) * g.D + kl;
     else arow[mb] = g.a + (bb * g.H * g.T + t) * g.N + kl;
   }
@@ -1098,21 +1101,26 @@ __global__ __launch_bounds__(256) void transpose_bf16_kernel(const float* __rest
 inline unsigned cdiv(int64_t a, int64_t b) { return (unsigned)((a + b - 1) / b); }
 
 // Few-row GEMM launch: one workgroup per (16-column block, K split).
-template <int KIND>
+template <int KIND, bool F32>
 hipError_t launch_skinny(const LayerGemmArgs& g, hipStream_t st) {
   const int64_t ncols = KIND == G_Z ? g.D : KIND == G_L ? g.V : g.H * g.N;
   const int64_t blocks = (KIND == G_X || KIND == G_Y) ? cdiv(cdiv(ncols, 16), 4)
                                                       : cdiv(ncols, 16) * (int64_t)(KIND == G_Z ? g.ks : 1);
   const dim3 grid((unsigned)blocks);
-  if (g.M <= 16) hipLaunchKernelGGL((skinny_gemm_kernel<KIND, 1>), grid, dim3(256), 0, st, g);
-  else if (g.M <= 32) hipLaunchKernelGGL((skinny_gemm_kernel<KIND, 2>), grid, dim3(256), 0, st, g);
-  else hipLaunchKernelGGL((skinny_gemm_kernel<KIND, 4>), grid, dim3(256), 0, st, g);
+  if (g.M <= 16) hipLaunchKernelGGL((skinny_gemm_kernel<KIND, 1, F32>), grid, dim3(256), 0, st, g);
+  else if (g.M <= 32) hipLaunchKernelGGL((skinny_gemm_kernel<KIND, 2, F32>), grid, dim3(256), 0, st, g);
+  else hipLaunchKernelGGL((skinny_gemm_kernel<KIND, 4, F32>), grid, dim3(256), 0, st, g);
   return hipGetLastError();
 }
 
 template <int KIND>
 hipError_t launch_gemm(const LayerGemmArgs& g, hipStream_t st) {
-  if (g.M <= SK_MAXM) return launch_skinny<KIND>(g, st);
+  if (g.M <= SK_MAXM) {
+    if constexpr (KIND == G_L) return launch_skinny<KIND, true>(g, st);
+    if constexpr (KIND == G_X)
+      if (g.af) return launch_skinny<KIND, true>(g, st);
+    return launch_skinny<KIND, false>(g, st);
+  }
   const int64_t total = (int64_t)g.mt * g.ct * (KIND == G_Z ? g.ks : 1);
   const int64_t slots = 2 * (int64_t)device_cus();  // two workgroups per CU
   const unsigned grid = (unsigned)(total < slots ? total : slots);
@@ -1346,15 +1354,15 @@ bdh_status run_layer(const LayerArgs& a, hipStream_t st, uint64_t* launches) {
     rho_out = (float*)r;
   }
 
-  // The layer input in bf16: the GEMMs' operand (few rows take the f32 one)
-  // and the attention's value (the decode step takes the f32 one).
+  // The layer input in bf16: the GEMMs' operand (few rows of a decode step
+  // take the f32 one) and the attention's value (the decode step takes the f32 one).
   if (!decode || M > SK_MAXM) {
     hipLaunchKernelGGL(to_bf16_kernel, dim3(cdiv(M * a.D, 1024)), dim3(256), 0, st, a.cur,
                        (bf16_t*)curb, M * a.D);
     BDH_HIP_TRY(hipGetLastError());
   }
   LayerGemmArgs g{};
-  g.af = a.cur;
+  g.af = decode ? a.cur : nullptr;
   g.B = a.B; g.H = a.H; g.T = a.T; g.N = a.N; g.D = a.D; g.M = M;
   g.mt = (int)cdiv(M, T256);
   g.ct = (int)(HN / (T256 / 2));
