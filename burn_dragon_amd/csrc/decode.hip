@@ -24,7 +24,7 @@
 // Readouts are reduced across waves in LDS in a fixed order; with G > 1 the
 // range partials go to a range buffer, and the last of a stream's workgroups
 // to finish sums them in range order, so the result is deterministic.  Where
-// the active lists are asked for, the step is dense, or the buffers are a
+// streams have at most 4 ranges (and no LayerNorm follows), the active lists are asked for, the step is dense, or the buffers are a
 // caller's (which overlapping calls may share), a finalize kernel sums the
 // partials (and concatenates the lists) instead.  At C3's shape with B = 1
 // (4 streams of 32 ranges) a kernel of 8.1 us and a finalize launch of 4.4 are
@@ -545,7 +545,10 @@ bdh_status run_decode(const DecodeArgs& a, hipStream_t st, uint64_t* launches) {
       void* c = nullptr;
       const bdh_status s = scratch(st, SLOT_DECODE_CTR, (size_t)device_cus() * sizeof(uint32_t), &c, true);
       if (s != BDH_OK) return s;
-      if (sparse && !a.idx_out && !a.cnt_out) p.ctr = (uint32_t*)c;
+      // Streams of 2 or 4 ranges keep the finalize launch outside the layer:
+      // with that many streams the next step's start hides it (B18 N8192 33.0
+      // against 33.9 us, B24 N4096 D128 16.3 against 17.5).
+      if (sparse && !a.idx_out && !a.cnt_out && (G > 4 || a.an)) p.ctr = (uint32_t*)c;
     }
   }
   // Float4 columns need D % 4 == 0 and 16-byte aligned rows.

@@ -20,10 +20,11 @@ def _inputs(torch, B, H, N, D, seed):
 
 @pytest.mark.parametrize("B,H,N,D", [
     (1, 4, 8192, 256),   # 32 ranges
-    (1, 1, 514, 96),     # 4 ranges, the last ragged
+    (1, 1, 514, 96),     # 4 ranges, the last ragged: the finalize launch in both forms
     (3, 4, 2050, 65),    # scalar columns, ranges not a multiple of 8 rows apart from the last
+    (1, 1, 1026, 96),    # 8 ranges, the fewest summed in the step, the last ragged
     (1, 2, 4096, 600),   # three column blocks
-    (32, 4, 1024, 64),   # 2 ranges on 128 streams, the most that are split
+    (32, 4, 1024, 64),   # 2 ranges on 128 streams, the most that are split: likewise
 ])
 def test_combined_readout_is_the_finalized_one(B, H, N, D):
     torch = need_gpu()
