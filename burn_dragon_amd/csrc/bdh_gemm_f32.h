@@ -699,8 +699,8 @@ hipError_t launch_gemm(const GemmF32& g, int64_t nwg, hipStream_t st) {
   const bool akc = g.sAk == 1, bkc = g.sBk == 1;
   if ((!akc && g.sAm != 1) || (!bkc && g.sBn != 1) || nwg > INT32_MAX) return hipErrorInvalidValue;
   const dim3 grid((unsigned)nwg);
-  if constexpr (EPI == E_CARRY_SNAP) {  // the state's operands are both contiguous along their rows
-    if (akc || bkc) return hipErrorInvalidValue;
+  if constexpr (EPI == E_CARRY_SNAP) {  // the state's operands are both contiguous along their rows (at one row or column: along k too)
+    if (g.sAm != 1 || g.sBn != 1) return hipErrorInvalidValue;
     hipLaunchKernelGGL((gemm_split_kernel<EPI, KSCALE, false, false, BT>), grid, dim3(256), 0, st, g, ntx, nty);
   } else if (akc && bkc)
     hipLaunchKernelGGL((gemm_split_kernel<EPI, KSCALE, true, true, BT>), grid, dim3(256), 0, st, g, ntx, nty);

@@ -25,6 +25,8 @@ TOL = 3e-6
     (1, 1, 1, 1030, 36, 12, True, [0.999]),        # the backward's second interval, three of the forward
     (2, 2, 1, 513, 130, 70, True, [0.99, 0.999]),  # two state intervals, the last short
     (16, 1, 1, 700, 1030, 72, False, None),        # two intervals, 128-row tiles, split k over both
+    (1, 2, 1, 1030, 6, 1, True, [0.99, 0.9]),      # three intervals, one column: both strides of an operand are 1
+    (2, 1, 1, 1030, 1, 3, True, None),             # three intervals, one row of the state
 ])
 def test_edges_match_oracle(oracle, B, H, Hv, T, N, D, rho, decay):
     torch = need_gpu()
