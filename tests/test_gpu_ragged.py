@@ -1,6 +1,8 @@
 """Sequences whose length is no multiple of a tile: the layer's 128-token
 tiles with missing rows (bdh_lowrank_layer_fwd), and a call of one interval
 that continues a state, on both of its routes."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -39,14 +41,38 @@ def test_layer_tiles_match_oracle(oracle, B, H, T, N, D, carried):
         assert rel_l2(host(out.rho), rref) <= TOL_BF16
 
 
-@pytest.mark.parametrize("B,T,N,D,rope,decay,inplace", [
-    (1, 130, 512, 96, 5, None, False),                          # few elements: gram, readout and state units
-    (1, 130, 512, 96, None, [0.99, 0.98, 0.97, 0.96], True),
-    (2, 390, 8192, 64, 5, None, False),                         # many: the state-carry form
-    (2, 390, 8192, 64, 5, None, True),
-    (2, 390, 8192, 64, None, [0.99, 0.98, 0.97, 0.96], False),
+def _launches(bd, run):
+    """run()'s result, and its launches of the prefill kernels and in all: a
+    call of one interval makes (2, 4) in the state-carry form; in the other
+    one launch of gram, readout and state units, (1, 4), or two in place,
+    (2, 5)."""
+    from burn_dragon_amd import _lib
+    lib = _lib.load()
+    bd.recurrent_profile_enable(True)
+    bd.recurrent_profile_reset()
+    assert lib.bdh_profile_kernel_timing(1) == _lib.BDH_OK
+    try:
+        out = run()
+        ms, n = ctypes.c_double(), ctypes.c_int64()
+        assert lib.bdh_profile_kernel_get(_lib.BDH_KERNEL_PREFILL, ctypes.byref(ms), ctypes.byref(n)) == _lib.BDH_OK
+        return out, (n.value, bd.recurrent_profile_snapshot().launches)
+    finally:
+        lib.bdh_profile_kernel_timing(0)
+        bd.recurrent_profile_enable(False)
+
+
+@pytest.mark.parametrize("B,T,N,D,rope,decay,inplace,carry", [
+    (1, 130, 512, 96, 5, None, False, False),                    # few elements: gram, readout and state units
+    (1, 130, 512, 96, None, [0.99, 0.98, 0.97, 0.96], True, False),
+    (2, 390, 8192, 64, 5, None, False, False),                   # many, few columns: the same
+    (2, 390, 8192, 64, 5, None, True, False),
+    (2, 390, 8192, 64, None, [0.99, 0.98, 0.97, 0.96], False, False),
+    (4, 390, 8192, 192, 5, None, False, True),                   # many: the state-carry form
+    (4, 390, 8192, 192, 5, None, True, True),
+    (4, 390, 8192, 192, None, [0.99, 0.98, 0.97, 0.96], False, True),
+    (4, 390, 8192, 192, 5, [0.99, 0.98, 0.97, 0.96], True, True),
 ])
-def test_one_interval_onto_a_state(oracle, B, T, N, D, rope, decay, inplace):
+def test_one_interval_onto_a_state(oracle, B, T, N, D, rope, decay, inplace, carry):
     torch = need_gpu()
     import burn_dragon_amd as bd
     H = 4
@@ -59,9 +85,11 @@ def test_one_interval_onto_a_state(oracle, B, T, N, D, rope, decay, inplace):
     tx, tv = dev(torch, x, torch.bfloat16), dev(torch, v, torch.bfloat16)
     tr, td = dev(torch, rho0), dev(torch, d) if decay else None
     kw = dict(inplace=inplace)
-    out = (bd.try_fused_recurrent_attention(tx, tv, tr, td, **kw) if rope is None else
-           bd.try_fused_recurrent_attention_rope(tx, tv, tr, td, position=rope, **kw))
+    out, n = _launches(bd, lambda: (
+        bd.try_fused_recurrent_attention(tx, tv, tr, td, **kw) if rope is None else
+        bd.try_fused_recurrent_attention_rope(tx, tv, tr, td, position=rope, **kw)))
     torch.cuda.synchronize()
+    assert n == ((2, 4) if carry else (2, 5) if inplace else (1, 4))
     assert (out.rho.data_ptr() == tr.data_ptr()) == inplace
     if not inplace:
         assert np.array_equal(host(tr), rho0)
