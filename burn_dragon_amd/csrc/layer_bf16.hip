@@ -7,9 +7,9 @@
 //   a    = LN(attn(q, v = cur))          [B, H, T, D]   (prefill_bf16.hip, ln_rows)
 //   y    = ReLU(a Ev_h) * x              [B, H, T, N]   (GEMM Y, written over x)
 //   z    = y' Dec, y' = [B*T, H*N]       [B, T, D]      (GEMM Z, split-K partials;
-//                                                         with T % 256 == 0 and D <= 256
-//                                                         one launch computes y tile by
-//                                                         tile and never stores it)
+//                                                         with D <= 256, where faster, one
+//                                                         launch computes y tile by tile
+//                                                         and never stores it)
 //   next = LN(cur + LN(z))               [B, T, D]      (residual_kernel)
 //
 // LN is DragonNorm's LayerNorm arm with gamma = 1, beta = 0, eps = 1e-5 and
@@ -18,6 +18,9 @@
 // K-contiguous bf16 rows: cur and the LN'd attention rows (K = D), the
 // packed weights (encoders [H, N, D], decoder [D, H*N]) and y (K = H*N,
 // contiguous inside a head's N).
+#include <algorithm>
+#include <type_traits>
+
 #include "bdh_mfma.h"
 
 namespace bdh {
@@ -324,11 +327,9 @@ __global__ __launch_bounds__(NT, 2) void layer_gemm_kernel(LayerGemmArgs g) {
 constexpr int XR_T = 128;                      // tile edge (tokens and latents)
 // Row tiles of a sequence of T tokens: of 128 tokens, the last perhaps fewer.
 __host__ __device__ inline int tiles_of(int64_t T) { return (int)((T + XR_T - 1) / XR_T); }
-// The wave-role GEMM X and the fused Y + Z launch fetch, multiply and do not
+// (The wave-role GEMM X and the fused Y + Z launch fetch, multiply and do not
 // store a sequence's last tile's missing rows, which the 256-row tiles of the
-// separate GEMMs pack away; they still win while at least half of their rows
-// are tokens (B2 T777 N8192 D256: X 76 -> 60 us, Y and Z 147 -> 110 us).
-bool tiles_filled(int64_t T) { return (int64_t)tiles_of(T) * XR_T <= 2 * T; }
+// separate GEMMs pack away: x_roles_groups and yz_splits weigh the two.)
 // Rows past a buffer's last that those tiles may fetch.
 constexpr int64_t kTilePad = XR_T;
 constexpr int XR_EBLK = XR_T * BK * 2;         // bytes of one 32-deep block of 128 rows
@@ -1130,17 +1131,24 @@ hipError_t launch_gemm(const LayerGemmArgs& g, hipStream_t st) {
 
 // Row-tile groups of the two-role GEMM X (layer_x_roles_kernel), or 0 where
 // the shape needs layer_gemm_kernel<G_X>: x wanted in f32 (the decode step),
-// few rows, mostly empty row tiles, N not a multiple of 128, D not a multiple
-// of 32, under 64 or above 256, or more 128-latent column tiles than CUs.  A workgroup per column
-// tile and group; the groups split the row tiles.
+// few rows, N not a multiple of 128, D not a multiple of 32, under 64 or above
+// 256, or more 128-latent column tiles than CUs; or is faster there.  A
+// workgroup per column tile and group; the groups split the row tiles.
+//
+// A workgroup's row tile of 128 tokens takes about 1 / 2.9 of the time of a
+// packed 256-row tile of layer_gemm_kernel (3.1 against 9 us at N8192 D256
+// nh4), which takes no less for a chip that 1.3 of them would fill.  Both
+// routes were measured over 5501 shapes (N 1024-8192, D 64-256, B 1-40, T
+// 9-1500), and the faster one is taken but for 4.9 % of a layer at most.  The
+// roles at N8192 D256 B16: T135 (32 tiles, 9 packed) 20 us slower, T160 3
+// slower, T180 (12 packed) 14 faster, T128 (16 and 8) 16 faster.
 int x_roles_groups(const LayerGemmArgs& g) {
-  if (g.xf || g.M <= SK_MAXM || !tiles_filled(g.T) || g.N % XR_T != 0 || g.D % BK != 0 || g.D < 2 * BK ||
-      g.D > T256)
-    return 0;
+  if (g.xf || g.M <= SK_MAXM || g.N % XR_T != 0 || g.D % BK != 0 || g.D < 2 * BK || g.D > T256) return 0;
   const int64_t ct = g.H * g.N / XR_T, mt = g.B * tiles_of(g.T), cus = device_cus();
   if (ct > cus) return 0;
-  const int64_t r = cus / ct;
-  return (int)(r < mt ? r : mt);
+  const int64_t groups = std::min<int64_t>(cus / ct, mt);
+  const double packed = (double)cdiv(g.M, T256) * ct / cus;
+  return (double)cdiv(mt, groups) <= 2.9 * std::max(1.3, packed) ? (int)groups : 0;
 }
 
 hipError_t launch_x(const LayerGemmArgs& g, hipStream_t st) {
@@ -1154,27 +1162,60 @@ hipError_t launch_x(const LayerGemmArgs& g, hipStream_t st) {
   return hipGetLastError();
 }
 
+// Decoder split-K of GEMM Z (256 x 128 tiles): the fewest splits (each an even
+// number of 32-deep steps) that give at least two workgroups per CU, at most
+// 16.  Few rows: about 8 steps per wave (32 per workgroup), at most 64.
+int z_splits(int64_t M, int64_t HN, int64_t D) {
+  const int64_t steps = HN / 32;
+  int ks = 1;
+  if (M <= SK_MAXM) {
+    while (ks < 64 && steps / (2 * ks) >= 32) ks *= 2;
+    return ks;
+  }
+  const int64_t tiles = (int64_t)cdiv(M, T256) * cdiv(D, T256 / 2);
+  for (int cand = 1; cand <= 16 && steps % (2 * cand) == 0; cand *= 2) {
+    ks = cand;
+    if (tiles * cand >= 512) break;
+  }
+  return ks;
+}
+
 // Split count of the fused Y + Z launch over the 128-latent chunks, or 0
-// where the shape needs GEMM Y and GEMM Z apart: few rows or mostly empty
-// token tiles, D not a multiple of 64 or above 256 (the z tile), DMA offsets
-// past 32 bits.  As many as fill two workgroups a CU, with at least 4 chunks
+// where the shape needs GEMM Y and GEMM Z apart (few rows, D not a multiple of
+// 64 or above 256 (the z tile), DMA offsets past 32 bits) or is faster so.
+// As many as fill two workgroups a CU, with at least 4 chunks
 // each where the chunks allow, and no more than needed for the same longest
 // range (C5: 128 token tiles x 4 splits of 64 chunks; 14 tiles and 256
 // chunks: 32 of 8, not 36: every split writes one more set of partials).
+//
+// Which is faster, from a fit (us) to both routes over the shapes of
+// x_roles_groups' comment.  Fused: the longest range's chunks, each of D / 32
+// Y steps and the z steps, twice as long for two workgroups a CU, and the
+// partials.  Apart: Y's packed tiles, one Z range's steps, its partials, y
+// written and read, a launch.  Apart on a near tie; the slower one is taken
+// by 9 % of a layer at most (8 us, 72 rows).  N8192 D256, fused against apart: B16 T17 +33 us, T65 +4,
+// T96 -16, T135 +3, T160 -38; B1 T65 -25.
 constexpr int YZ_NW = 4;  // waves of the fused launch: 128-token tiles, two workgroups a CU
 constexpr int YZ_TM = YZGeom<YZ_NW>::TM;
 static_assert(YZ_TM == XR_T, "one tiling of the sequences");
 
 int yz_splits(int64_t M, int64_t H, int64_t T, int64_t N, int64_t D) {
-  if (M <= SK_MAXM || !tiles_filled(T) || D % 64 != 0 || D > T256) return 0;
-  const int64_t HN = H * N;
+  if (M <= SK_MAXM || D % 64 != 0 || D > T256) return 0;
+  const int64_t HN = H * N, cus = device_cus();
   if (HN % YZ_C != 0 || (int64_t)YZ_TM * N * 2 >= ((int64_t)1 << 32)) return 0;
   const int64_t tiles = M / T * tiles_of(T), nc = HN / YZ_C;
-  int64_t ks = (int64_t)device_cus() * (8 / YZ_NW) / tiles;
-  if (ks > nc / 4) ks = nc / 4;
-  if (ks < 1) ks = 1;
-  const int64_t longest = (nc + ks - 1) / ks;
-  return (int)((nc + longest - 1) / longest);
+  int64_t ks = std::max<int64_t>(1, std::min(cus * (8 / YZ_NW) / tiles, nc / 4));
+  const int64_t longest = cdiv(nc, ks);
+  ks = cdiv(nc, longest);
+  auto rounds = [&](int64_t wgs) { return wgs <= cus ? 1.0 : 2.0 * cdiv(wgs, 2 * cus); };
+  const int64_t packed = cdiv(M, T256);
+  const int kz = z_splits(M, HN, D);
+  const double steps = (double)D / 32, partial = 0.6 * (double)(M * D) * 8 / 4.5e6;
+  const double fused = (double)longest * (0.3 * steps + 2.25) * rounds(tiles * ks) + (double)ks * partial;
+  const double apart = std::max(1.0, (double)(packed * nc) / cus) * (0.5 * steps + 1.0) +
+                       0.55 * (double)(HN / 32) / kz * rounds(packed * cdiv(D, T256 / 2) * kz) + kz * partial +
+                       0.85 * (double)(M * HN) * 4 / 4.5e6 + 3.0;
+  return fused <= 0.95 * apart ? (int)ks : 0;
 }
 
 hipError_t launch_yz(const LayerGemmArgs& g, hipStream_t st) {
@@ -1306,24 +1347,9 @@ bdh_status run_layer(const LayerArgs& a, hipStream_t st, uint64_t* launches) {
   // write all of rho.
   const bool decode = a.T == 1 && a.rho_in != nullptr && a.rho_in == a.rho_out;
   void *curb = nullptr, *xy = nullptr, *attn = nullptr, *an = nullptr, *zp = nullptr;
-  // Decoder split-K.  256 x 128 tiles: the fewest splits (each an even
-  // number of 32-deep steps) that give at least two workgroups per CU, at
-  // most 16.  Few rows: about 8 steps per wave (32 per workgroup), at most 64.
-  const int64_t nkz = HN / 32;
-  // GEMM Y fused into GEMM Z (y never reaches HBM) where the shape allows.
+  // GEMM Y fused into GEMM Z (y never reaches HBM) where that is possible and faster.
   const int ks_yz = decode ? 0 : yz_splits(M, a.H, a.T, a.N, a.D);
-  int ks = 1;
-  if (ks_yz > 0) {
-    ks = ks_yz;
-  } else if (M <= SK_MAXM) {
-    while (ks < 64 && nkz / (2 * ks) >= 32) ks *= 2;
-  } else {
-    const int64_t tiles_z = (int64_t)cdiv(M, T256) * cdiv(a.D, T256 / 2);
-    for (int cand = 1; cand <= 16 && nkz % (2 * cand) == 0; cand *= 2) {
-      ks = cand;
-      if (tiles_z * cand >= 512) break;
-    }
-  }
+  const int ks = ks_yz > 0 ? ks_yz : z_splits(M, HN, a.D);
   bdh_status s = scratch(st, SLOT_LAYER_CUR, (size_t)((M + kTilePad) * a.D) * sizeof(bf16_t), &curb);
   if (s != BDH_OK) return s;
   s = scratch(st, SLOT_LAYER_XY, (size_t)((S * a.T + kTilePad) * a.N) * sizeof(bf16_t), &xy);

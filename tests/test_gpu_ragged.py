@@ -11,36 +11,6 @@ from tests.gpu_util import TOL_BF16, announce, dev, host, need_gpu, rel_l2
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("B,H,T,N,D,carried", [
-    (2, 2, 65, 256, 64, False),    # one tile a sequence, just over half filled
-    (2, 2, 63, 256, 64, True),     # under half: the separate GEMMs
-    (3, 1, 129, 256, 128, True),   # a second tile of one row
-    (1, 2, 255, 512, 256, False),  # one row short of two tiles
-    (5, 2, 200, 256, 192, True),   # ten tiles, splits of unequal chunk counts
-])
-def test_layer_tiles_match_oracle(oracle, B, H, T, N, D, carried):
-    torch = need_gpu()
-    import burn_dragon_amd as bd
-    rng = np.random.default_rng(T * 3 + N)
-    cur = oracle.layer_norm_f64(rng.standard_normal((B, T, D))).astype(np.float32)
-    enc, encv = ((rng.standard_normal((H, D, N)) * 0.05).astype(np.float32) for _ in range(2))
-    dec = (rng.standard_normal((H * N, D)) * 0.05).astype(np.float32)
-    rho0 = (rng.standard_normal((B, H, N, D)) * 0.05).astype(np.float32) if carried else None
-    w = bd.LowRankWeights.pack(dev(torch, enc[None]), dev(torch, encv[None]), dev(torch, dec))
-    announce("layer tiles", B, H, T, N, D, carried)
-    # Scratch rows past the last token hold whatever was there: make it NaN.
-    big = torch.full((B, T + 200, D), float("nan"), device="cuda")
-    bd.lowrank_layer_forward(big, w, position=0)
-    out = bd.lowrank_layer_forward(dev(torch, cur), w, position=7, rho=dev(torch, rho0) if carried else None,
-                                   want_rho=carried)
-    torch.cuda.synchronize()
-    nref, rref = oracle.lowrank_layer_f64(cur, oracle.round_bf16(enc), oracle.round_bf16(encv),
-                                          oracle.round_bf16(dec), pos0=7, rho0=rho0)
-    assert rel_l2(host(out.next), nref) <= TOL_BF16
-    if carried:
-        assert rel_l2(host(out.rho), rref) <= TOL_BF16
-
-
 def _launches(bd, run):
     """run()'s result, and its launches of the prefill kernels and in all: a
     call of one interval makes (2, 4) in the state-carry form; in the other
@@ -59,6 +29,46 @@ def _launches(bd, run):
     finally:
         lib.bdh_profile_kernel_timing(0)
         bd.recurrent_profile_enable(False)
+
+
+# x: the wave-role GEMM X; yz: GEMM Y and the decoder in one launch.  Both take
+# a sequence in tiles of 128 tokens, the other routes pack the rows.
+@pytest.mark.parametrize("B,H,T,N,D,carried,yz", [
+    (2, 2, 65, 256, 64, False, False),     # x: one tile a sequence, just over half filled
+    (2, 2, 63, 256, 64, True, False),      # x: just under half
+    (3, 1, 129, 512, 128, True, False),    # x: a second tile of one row
+    (1, 2, 255, 512, 256, False, False),   # x: one row short of two tiles
+    (5, 2, 200, 256, 192, True, False),    # x: ten tiles
+    (5, 4, 20, 8192, 64, False, True),     # packed x: five row tiles for 100 rows
+    (2, 4, 33, 2048, 64, False, True),     # a quarter filled
+    (3, 2, 129, 4096, 128, True, True),    # a second tile of one row
+    (1, 4, 255, 4096, 256, False, True),   # one row short of two tiles
+    (20, 4, 100, 3328, 64, True, True),    # 20 tiles, ranges of unequal chunk counts
+])
+def test_layer_tiles_match_oracle(oracle, B, H, T, N, D, carried, yz):
+    torch = need_gpu()
+    import burn_dragon_amd as bd
+    rng = np.random.default_rng(T * 3 + N)
+    cur = oracle.layer_norm_f64(rng.standard_normal((B, T, D))).astype(np.float32)
+    enc, encv = ((rng.standard_normal((H, D, N)) * 0.05).astype(np.float32) for _ in range(2))
+    dec = (rng.standard_normal((H * N, D)) * 0.05).astype(np.float32)
+    rho0 = (rng.standard_normal((B, H, N, D)) * 0.05).astype(np.float32) if carried else None
+    w = bd.LowRankWeights.pack(dev(torch, enc[None]), dev(torch, encv[None]), dev(torch, dec))
+    announce("layer tiles", B, H, T, N, D, carried, yz)
+    # Scratch rows past the last token hold whatever was there: make it NaN.
+    big = torch.full((B, T + 200, D), float("nan"), device="cuda")
+    bd.lowrank_layer_forward(big, w, position=0)
+    out, (_, n) = _launches(bd, lambda: bd.lowrank_layer_forward(
+        dev(torch, cur), w, position=7, rho=dev(torch, rho0) if carried else None, want_rho=carried))
+    torch.cuda.synchronize()
+    # Rows to bf16, X, LayerNorm, Y and decoder, residual; the attention's v^T,
+    # scores, context and, onto a state, the readout's sum.
+    assert n == (5 if yz else 6) + (4 if carried else 3)
+    nref, rref = oracle.lowrank_layer_f64(cur, oracle.round_bf16(enc), oracle.round_bf16(encv),
+                                          oracle.round_bf16(dec), pos0=7, rho0=rho0)
+    assert rel_l2(host(out.next), nref) <= TOL_BF16
+    if carried:
+        assert rel_l2(host(out.rho), rref) <= TOL_BF16
 
 
 @pytest.mark.parametrize("B,T,N,D,rope,decay,inplace,carry", [
