@@ -38,7 +38,7 @@ enum ScratchSlot {
   SLOT_LAYER_Z,      // decoder split-K partials     [ks, B*T, D] f32
   SLOT_LAYER_RHO,    // a successor state not kept   [B, H, N, D] f32
   SLOT_DECODE_PART,  // decode range readouts [S, G, D] f32, lists and counts (decode_part_bytes)
-  SLOT_DECODE_CTR,   // decode: ranges of a stream that have finished  [CUs] uint32, 0 between launches
+  SLOT_DECODE_CTR,   // decode: ranges of a stream that have finished, by their count G  [log2 G - 1, CUs] uint32
   SLOT_VJP_S,        // VJP scores tril(QQ^T) * D    [S, T, T] f32
   SLOT_VJP_M,        // VJP tril(G V^T)*D + its transpose  [S, T, T] f32
   SLOT_VJP_TD,       // VJP per-head grad_v, IC, G*d^t  3 x [S, T, D] f32

@@ -43,7 +43,8 @@ constexpr int DR_SMALL_THREADS = 512;
 constexpr int DR_SMALL = 256;
 constexpr int DR_SEG = 8192;       // rows compacted per pass (LDS list capacity)
 constexpr int DR_UNROLL = 8;
-constexpr int DR_MAXG = 32;        // row ranges of a stream
+constexpr int DR_LOGG = 5;
+constexpr int DR_MAXG = 1 << DR_LOGG;  // row ranges of a stream (a power of two)
 constexpr int ROWS_PER_THREAD = 8;  // 4 whole (even, odd) RoPE pairs
 constexpr int DD_THREADS = 256;     // dense step
 constexpr int DD_WAVES = DD_THREADS / 64;
@@ -63,7 +64,7 @@ struct DecodeKernelArgs {
   int H, Hv, N, D;
   int G, rows;        // ranges per stream, rows per range (a multiple of 8)
   float pos;
-  uint32_t* ctr;      // sparse step, G > 1: ranges of each stream done [S] (0 before and after), or null: finalize launch
+  uint32_t* ctr;      // sparse step, G > 1: ranges of each stream done [S] (a multiple of G before and after), or null: finalize launch
   float* a_final;     // with ctr: [S, D]
   bf16_t* an;         // LayerNorm of the readout [S, D] in its place, or null (D <= 256)
 };
@@ -271,11 +272,12 @@ __global__ __launch_bounds__(THREADS) void decode_kernel(DecodeKernelArgs p) {
     // others' rho rows are read by later launches alone.)
     if (wave * 64 < CB) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (tid == 0) {
-      arrived = __hip_atomic_fetch_add(p.ctr + s, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (arrived == (uint32_t)p.G - 1)
-        __hip_atomic_store(p.ctr + s, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    // The counter is never set back: G is a power of two and only steps of G
+    // ranges count on it, so it is a multiple of G between steps (and stays
+    // one through its wrap).  Steps that overlap on one buffer, against the
+    // rule, then spoil their own readouts only, not those of every later step.
+    if (tid == 0)
+      arrived = __hip_atomic_fetch_add(p.ctr + s, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & ((uint32_t)p.G - 1);
     __syncthreads();
     if (arrived != (uint32_t)p.G - 1) return;
     const float* part = p.a_out + s * p.G * p.D;
@@ -540,15 +542,17 @@ bdh_status run_decode(const DecodeArgs& a, hipStream_t st, uint64_t* launches) {
     }
     if (a.idx_out || a.cnt_out) p.cnt_out = (int32_t*)buf;
     if (!a.part_buf) {
-      // (S < CUs wherever a sparse step is split.  Kept by every split step on
-      // the stream, so that a later capture of another form finds it.)
+      // A counter per stream (S < CUs wherever a sparse step is split) for each
+      // count of ranges.  Kept by every split step on the stream, so that a
+      // later capture of another form finds it.
       void* c = nullptr;
-      const bdh_status s = scratch(st, SLOT_DECODE_CTR, (size_t)device_cus() * sizeof(uint32_t), &c, true);
+      const size_t cus = (size_t)device_cus();
+      const bdh_status s = scratch(st, SLOT_DECODE_CTR, DR_LOGG * cus * sizeof(uint32_t), &c, true);
       if (s != BDH_OK) return s;
       // Streams of 2 or 4 ranges keep the finalize launch outside the layer:
       // with that many streams the next step's start hides it (B18 N8192 33.0
       // against 33.9 us, B24 N4096 D128 16.3 against 17.5).
-      if (sparse && !a.idx_out && !a.cnt_out && (G > 4 || a.an)) p.ctr = (uint32_t*)c;
+      if (sparse && !a.idx_out && !a.cnt_out && (G > 4 || a.an)) p.ctr = (uint32_t*)c + (__builtin_ctz(G) - 1) * cus;
     }
   }
   // Float4 columns need D % 4 == 0 and 16-byte aligned rows.

@@ -66,6 +66,45 @@ def test_replays_with_other_steps_between_them():
     bd.release_stream_scratch(st)
 
 
+def test_overlapped_replays_spoil_no_later_step():
+    # Two graphs captured on one stream share its buffers and must not overlap;
+    # where they do all the same, every later replay is right again.
+    torch = need_gpu()
+    import burn_dragon_amd as bd
+    announce("decode combine after overlapped replays")
+    sizes = [(1, 4, 8192, 256), (2, 4, 4096, 128)]  # 32 ranges, 16
+    st, other = torch.cuda.Stream(), torch.cuda.Stream()
+    graphs = []
+    for seed, (B, H, N, D) in enumerate(sizes):
+        x, v, rho = _inputs(torch, B, H, N, D, seed)
+        want = bd.decode_step(x, v, rho.clone(), position=9).readout
+        out, r = torch.empty(B, H, D, device="cuda"), rho.clone()
+        with torch.cuda.stream(st):
+            bd.decode_step(x, v, r, position=9)
+        torch.cuda.synchronize()
+        graphs.append([x, v, rho, r, out, want])
+    for c in graphs + graphs[:1]:
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=st):
+            bd.decode_step(c[0], c[1], c[3], position=9, out=c[4])
+        c.append(g)
+    for i in range(20):
+        for a, b in ((graphs[0][6], graphs[1][6]), (graphs[0][6], graphs[0][7])):
+            with torch.cuda.stream(st):
+                a.replay()
+            with torch.cuda.stream(other):
+                b.replay()
+            torch.cuda.synchronize()
+        for c in graphs:
+            c[3].copy_(c[2])
+            c[4].zero_()
+            c[6].replay()
+            torch.cuda.synchronize()
+            assert torch.equal(c[4], c[5]), i
+    del graphs
+    bd.release_stream_scratch(st)
+
+
 def test_short_streams_are_captured_without_an_eager_call():
     # Fewer than 512 rows: the step takes no scratch, so a stream's first call may be a captured one.
     torch = need_gpu()
