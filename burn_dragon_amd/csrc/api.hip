@@ -55,6 +55,7 @@ struct CallCounters {
   uint64_t allocations = 0, upload_bytes = 0, reuse_hits = 0, reuse_bytes = 0;
 };
 thread_local CallCounters t_call;
+thread_local bool t_no_memory = false;  // the last scratch() found no device memory
 }  // namespace
 
 bdh_status stream_capturing(hipStream_t st, bool* capturing) {
@@ -68,6 +69,7 @@ bdh_status stream_capturing(hipStream_t st, bool* capturing) {
 }
 
 bdh_status scratch(hipStream_t st, int slot, size_t bytes, void** out, bool zero_on_alloc) {
+  t_no_memory = false;
   int dev = 0;
   BDH_HIP_TRY(hipGetDevice(&dev));
   bool capturing = false;
@@ -105,15 +107,52 @@ bdh_status scratch(hipStream_t st, int slot, size_t bytes, void** out, bool zero
       ss.ptr[slot] = nullptr;
       ss.bytes[slot] = 0;
     }
-    const size_t grow = bytes + bytes / 4;
+    size_t grow = bytes + bytes / 4;
     void* p = nullptr;
-    BDH_HIP_TRY(hipMalloc(&p, grow));
+    hipError_t e = hipMalloc(&p, grow);
+    if (e == hipErrorOutOfMemory) {
+      (void)hipGetLastError();
+      grow = bytes;
+      e = hipMalloc(&p, grow);
+    }
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      t_no_memory = e == hipErrorOutOfMemory;
+      return hip_fail(e, "scratch allocation");
+    }
     ++t_call.allocations;
     if (zero_on_alloc) BDH_HIP_TRY(hipMemsetAsync(p, 0, grow, st));
     ss.ptr[slot] = p;
     ss.bytes[slot] = grow;
   }
   *out = ss.ptr[slot];
+  return BDH_OK;
+}
+
+bool scratch_no_memory() { return t_no_memory; }
+
+size_t scratch_held(hipStream_t st, int slot, void** out) {
+  *out = nullptr;
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return 0;
+  std::lock_guard<std::mutex> lock(g_scratch_mu);
+  const ScratchSet& ss = g_sets[{dev, st}];
+  *out = ss.ptr[slot];
+  return ss.bytes[slot];
+}
+
+bdh_status scratch_drop(hipStream_t st, std::initializer_list<int> slots) {
+  int dev = 0;
+  BDH_HIP_TRY(hipGetDevice(&dev));
+  std::lock_guard<std::mutex> lock(g_scratch_mu);
+  ScratchSet& ss = g_sets[{dev, st}];
+  if (ss.captured) return BDH_OK;
+  BDH_HIP_TRY(hipStreamSynchronize(st));
+  for (const int i : slots) {
+    if (ss.ptr[i]) BDH_HIP_TRY(hipFree(ss.ptr[i]));
+    ss.ptr[i] = nullptr;
+    ss.bytes[i] = 0;
+  }
   return BDH_OK;
 }
 
@@ -384,20 +423,8 @@ bdh_status forward_common(const bdh_recurrent_plan* plan, int32_t dtype, const v
       qr = (const float*)rot;
     }
     F32Args a{qr, (const float*)v, want_rho ? rho_in : nullptr, decay, ctx, rho_out, B, H, Hv, T, N, D, want_rho};
-    const F32Scratch need = f32_path_scratch(a);
-    const struct {
-      int slot;
-      size_t elems;
-      float** out;
-    } bufs[] = {{SLOT_SCORES, need.scores, &a.scores}, {SLOT_SNAP, need.states, &a.states},
-                {SLOT_GEMM_PART, need.part, &a.part}};
-    for (const auto& buf : bufs) {
-      if (!buf.elems) continue;
-      void* p = nullptr;
-      st = scratch(hs, buf.slot, buf.elems * sizeof(float), &p);
-      if (st != BDH_OK) return st;
-      *buf.out = (float*)p;
-    }
+    st = f32_path_buffers(&a, hs);
+    if (st != BDH_OK) return st;
     hipError_t e = run_f32_path(a, hs, &prof.launches);
     if (e != hipSuccess) return hip_fail(e, "fp32 path launch");
     prof.done(true);

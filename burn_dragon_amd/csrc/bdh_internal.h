@@ -5,6 +5,7 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <initializer_list>
 #include <string>
 
 #include "bdh_common.h"
@@ -52,6 +53,12 @@ enum ScratchSlot {
 // Scratch of the calling stream (see api.hip): grows on first use of a
 // larger shape, refused (BDH_UNSUPPORTED) while the stream is capturing.
 bdh_status scratch(hipStream_t st, int slot, size_t bytes, void** out, bool zero_on_alloc = false);
+// True when this thread's last scratch() found no device memory.
+bool scratch_no_memory();
+// What a slot holds now, without growing it (0 bytes: nothing).
+size_t scratch_held(hipStream_t st, int slot, void** out);
+// Frees these slots' buffers (after the stream's queued work).  Not under capture.
+bdh_status scratch_drop(hipStream_t st, std::initializer_list<int> slots);
 // Frees the scratch kept for `st` on the current device (after the stream's
 // queued work), including buffers retired while a graph held them.
 bdh_status scratch_release(hipStream_t st);
@@ -89,17 +96,18 @@ struct F32Args {
   float* rho_out;       // [S, N, D]
   int64_t B, H, Hv, T, N, D;
   bool state;           // false: context only (single interval, no rho)
-  // Scratch (f32_path_scratch).
-  float* scores = nullptr;
-  float* states = nullptr;
-  float* part = nullptr;
+  // Scratch, set by f32_path_buffers, and the limits it was sized for.
+  float* scores = nullptr;  // of a group of intervals [intervals, S, L, L]
+  float* states = nullptr;  // at its interval starts but the first [intervals - 1, S, N, D]
+  float* part = nullptr;    // the GEMMs' split-K partials
+  size_t part_elems = 0;
+  int64_t max_len = kF32Interval;  // most tokens of an interval
+  int64_t max_group = INT64_MAX;   // most intervals of a group
 };
-struct F32Scratch {
-  size_t scores;  // floats: scores of a group of intervals [intervals, S, L, L]
-  size_t states;  // states at its interval starts but the first [intervals - 1, S, N, D]
-  size_t part;    // the GEMMs' split-K partials
-};
-F32Scratch f32_path_scratch(const F32Args& a);
+// Takes the stream's scratch for the call.  Where device memory is short, or
+// under capture what the stream holds, the groups shrink to one interval, and
+// the intervals to 256 tokens.
+bdh_status f32_path_buffers(F32Args* a, hipStream_t st);
 hipError_t run_f32_path(const F32Args& a, hipStream_t st, uint64_t* launches);
 
 // --- bf16 MFMA path (prefill_bf16.hip) --------------------------------------

@@ -677,8 +677,17 @@ bdh_status run_bf16_path(const Bf16Args& a, hipStream_t st, uint64_t* launches) 
   const bool carried1 =
       a.rho_in != nullptr && a.T > T256 && a.D > T256 / 2 && S * a.T * a.N >= ((int64_t)48 << 20);
   if (a.state && (n_iv >= 2 || carried1) && a.D * a.N * 2 < ((int64_t)1 << 31) &&
-      (size_t)(n_iv * S * a.N * a.D) * sizeof(bf16_t) <= kCarrySnapMax)
-    return run_carry_path(a, st, launches, S, Tp, Dp, n_iv, Lp, nb, nk);
+      (size_t)(n_iv * S * a.N * a.D) * sizeof(bf16_t) <= kCarrySnapMax) {
+    const bdh_status r = run_carry_path(a, st, launches, S, Tp, Dp, n_iv, Lp, nb, nk);
+    // (One interval also runs without the snapshot and the q stream, where
+    // there is no memory for them or, under capture, the stream holds none;
+    // they are taken before the first launch.)
+    const bool short_of_memory = scratch_no_memory();
+    if (n_iv >= 2 || (r != BDH_UNSUPPORTED && !short_of_memory)) return r;
+    const bdh_status d =
+        short_of_memory ? scratch_drop(st, {SLOT_SCORES, SLOT_SNAP, SLOT_READOUT, SLOT_ROTATED}) : BDH_OK;
+    if (d != BDH_OK) return d;
+  }
   if (!a.state && a.rho_in == nullptr && a.freqs == nullptr && a.decay == nullptr && n_iv == 1)
     return run_gram_path(a, st, launches, S, Tp, Dp, Lp, nb, nk);
   if (n_iv == 1 && a.freqs != nullptr && a.decay == nullptr && a.rho_in == nullptr && a.T % T256 == 0 &&

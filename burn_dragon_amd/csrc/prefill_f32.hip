@@ -26,9 +26,12 @@ using namespace gf32;
 namespace {
 
 // Most scratch for scores and states between intervals: longer sequences run
-// as groups of intervals, each group as above.
-constexpr int64_t kScoresMax = (int64_t)1 << 30;  // bytes
-constexpr int64_t kStatesMax = (int64_t)4 << 30;
+// as groups of intervals, each group as above.  (B8 nh4 T4096 N8192 D256: 5
+// intervals a group, 1.1 GB of states.)
+constexpr int64_t kScoresMax = (int64_t)256 << 20;  // bytes
+constexpr int64_t kStatesMax = (int64_t)1 << 30;
+// Interval a call falls back to where memory is short.
+constexpr int64_t kShortInterval = 256;
 
 struct Intervals {
   int64_t L, n, group;  // tokens of an interval, intervals, intervals of a group
@@ -46,22 +49,24 @@ Intervals intervals(const F32Args& a) {
     v.n = v.group = 1;
     return v;
   }
-  v.n = (a.T + kF32Interval - 1) / kF32Interval;
+  v.n = (a.T + a.max_len - 1) / a.max_len;
   v.L = v.n == 1 ? a.T : ((a.T + v.n - 1) / v.n + 127) / 128 * 128;
   v.n = (a.T + v.L - 1) / v.L;
   int64_t g = kScoresMax / (S * v.L * v.L * 4);
   g = std::min(g, kStatesMax / (S * a.N * a.D * 4) + 1);
-  g = std::min(g, kMaxBatch / S);
+  g = std::min({g, kMaxBatch / S, a.max_group});
   v.group = std::max<int64_t>(1, std::min(g, v.n));
   return v;
 }
 
-}  // namespace
+struct Scratch {
+  size_t scores, states, part;  // floats of F32Args' buffers
+};
 
-F32Scratch f32_path_scratch(const F32Args& a) {
+Scratch scratch_of(const F32Args& a) {
   const int64_t S = a.B * a.H;
   const Intervals v = intervals(a);
-  F32Scratch w;
+  Scratch w;
   w.scores = (size_t)(v.group * S * v.L * v.L);
   w.states = (size_t)((v.group - 1) * S * a.N * a.D);
   // Split-K partials: the gram and readout (K = N) and S V (K = L), of the
@@ -77,10 +82,45 @@ F32Scratch f32_path_scratch(const F32Args& a) {
   return w;
 }
 
+}  // namespace
+
+bdh_status f32_path_buffers(F32Args* a, hipStream_t st) {
+  for (;;) {
+    const Scratch need = scratch_of(*a);
+    void *scores = nullptr, *states = nullptr, *part = nullptr;
+    bdh_status s = scratch(st, SLOT_SCORES, need.scores * sizeof(float), &scores);
+    if (s == BDH_OK && need.states) s = scratch(st, SLOT_SNAP, need.states * sizeof(float), &states);
+    a->part_elems = need.part;
+    if (s == BDH_OK && need.part) {
+      s = scratch(st, SLOT_GEMM_PART, need.part * sizeof(float), &part);
+      if (s == BDH_UNSUPPORTED) {  // capturing: fewer split-K ranges in what is there
+        a->part_elems = std::min(need.part, scratch_held(st, SLOT_GEMM_PART, &part) / sizeof(float));
+        s = BDH_OK;
+      }
+    }
+    a->scores = (float*)scores;
+    a->states = (float*)states;
+    a->part = (float*)part;
+    const bool short_of_memory = scratch_no_memory();
+    if (s == BDH_OK || (s != BDH_UNSUPPORTED && !short_of_memory)) return s;
+    const Intervals v = intervals(*a);
+    if (v.group > 1) {
+      a->max_group = v.group / 2;
+    } else if (a->state && v.L > kShortInterval) {
+      a->max_len = kShortInterval;
+      a->max_group = 1;
+    } else {
+      return s;
+    }
+    if (short_of_memory) s = scratch_drop(st, {SLOT_SCORES, SLOT_SNAP, SLOT_GEMM_PART});
+    if (short_of_memory && s != BDH_OK) return s;
+  }
+}
+
 hipError_t run_f32_path(const F32Args& a, hipStream_t st, uint64_t* launches) {
   const int64_t S = a.B * a.H, H = a.H, T = a.T, N = a.N, D = a.D;
   const Intervals v = intervals(a);
-  const size_t pe = f32_path_scratch(a).part;
+  const size_t pe = a.part_elems;
   const int64_t L = v.L, sVo = a.Hv * T * D, sVi = a.Hv == 1 ? 0 : T * D;
   const float* rho_cur = a.rho_in;
   uint64_t n = 0;

@@ -92,3 +92,92 @@ def test_values_without_bf16_parts(T, N, D):
         cols = np.arange(D) != 4 if rows.start == 0 else slice(None)
         np.testing.assert_allclose(got[rows][:, cols], ctx[rows][:, cols], rtol=1e-5)
     np.testing.assert_allclose(host(out.rho)[0, 0], rho, rtol=1e-5)
+
+
+@pytest.mark.parametrize("T,decay", [(4200, [0.999, 0.99, 0.9999, 0.9]), (4608, None)])
+def test_groups_of_intervals(oracle, T, decay):
+    # The scores of 128 streams fill a group with two intervals: nine of them
+    # are five groups, the last a single (and, at T = 4200, a shorter) one.
+    torch = need_gpu()
+    import burn_dragon_amd as bd
+    B, H, N, D = 32, 4, 32, 16
+    g = torch.Generator(device="cuda").manual_seed(T)
+    q = torch.randn(B, H, T, N, generator=g, device="cuda")
+    v = torch.randn(B, 1, T, D, generator=g, device="cuda") / 16
+    rho = torch.randn(B, H, N, D, generator=g, device="cuda") * 0.2
+    d = dev(torch, np.asarray(decay, np.float32)) if decay else None
+    announce("f32 groups of intervals", T, decay)
+    out = bd.try_fused_recurrent_attention(q, v, rho.clone(), d)
+    r = rho.clone()
+    inplace = bd.try_fused_recurrent_attention(q, v, r, d, inplace=True)
+    torch.cuda.synchronize()
+    assert torch.equal(out.context, inplace.context) and torch.equal(out.rho, r)
+    for b, h in ((0, 0), (13, 2), (31, 3)):
+        ctx, rho1 = oracle.recurrent_f64(host(q[b, h])[None, None], host(v[b, 0])[None, None], host(rho[b, h])[None, None],
+                                         np.asarray(decay[h:h + 1], np.float32) if decay else None)
+        assert rel_l2(host(out.context[b, h]), ctx[0, 0]) <= TOL
+        assert rel_l2(host(out.rho[b, h]), rho1[0, 0]) <= TOL
+
+
+def test_groups_shrink_where_memory_is_short():
+    # Eight intervals in one group hold 0.7 GB of states and scores: with less
+    # than that left on the device the call runs in smaller groups.
+    torch = need_gpu()
+    import burn_dragon_amd as bd
+    B, H, T, N, D = 4, 4, 4096, 4096, 256
+    g = torch.Generator(device="cuda").manual_seed(1)
+    q = torch.randn(B, H, T, N, generator=g, device="cuda")
+    v = torch.randn(B, 1, T, D, generator=g, device="cuda") / 16
+    announce("f32 groups, memory short")
+    want = bd.try_fused_recurrent_attention(q, v)
+    spare = bd.try_fused_recurrent_attention(q, v)  # its outputs' memory, kept for the next call
+    torch.cuda.synchronize()
+    bd.release_stream_scratch()
+    del spare
+    hold = []
+    try:
+        free = torch.cuda.mem_get_info()[0]
+        while free > 400 << 20:
+            hold.append(torch.empty(min(free - (300 << 20), 32 << 30), dtype=torch.uint8, device="cuda"))
+            free = torch.cuda.mem_get_info()[0]
+        out = bd.try_fused_recurrent_attention(q, v)
+        torch.cuda.synchronize()
+    finally:
+        del hold
+        bd.release_stream_scratch()
+        torch.cuda.empty_cache()
+    assert rel_l2(host(out.context), host(want.context)) <= TOL
+    assert rel_l2(host(out.rho), host(want.rho)) <= TOL
+
+
+@pytest.mark.parametrize("warm,T", [(256, 1500), (1024, 4096), (4096, 700)])
+def test_captured_in_the_scratch_of_another_length(warm, T):
+    # A capture takes the groups and split-K ranges that the stream's scratch has room for.
+    torch = need_gpu()
+    import burn_dragon_amd as bd
+    B, H, N, D = 1, 4, 512, 64
+    g = torch.Generator(device="cuda").manual_seed(T)
+    q = torch.randn(B, H, max(warm, T), N, generator=g, device="cuda")
+    v = torch.randn(B, 1, max(warm, T), D, generator=g, device="cuda") / 16
+    qt, vt = q[:, :, :T].contiguous(), v[:, :, :T].contiguous()
+    announce("f32 captured", warm, T)
+    want = bd.try_fused_recurrent_attention(qt, vt)
+    st = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(st):
+        bd.try_fused_recurrent_attention(q[:, :, :warm].contiguous(), v[:, :, :warm].contiguous())
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=st):
+        out = bd.try_fused_recurrent_attention(qt, vt)
+    assert out is not None
+    for _ in range(3):
+        out.context.zero_()
+        out.rho.zero_()
+        bd.try_fused_recurrent_attention(qt, vt)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert rel_l2(host(out.context), host(want.context)) <= TOL
+        assert rel_l2(host(out.rho), host(want.rho)) <= TOL
+    del graph
+    bd.release_stream_scratch(st)
