@@ -6,8 +6,8 @@
 //   X(i, j) = X + (b / H) * sXo + (b % H) * sXi + i * sXr + j * sXc
 //
 // The fp32 MFMAs run at 1/16 of the bf16 rate, so each operand value is split
-// into three bf16 parts whose sum is the value itself (24 significant bits;
-// x = h + m + l, each part the bf16 nearest to what is left) and the product
+// into three bf16 parts whose sum is the value itself (24 significant bits
+// above 2^-110; x = h + m + l, each part the bf16 nearest to what is left) and the product
 // is the six part products down to 2^-16 of the largest:
 //   a b = ah bh + (ah bm + am bh) + (am bm + ah bl + al bh)
 // on v_mfma_f32_32x32x16_bf16 (exact products, fp32 accumulation).  What is
@@ -22,8 +22,8 @@
 // Workgroups of 256 threads own BT x BT output tiles (BT = 128, or 64 for
 // small products), each wave a quarter.  K steps are 16 deep: two steps'
 // operands are in flight in registers while a third is multiplied from LDS;
-// a thread splits each value it fetched once per tile (5.5 VALU instructions
-// a value, about half the step's MFMA time) and writes the three parts to
+// a thread splits each value it fetched once per tile (6 VALU instructions
+// a value with the largest operand's, about half the step's MFMA time) and writes the three parts to
 // LDS, double-buffered, so one barrier a step suffices and two workgroups a
 // CU overlap one's splitting with the other's MFMAs.
 // A long K with few tiles is split into P ranges (split-K): each range's
@@ -31,8 +31,12 @@
 // adds the P partials in range order (deterministic) and applies the
 // epilogue.
 // Values whose parts do not exist (infinities, NaN, or above bf16's largest)
-// and sums past fp32's range make the result not finite; a wave that sees
-// one in its block computes the block again with the fp32 MFMA.
+// and sums past fp32's range make the result not finite, and operands below
+// about 2^-110 lose low bits in their parts; a wave that sees a sum that is
+// not finite, or one so much smaller than the tile's largest operand that lost
+// bits could show (kLost), computes its block again with the fp32 MFMA.  (What
+// stays lost: an operand below 2^-134 has no parts, so a sum of products of
+// such operands alone is 0.)
 #pragma once
 
 #include <type_traits>
@@ -89,6 +93,12 @@ struct GemmF32 {
 constexpr int GK = 16;               // k step
 constexpr int TRI = 128;             // edge of the blocks a masked product is computed (and written) in
 constexpr int DSCALE = 1024;         // KSCALE: most k of one workgroup (LDS table of d^(kpow - k))
+
+// A sum smaller than this share of the tile's largest operand may lack bits:
+// an operand's parts end at 2^-133, bf16's smallest, so the sum is off by up
+// to sqrt(K) 2^-134 of the largest operand (2^-127.5 at K = 8192), and that
+// has to stay below its own 2^-24.
+constexpr float kLost = 0x1p-104f;
 
 __device__ __forceinline__ float dpowf(float d, int e) { return powf(d, (float)e); }
 
@@ -210,9 +220,13 @@ __device__ __forceinline__ void split_store(char* lds, const Loader<BT, KC>& l, 
 #pragma unroll
   for (int i = 0; i < E / 2; ++i) {
     const float x = v[2 * i], y = v[2 * i + 1];
-    const uint32_t h = pack_bf16x2(x, y);
+    // (The pair stays one register: left to itself the compiler converts the
+    // low value a second time, 16 more instructions a step of 107.)
+    uint32_t h = pack_bf16x2(x, y);
+    asm("" : "+v"(h));
     const float rx = x - bf16_lo(h), ry = y - bf16_hi(h);
-    const uint32_t m = pack_bf16x2(rx, ry);
+    uint32_t m = pack_bf16x2(rx, ry);
+    asm("" : "+v"(m));
     w[0][i] = h;
     w[1][i] = m;
     w[2][i] = pack_bf16x2(rx - bf16_lo(m), ry - bf16_hi(m));
@@ -255,6 +269,8 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
   constexpr int E = BT / 16, NB = BT / 64;  // values a thread stages; 32 x 32 blocks a wave, each way
   constexpr int PA = kPart<BT, AKC>, PB = kPart<BT, BKC>, STAGE = 3 * (PA + PB);
   __shared__ __attribute__((aligned(16))) char lds[2 * STAGE + (KSCALE ? 4 * (DSCALE + 3 * GK) : 0)];
+  __shared__ float wmax[4];  // the waves' largest staged operands
+  __shared__ int wask[4];
   const int t = threadIdx.x, lane = t & 63, w = wave_id();
   const int wm = w >> 1, wn = w & 1;
   // Workgroup ids are remapped so that each XCD (id % 8) takes a contiguous
@@ -332,6 +348,7 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
   int siv = 0, soff = 0;  // the interval and offset of the step staged next
 
   float va[2][E], vb[2][E];
+  float mx = 0.0f;  // the largest operand staged by this thread
   auto load = [&](int s, float (&a)[E], float (&bv)[E]) {
     la.load(s * GK, Kt, a);
     lb.load(s * GK, Kt, bv);
@@ -349,8 +366,17 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
         }
       }
     }
+    // (After the splitting where both operands are contiguous along k: the f32
+    // C2 shape's gram 398 us against 420; the others' best place is before it.)
+    auto largest = [&]() {
+#pragma unroll
+      for (int e = 0; e < E; ++e) mx = fmaxf(fmaxf(mx, fabsf(a[e])), fabsf(bv[e]));
+      asm volatile("" : "+v"(mx));  // here, not where copies of the values would have to live to
+    };
+    if (!(AKC && BKC)) largest();
     split_store(o, la, a);
     split_store(o + 3 * PA, lb, bv);
+    if (AKC && BKC) largest();
   };
 
   floatx16 big[NB][NB], small[NB][NB];
@@ -392,7 +418,14 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
   // an interval's sum always was: one sum over all of them would round to the
   // growing state's last bit).
   const float* X = P > 1 ? nullptr : epi_addend<EPI>(g, c0);
-  bool bad = false;  // a sum is not finite
+  // Of the sums seen: one is not finite; the smallest that is not 0, as twice
+  // its bits less one (0: the largest number there is).
+  bool bad = false;
+  uint32_t least = ~0u;
+  auto look = [&](float v, float& nan) {
+    nan = fmaf(v, 0.0f, nan);
+    least = min(least, (__builtin_bit_cast(uint32_t, v) << 1) - 1);
+  };
   auto snapshot = [&](int i) {
     float* o = g.snap + i * g.sSnap + c0;
     // (The block's addresses are not kept through the step loop: 64 of them
@@ -400,6 +433,7 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
     int mo = mw + acc_row(lane, 0);
     asm volatile("" : "+v"(mo));
     const float dl = g.decay ? dpowf(d, len_of(i)) : 1.0f;
+    float nan = 0.0f;
 #pragma unroll
     for (int i2 = 0; i2 < NB; ++i2)
 #pragma unroll
@@ -415,7 +449,7 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const float v = big[i2][j][r] + small[i2][j][r];
-          bad |= !__builtin_isfinite(v);
+          look(v, nan);
           if (mo + 32 * i2 + acc_row(0, r) < M && n < N)
             o[off + acc_row(0, r) * g.sCm] = X != nullptr ? v + x[r] * dl : v;
         }
@@ -423,6 +457,7 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
         small[i2][j] = zero16();
         __builtin_amdgcn_sched_barrier(0);
       }
+    bad |= nan != 0.0f;
     X = o;
   };
 
@@ -461,6 +496,7 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
     }
   }
 
+  float nan = 0.0f;
 #pragma unroll
   for (int i = 0; i < NB; ++i)
 #pragma unroll
@@ -469,10 +505,26 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
       for (int r = 0; r < 16; ++r) {
         big[i][j][r] += small[i][j][r];
         small[i][j][r] = 0.0f;
-        bad |= !__builtin_isfinite(big[i][j][r]);
+        look(big[i][j][r], nan);
       }
+  bad |= nan != 0.0f;
+  // A sum below kLost of the largest operand of the workgroup asks for the
+  // block again; the largest operand is looked for where one is above kLarge
+  // or a sum below its share.
+  constexpr float kLarge = 0x1p40f;
+  const bool ask = __any(mx >= kLarge || least < (__builtin_bit_cast(uint32_t, kLarge * kLost) << 1) - 1);
+  if (lane == 0) wask[w] = ask;
+  __syncthreads();  // also: every wave has read its last fragments
+  if (wask[0] || wask[1] || wask[2] || wask[3]) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    if (lane == 0) wmax[w] = mx;
+    __syncthreads();
+    const float lost = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3])) * kLost;
+    bad |= least < (__builtin_bit_cast(uint32_t, lost) << 1) - 1;
+  }
   if (__any(bad)) {
-    // Not finite: the block again on v_mfma_f32_32x32x2_f32, straight from memory.
+    // The block again on v_mfma_f32_32x32x2_f32, straight from memory.
     if (SNAP) X = epi_addend<EPI>(g, c0);
 #pragma unroll
     for (int i = 0; i < NB; ++i)
@@ -507,7 +559,6 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
   constexpr bool ROWS = EPI == E_ROWSCALE || EPI == E_ROWSCALE_ACC || EPI == E_ROWREV_ACC;
   float* pw = reinterpret_cast<float*>(lds);
   if ((DIFF || ROWS) && P == 1 && g.decay) {
-    __syncthreads();  // every wave has read its last fragments
     if (DIFF && t < 2 * BT) pw[t] = dpowf(d, max(0, m0 - n0 - BT + 1 + t));
     if (ROWS && t < BT) pw[t] = dpowf(d, EPI == E_ROWREV_ACC ? g.kpow - (m0 + t) : m0 + t);
     __syncthreads();
@@ -555,7 +606,7 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
     }
     return;
   }
-  // Out through LDS (free once every wave has read its last fragments), 32
+  // Out through LDS, 32
   // rows of the wave's block at a time in a region of its own, so that a lane
   // stores 16 bytes and a wave whole 256-byte pieces of rows (from the
   // accumulators' layout, 4 bytes a lane in 128-byte pieces, the 268 MB state
@@ -563,7 +614,6 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
   constexpr int EP = 32 * NB + 4, LPR = 8 * NB, RPI = 64 / LPR;  // row pitch; lanes a row; rows an access
   float* eb = reinterpret_cast<float*>(lds + 1024) + w * 32 * EP;  // past the power table
   static_assert(1024 + 4 * 32 * EP * 4 <= 2 * STAGE && 2 * BT * 4 <= 1024, "the epilogue's LDS");
-  __syncthreads();
   const int er = lane / LPR, n = nw + (lane % LPR) * 4;
   const bool quad = g.sCn == 1 && n + 4 <= N;
 #pragma unroll

@@ -94,6 +94,30 @@ def test_values_without_bf16_parts(T, N, D):
     np.testing.assert_allclose(host(out.rho)[0, 0], rho, rtol=1e-5)
 
 
+@pytest.mark.parametrize("T,N,D", [(40, 32, 24), (300, 96, 160), (600, 160, 24)])
+def test_operands_too_small_for_their_parts(oracle, T, N, D):
+    # Operands near 2^-120, whose low part ends at bf16's smallest (2^-133) and
+    # keeps 13 bits of 24: queries against large values (the state), and an
+    # output gradient (every product of the backward but the scores).
+    torch = need_gpu()
+    import burn_dragon_amd as bd
+    rng = np.random.default_rng(T)
+    small, large = np.float32(2.0 ** -120), np.float32(2.0 ** 100)
+    q = rng.standard_normal((1, 2, T, N)).astype(np.float32)
+    v = rng.standard_normal((1, 1, T, D)).astype(np.float32)
+    rho = rng.standard_normal((1, 2, N, D)).astype(np.float32)
+    g = rng.standard_normal((1, 2, T, D)).astype(np.float32) * small
+    announce("f32 split, small operands", T, N, D)
+    out = bd.try_fused_recurrent_attention(dev(torch, q * small), dev(torch, v * large))
+    grads = bd.recurrent_attention_vjp(dev(torch, g), dev(torch, q), dev(torch, v), dev(torch, rho))
+    torch.cuda.synchronize()
+    assert rel_l2(host(out.rho), oracle.recurrent_f64(q * small, v * large)[1]) <= TOL
+    ref = oracle.attention_vjp_f64(q, v, g, None, rho, safe="recurrent")
+    assert rel_l2(host(grads.grad_query), ref[0]) <= TOL
+    assert rel_l2(host(grads.grad_value), ref[1]) <= TOL
+    assert rel_l2(host(grads.grad_rho), ref[3]) <= TOL
+
+
 @pytest.mark.parametrize("T,decay", [(4200, [0.999, 0.99, 0.9999, 0.9]), (4608, None)])
 def test_groups_of_intervals(oracle, T, decay):
     # The scores of 128 streams fill a group with two intervals: nine of them
