@@ -178,7 +178,7 @@ def load_model_state(path: str, device: torch.device) -> BdhModelState:
         ptrs[i] = r.data_ptr()
         state.rho.append(r)
     st = lib.bdh_state_record_load(str(path).encode(), n.value, descs, ptrs,
-                                   _stream_ptr(device))
+                                   torch.cuda.current_stream(device).cuda_stream)
     if st != _lib.BDH_OK:
         raise _lib.BdhError(f"bdh_state_record_load: {_lib.last_error()}")
     return state

@@ -89,9 +89,9 @@ def _dtype_code(t: torch.Tensor) -> Optional[int]:
 
 
 def _stream_ptr(device: torch.device) -> int:
-    """The current stream's handle, without building a Stream object."""
-    index = device.index if device.index is not None else torch.cuda.current_device()
-    return torch._C._cuda_getCurrentRawStream(index)
+    """The current stream's handle on a CUDA tensor's device, without building
+    a Stream object."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def _on_device(*ts) -> bool:

@@ -108,3 +108,18 @@ def test_failed_load_leaves_the_destination_unchanged(tmp_path):
     torch.cuda.synchronize()
     for t, r in zip(live, rec):
         assert np.array_equal(host(t), r)
+
+
+def test_load_takes_a_device_as_torch_does(tmp_path):
+    torch = need_gpu()
+    import burn_dragon_amd as bd
+    r0 = np.random.default_rng(33).standard_normal((1, 2, 64, 32)).astype(np.float32)
+    path = tmp_path / "dev.bdh"
+    staterec.write_record(path, 5, [(r0, 1, 1)])
+    announce("state record devices")
+    for device in ("cuda", "cuda:0", 0, torch.device("cuda"), torch.device("cuda", 0)):
+        st = bd.load_model_state(path, device)
+        torch.cuda.synchronize()
+        assert np.array_equal(host(st.rho[0]), r0), device
+    with pytest.raises(ValueError):
+        bd.load_model_state(path, torch.device("cpu"))
