@@ -131,6 +131,8 @@ bdh_status scratch(hipStream_t st, int slot, size_t bytes, void** out, bool zero
 
 bool scratch_no_memory() { return t_no_memory; }
 
+bool scratch_short(bdh_status s) { return s == BDH_UNSUPPORTED || (s != BDH_OK && t_no_memory); }
+
 size_t scratch_held(hipStream_t st, int slot, void** out) {
   *out = nullptr;
   int dev = 0;

@@ -55,6 +55,9 @@ enum ScratchSlot {
 bdh_status scratch(hipStream_t st, int slot, size_t bytes, void** out, bool zero_on_alloc = false);
 // True when this thread's last scratch() found no device memory.
 bool scratch_no_memory();
+// Whether scratch() gave `s` for want of room alone (a capturing stream that
+// holds too little, or no device memory), where fewer split ranges may do.
+bool scratch_short(bdh_status s);
 // What a slot holds now, without growing it (0 bytes: nothing).
 size_t scratch_held(hipStream_t st, int slot, void** out);
 // Frees these slots' buffers (after the stream's queued work).  Not under capture.

@@ -455,6 +455,9 @@ __global__ __launch_bounds__(256) void decode_finalize_kernel(
 bool sparse_step(const DecodeArgs& a) { return a.decay == nullptr && a.rho_in != nullptr && a.rho_in == a.rho; }
 
 // Ranges per stream and rows per range.
+// Rows of each of G ranges: a multiple of 8.
+int range_rows(int64_t N, int G) { return (int)(((N + G - 1) / G + 7) / 8 * 8); }
+
 void decode_ranges(const DecodeArgs& a, int* G, int* rows) {
   if (sparse_step(a)) {
     // Double while the grid stays within one workgroup per CU and a range
@@ -471,7 +474,7 @@ void decode_ranges(const DecodeArgs& a, int* G, int* rows) {
            (ordinary ? g < DR_MAXG && a.N / (2 * g) >= 128 : g < 16 && a.N / (2 * g) >= 256))
       g *= 2;
     *G = g;
-    *rows = (int)(((a.N + g - 1) / g + 7) / 8 * 8);
+    *rows = range_rows(a.N, g);
   } else {
     *G = (int)((a.N + DD_ROWS - 1) / DD_ROWS);
     *rows = DD_ROWS;
@@ -483,17 +486,21 @@ void decode_ranges(const DecodeArgs& a, int* G, int* rows) {
 // 256-byte aligned.
 size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 
-}  // namespace
-
-size_t decode_part_bytes(const DecodeArgs& a) {
-  int G = 1, rows = 0;
-  decode_ranges(a, &G, &rows);
+size_t part_bytes(const DecodeArgs& a, int G) {
   if (G == 1) return 0;
   const int64_t S = a.B * a.H;
   size_t n = align256((size_t)(S * G * a.D) * sizeof(float));
   if (a.idx_out) n += align256((size_t)(S * a.N) * sizeof(int32_t));
   if (a.idx_out || a.cnt_out) n += align256((size_t)(S * G) * sizeof(int32_t));
   return n;
+}
+
+}  // namespace
+
+size_t decode_part_bytes(const DecodeArgs& a) {
+  int G = 1, rows = 0;
+  decode_ranges(a, &G, &rows);
+  return part_bytes(a, G);
 }
 
 bdh_status run_decode(const DecodeArgs& a, hipStream_t st, uint64_t* launches) {
@@ -524,14 +531,20 @@ bdh_status run_decode(const DecodeArgs& a, hipStream_t st, uint64_t* launches) {
   if (a.an && (!sparse || a.D % 64 != 0 || a.D > kDecodeNormMaxD || a.idx_out || a.cnt_out || a.part_buf))
     return fail(BDH_EINVAL, "a normalised readout needs the sparse step and whole rows");
   if (G > 1) {
-    const size_t need = decode_part_bytes(a);
     char* buf = (char*)a.part_buf;
     if (buf) {
-      if (a.part_bytes < need) return fail(BDH_EINVAL, "decode range buffer too small");
+      if (a.part_bytes < part_bytes(a, G)) return fail(BDH_EINVAL, "decode range buffer too small");
     } else {
       void* sp = nullptr;
-      bdh_status s = scratch(st, SLOT_DECODE_PART, need, &sp);
+      bdh_status s = scratch(st, SLOT_DECODE_PART, part_bytes(a, G), &sp);
+      while (sparse && G > 2 && scratch_short(s)) {  // capturing: the ranges that what is there holds
+        G /= 2;
+        rows = range_rows(a.N, G);
+        s = scratch(st, SLOT_DECODE_PART, part_bytes(a, G), &sp);
+      }
       if (s != BDH_OK) return s;
+      p.G = G;
+      p.rows = rows;
       buf = (char*)sp;
     }
     p.a_out = (float*)buf;

@@ -1348,8 +1348,8 @@ bdh_status run_layer(const LayerArgs& a, hipStream_t st, uint64_t* launches) {
   const bool decode = a.T == 1 && a.rho_in != nullptr && a.rho_in == a.rho_out;
   void *curb = nullptr, *xy = nullptr, *attn = nullptr, *an = nullptr, *zp = nullptr;
   // GEMM Y fused into GEMM Z (y never reaches HBM) where that is possible and faster.
-  const int ks_yz = decode ? 0 : yz_splits(M, a.H, a.T, a.N, a.D);
-  const int ks = ks_yz > 0 ? ks_yz : z_splits(M, HN, a.D);
+  int ks_yz = decode ? 0 : yz_splits(M, a.H, a.T, a.N, a.D);
+  int ks = ks_yz > 0 ? ks_yz : z_splits(M, HN, a.D);
   bdh_status s = scratch(st, SLOT_LAYER_CUR, (size_t)((M + kTilePad) * a.D) * sizeof(bf16_t), &curb);
   if (s != BDH_OK) return s;
   s = scratch(st, SLOT_LAYER_XY, (size_t)((S * a.T + kTilePad) * a.N) * sizeof(bf16_t), &xy);
@@ -1368,8 +1368,10 @@ bdh_status run_layer(const LayerArgs& a, hipStream_t st, uint64_t* launches) {
   if (s != BDH_OK) return s;
   s = scratch(st, SLOT_LAYER_AN, (size_t)((S * a.T + kTilePad) * a.D) * sizeof(bf16_t), &an);
   if (s != BDH_OK) return s;
-  s = scratch(st, SLOT_LAYER_Z, (size_t)(ks * M * a.D) * sizeof(float), &zp);
-  if (s != BDH_OK) return s;
+  while ((s = scratch(st, SLOT_LAYER_Z, (size_t)(ks * M * a.D) * sizeof(float), &zp)) != BDH_OK) {
+    if (ks_yz <= 1 || !scratch_short(s)) return s;
+    ks = ks_yz = ks_yz / 2;  // the partials that there is room for
+  }
   // A carried state whose successor is not kept still needs the state path
   // (readout of rho_in); its rho goes to scratch.
   float* rho_out = a.rho_out;

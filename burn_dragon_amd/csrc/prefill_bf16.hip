@@ -428,13 +428,21 @@ double snap_time(int64_t units, int nk, int k, double mb) {
 }
 // The fastest count of N ranges by that model; at least 8 steps a range, and
 // with `even` an even number of them.
+bool snap_ranges_ok(int nk, int k, bool even) { return nk / k >= 8 && (!even || nk % (2 * k) == 0); }
 int snap_ranges(int64_t units, int nk, double mb, bool even) {
   int best = 1;
   for (const int k : {2, 3, 4, 8}) {
-    if (nk / k < 8 || (even && nk % (2 * k) != 0)) continue;
+    if (!snap_ranges_ok(nk, k, even)) continue;
     if (snap_time(units, nk, k, mb) < snap_time(units, nk, best, mb)) best = k;
   }
   return best;
+}
+
+// The next fewer: where the stream's scratch has no room for the partials.
+int fewer_ranges(int nk, int k, bool even) {
+  do --k;
+  while (k > 1 && !snap_ranges_ok(nk, k, even));
+  return k;
 }
 
 // Two or more intervals, or one onto a large carried state: v^T, the state-carry kernel (which also
@@ -454,23 +462,26 @@ bdh_status run_carry_path(const Bf16Args& a, hipStream_t st, uint64_t* launches,
   const int ndb256 = (int)cdiv(a.D, T256);
   const int rd_pg = nb * ndb256;
   const int64_t upg = (int64_t)nb * (nb + 1) / 2;
-  const int ks = snap_ranges(S * n_iv * (upg + rd_pg), nk,
+  int ks = snap_ranges(S * n_iv * (upg + rd_pg), nk,
                              ((double)S * n_iv * upg * T256 * T256 + (double)S * a.T * a.D) * 4e-6, false);
-  const int kr = ks;
 
   void *vt = nullptr, *part = nullptr, *snap = nullptr, *rdp = nullptr, *q = nullptr;
   bdh_status stt = scratch(st, SLOT_VT, (size_t)(a.B * a.Hv * Dp * Tp) * sizeof(bf16_t), &vt);
   if (stt != BDH_OK) return stt;
-  stt = scratch(st, SLOT_SCORES, (size_t)(ks * S * n_iv * Lp * Lp) * sizeof(float), &part);
-  if (stt != BDH_OK) return stt;
   stt = scratch(st, SLOT_SNAP, (size_t)(n_iv * S * a.D * a.N) * sizeof(bf16_t), &snap);
-  if (stt != BDH_OK) return stt;
-  stt = scratch(st, SLOT_READOUT, (size_t)(kr * S * a.T * a.D) * sizeof(float), &rdp);
   if (stt != BDH_OK) return stt;
   if (rope) {
     stt = scratch(st, SLOT_ROTATED, (size_t)(S * a.T * a.N) * sizeof(bf16_t), &q);
     if (stt != BDH_OK) return stt;
   }
+  for (;;) {
+    stt = scratch(st, SLOT_SCORES, (size_t)(ks * S * n_iv * Lp * Lp) * sizeof(float), &part);
+    if (stt == BDH_OK) stt = scratch(st, SLOT_READOUT, (size_t)(ks * S * a.T * a.D) * sizeof(float), &rdp);
+    if (stt == BDH_OK) break;
+    if (ks == 1 || !scratch_short(stt)) return stt;
+    ks = fewer_ranges(nk, ks, false);
+  }
+  const int kr = ks;
 
   hipLaunchKernelGGL(transpose_v_kernel, dim3(cdiv(Tp, VT_TILE), cdiv(Dp, VT_TILE), (unsigned)(a.B * a.Hv)),
                      dim3(256), 0, st, a.v, (bf16_t*)vt, a.T, a.D, Tp, Dp);
@@ -537,14 +548,16 @@ bdh_status run_gram_path(const Bf16Args& a, hipStream_t st, uint64_t* launches, 
                          int64_t Dp, int64_t Lp, int nb, int nk) {
   const int64_t L = a.L;
   const int64_t upg = (int64_t)nb * (nb + 1) / 2;
-  const int ks = snap_ranges(S * upg, nk, (double)S * upg * T256 * T256 * (a.part16 ? 2e-6 : 4e-6), true);
+  int ks = snap_ranges(S * upg, nk, (double)S * upg * T256 * T256 * (a.part16 ? 2e-6 : 4e-6), true);
 
   void *vt = nullptr, *part = nullptr;
   bdh_status stt = scratch(st, SLOT_VT, (size_t)(a.B * a.Hv * Dp * Tp) * sizeof(bf16_t), &vt);
   if (stt != BDH_OK) return stt;
   const size_t pbytes = a.part16 ? sizeof(bf16_t) : sizeof(float);
-  stt = scratch(st, SLOT_SCORES, (size_t)(ks * S * Lp * Lp) * pbytes, &part);
-  if (stt != BDH_OK) return stt;
+  while ((stt = scratch(st, SLOT_SCORES, (size_t)(ks * S * Lp * Lp) * pbytes, &part)) != BDH_OK) {
+    if (ks == 1 || !scratch_short(stt)) return stt;
+    ks = fewer_ranges(nk, ks, true);
+  }
 
   hipLaunchKernelGGL(transpose_v_kernel, dim3(cdiv(Tp, VT_TILE), cdiv(Dp, VT_TILE), (unsigned)(a.B * a.Hv)),
                      dim3(256), 0, st, a.v, (bf16_t*)vt, a.T, a.D, Tp, Dp);
@@ -738,8 +751,6 @@ bdh_status run_bf16_path(const Bf16Args& a, hipStream_t st, uint64_t* launches) 
   void *vt = nullptr, *part = nullptr, *rdp = nullptr, *rho_a = nullptr, *rho_b = nullptr;
   bdh_status stt = scratch(st, SLOT_VT, (size_t)(a.B * a.Hv * Dp * Tp) * sizeof(bf16_t), &vt);
   if (stt != BDH_OK) return stt;
-  stt = scratch(st, SLOT_SCORES, (size_t)(ks * S * n_iv * Lp * Lp) * sizeof(float), &part);
-  if (stt != BDH_OK) return stt;
   // With two or more intervals every launch would re-rotate its x tiles;
   // rotating x once (one read and one write of x) lets every launch run the
   // rotation-free units instead.
@@ -762,6 +773,10 @@ bdh_status run_bf16_path(const Bf16Args& a, hipStream_t st, uint64_t* launches) 
       stt = scratch(st, SLOT_RHO_B, (size_t)(S * a.N * a.D) * sizeof(float), &rho_b);
       if (stt != BDH_OK) return stt;
     }
+  }
+  while ((stt = scratch(st, SLOT_SCORES, (size_t)(ks * S * n_iv * Lp * Lp) * sizeof(float), &part)) != BDH_OK) {
+    if (ks == 1 || !scratch_short(stt)) return stt;
+    ks /= 2;
   }
   const bool rope = a.freqs != nullptr && !prerot;
 

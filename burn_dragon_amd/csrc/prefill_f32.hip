@@ -109,6 +109,10 @@ bdh_status f32_path_buffers(F32Args* a, hipStream_t st) {
     } else if (a->state && v.L > kShortInterval) {
       a->max_len = kShortInterval;
       a->max_group = 1;
+    } else if (scores && (states || !need.states)) {  // no room for partials alone: unsplit
+      a->part = nullptr;
+      a->part_elems = 0;
+      return BDH_OK;
     } else {
       return s;
     }

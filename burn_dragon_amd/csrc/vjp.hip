@@ -27,6 +27,8 @@
 // so transposed operands need no copy.  The decay gradient's terms are summed
 // in f64 by tile or block into slots of their own, then per head in a fixed
 // order: the result is deterministic.
+#include <algorithm>
+
 #include "bdh_gemm_f32.h"
 
 namespace bdh {
@@ -214,7 +216,10 @@ bdh_status run_attention_vjp(const VjpArgs& a, hipStream_t st, uint64_t* launche
   const int t_slots = n_iv > 1 ? (int)gf32::tile_count((int)Lv, (int)Lv, 64, true) : gf32::sym_slots(S, (int)Lv);
   const int st_slots = a.rho0 || n_iv > 1 ? kStateBlocks : 0;
   const int slots = t_slots + st_slots + (n_iv > 1 ? kCrossBlocks : 0);
-  s = scratch(st, SLOT_VJP_PART, (size_t)(S * slots) * sizeof(double), &ppart);
+  // (Room for any call of as many streams, so that a capture never finds less
+  // than a longer or shorter eager call took.)
+  const int64_t most = gf32::tile_count(kVjpInterval, kVjpInterval, 64, true) + kStateBlocks + kCrossBlocks;
+  s = scratch(st, SLOT_VJP_PART, (size_t)(S * most) * sizeof(double), &ppart);
   if (s != BDH_OK) return s;
   if (n_iv > 1) {
     // states at the interval starts 1 .. n_iv - 1, and two Gamma buffers
@@ -233,6 +238,10 @@ bdh_status run_attention_vjp(const VjpArgs& a, hipStream_t st, uint64_t* launche
   if (pe) {
     void* pp = nullptr;
     s = scratch(st, SLOT_GEMM_PART, pe * sizeof(float), &pp);
+    if (scratch_short(s)) {  // fewer ranges, or none
+      pe = std::min(pe, scratch_held(st, SLOT_GEMM_PART, &pp) / sizeof(float));
+      s = BDH_OK;
+    }
     if (s != BDH_OK) return s;
     part = (float*)pp;
   }
