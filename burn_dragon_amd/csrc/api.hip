@@ -745,9 +745,8 @@ bdh_status bdh_lm_logits(const float* hidden, int64_t rows, int64_t embd,
   if ((rows + 255) / 256 * ((vocab + 127) / 128) > ((int64_t)1 << 31) - 1)
     return fail(BDH_UNSUPPORTED, "too large for one launch");
   bdh_status st = lm_logits(hidden, rows, embd, (const bf16_t*)lm_head_packed, vocab, logits,
-                            (hipStream_t)stream);
+                            (hipStream_t)stream, &prof.launches);
   if (st != BDH_OK) return st;
-  prof.launches = 2;
   prof.done(true);
   return BDH_OK;
 }

@@ -160,7 +160,7 @@ bdh_status embed_norm(const int32_t* tokens, int64_t n, const float* embed, int6
                       int64_t D, float* out, hipStream_t st);
 bdh_status pack_lm_head(int64_t D, int64_t V, const float* head, bf16_t* packed, hipStream_t st);
 bdh_status lm_logits(const float* hidden, int64_t M, int64_t D, const bf16_t* head, int64_t V,
-                     float* logits, hipStream_t st);
+                     float* logits, hipStream_t st, uint64_t* launches);
 
 // --- decode (decode.hip) ------------------------------------------------------
 // One token per stream (T = 1).  rho_in == rho (not null) and no decay:

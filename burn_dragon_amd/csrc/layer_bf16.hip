@@ -1318,7 +1318,7 @@ bdh_status pack_lm_head(int64_t D, int64_t V, const float* head, bf16_t* packed,
 }
 
 bdh_status lm_logits(const float* hidden, int64_t M, int64_t D, const bf16_t* head, int64_t V,
-                     float* logits, hipStream_t st) {
+                     float* logits, hipStream_t st, uint64_t* launches) {
   void* hb = nullptr;
   if (M > SK_MAXM) {
     const bdh_status s = scratch(st, SLOT_LAYER_CUR, (size_t)(M * D) * sizeof(bf16_t), &hb);
@@ -1337,6 +1337,7 @@ bdh_status lm_logits(const float* hidden, int64_t M, int64_t D, const bf16_t* he
   g.ct = (int)cdiv(V, T256 / 2);
   g.ks = 1;
   BDH_HIP_TRY(launch_gemm<G_L>(g, st));
+  *launches += M > SK_MAXM ? 2 : 1;
   return BDH_OK;
 }
 

@@ -166,3 +166,29 @@ def test_kernel_timing_records_the_dominant_kernels():
     bd.try_fused_recurrent_attention_rope(x, v, position=0)
     torch.cuda.synchronize()
     assert got(_lib.BDH_KERNEL_PREFILL) == (0.0, 0)
+
+
+@pytest.mark.parametrize("rows,launches", [(1, 1), (64, 1), (65, 2)])
+def test_logits_launches(rows, launches):
+    # Up to 64 rows the product rounds the f32 rows itself; beyond, a launch does.
+    torch = need_gpu()
+    import burn_dragon_amd as bd
+    from burn_dragon_amd import _lib
+    lib = _lib.load()
+    D, V = 64, 130
+    hidden, head = torch.randn(rows, D, device="cuda"), torch.randn(D, V, device="cuda")
+    packed = torch.empty(V, D, device="cuda", dtype=torch.bfloat16)
+    out = torch.empty(rows, V, device="cuda")
+    announce("logits launches", rows)
+    stream = torch.cuda.current_stream().cuda_stream
+    assert lib.bdh_lm_head_pack(D, V, head.data_ptr(), packed.data_ptr(), stream) == _lib.BDH_OK
+    bd.recurrent_profile_enable(True)
+    bd.recurrent_profile_reset()
+    try:
+        assert lib.bdh_lm_logits(hidden.data_ptr(), rows, D, packed.data_ptr(), V, out.data_ptr(), stream) == _lib.BDH_OK
+        assert bd.recurrent_profile_snapshot().launches == launches
+    finally:
+        bd.recurrent_profile_enable(False)
+    torch.cuda.synchronize()
+    want = hidden.bfloat16().double() @ head.bfloat16().double()
+    assert rel_l2(host(out), want.cpu().numpy()) <= 1e-6  # f32 sums of 64 products of bf16 values
