@@ -5,7 +5,7 @@ step, and in graph replays with other work between them."""
 import numpy as np
 import pytest
 
-from tests.gpu_util import announce, dev, need_gpu
+from tests.gpu_util import TOL_F32, announce, dev, host, need_gpu, rel_l2
 
 pytestmark = pytest.mark.gpu
 
@@ -26,12 +26,18 @@ def _inputs(torch, B, H, N, D, seed):
     (1, 2, 4096, 600),   # three column blocks
     (32, 4, 1024, 64),   # 2 ranges on 128 streams, the most that are split: likewise
 ])
-def test_combined_readout_is_the_finalized_one(B, H, N, D):
+def test_combined_readout_is_the_finalized_one(oracle, B, H, N, D):
+    # (Where both forms end in the finalize launch, the oracle's step is the other side.)
     torch = need_gpu()
     import burn_dragon_amd as bd
     announce("decode combine", B, H, N, D)
     x, v, rho = _inputs(torch, B, H, N, D, N)
     r1, r2 = rho.clone(), rho.clone()
+    rho_ref = host(rho)
+    a_ref, _, _ = oracle.decode_step_f32(host(x), host(v), rho_ref, 3)
+    r3 = rho.clone()
+    assert rel_l2(host(bd.decode_step(x, v, r3, position=3).readout), a_ref) <= TOL_F32
+    assert rel_l2(host(r3), rho_ref) <= TOL_F32
     for step in range(6):
         a = bd.decode_step(x, v, r1, position=step).readout
         b = bd.decode_step(x, v, r2, position=step, want_active=True).readout
