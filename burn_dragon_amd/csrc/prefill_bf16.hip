@@ -682,13 +682,23 @@ bdh_status run_bf16_path(const Bf16Args& a, hipStream_t st, uint64_t* launches) 
   // One interval with a carried state takes the state-carry form (which reads
   // rho once, for its snapshot and its successor) where its gram has more than
   // one block of 256 tokens, its columns fill the carry kernel's 256-column
-  // block and x has 48 M elements: B8 nh4 T300 N8192 D256 418 -> 380 us, T512
-  // 494 -> 467, B24 T512 N2048 438 -> 374, B3 T512 N8192 205 -> 201.  Elsewhere
-  // its extra launches and the q stream cost more: B8 T400 N2048 (25 M) 138
-  // against 144 us, B8 T256 N8192 310 against 334, B16 T512 N4096 D64 378
-  // against 396, B16 T400 N4096 D128 with decay 330 against 392.
-  const bool carried1 =
-      a.rho_in != nullptr && a.T > T256 && a.D > T256 / 2 && S * a.T * a.N >= ((int64_t)48 << 20);
+  // block and x has 48 M elements.  Both routes were measured over 320 shapes
+  // (B 1-16 nh4, T 200-512, N 2048-8192, D 64-256).  In place, where the other
+  // form takes a second launch for the state, that is 11-38 % faster.  Out of
+  // place the carry kernel's own work on x weighs more, with the tokens where
+  // the other form's 256-token tiles do not: it writes q with RoPE (B8 T257
+  // N8192 D256 417 -> 378 us, B3 T512 224 -> 202, but B8 T400 N4096 D192 225 ->
+  // 234), and scales its rows with decay (B16 T257 N6144 D192 529 -> 508, but
+  // B8 T257 256 -> 291), so longer sequences of many streams, and with decay
+  // wider values, need more elements.  The slower form is chosen by 4 % at most
+  // (6 % for one shape of N 2048; with few streams, whose x and rho stay in the
+  // Infinity Cache where a call is repeated on them, by 7 % in such a loop).
+  const int64_t x_m = S * a.T * a.N >> 20;
+  bool carried1 = a.rho_in != nullptr && a.T > T256 && a.D > T256 / 2 && x_m >= 48;
+  if (carried1 && a.rho_out != a.rho_in) {
+    if (a.decay != nullptr) carried1 = a.T > 400 ? x_m >= 72 || S > 16 : a.D <= 192 && x_m >= 72;
+    else if (a.freqs != nullptr && a.T > 320) carried1 = x_m >= 56 || S <= 16;
+  }
   if (a.state && (n_iv >= 2 || carried1) && a.D * a.N * 2 < ((int64_t)1 << 31) &&
       (size_t)(n_iv * S * a.N * a.D) * sizeof(bf16_t) <= kCarrySnapMax) {
     const bdh_status r = run_carry_path(a, st, launches, S, Tp, Dp, n_iv, Lp, nb, nk);
