@@ -49,7 +49,6 @@ namespace gf32 {
 
 enum Epi {
   E_STORE = 0,     // C = acc
-  E_TRIL,          // C = n < m ? acc : 0
   E_TRIL_DECAY,    // C = n < m ? acc * d^(m-n) : 0
   E_ROWSCALE,      // C = acc * d^m
   E_ROWSCALE_ACC,  // C += acc * d^m
@@ -133,7 +132,6 @@ __device__ __forceinline__ const float* epi_addend(const GemmF32& g, int64_t c0)
 // (when the kind has one).
 template <int EPI, class Pow>
 __device__ __forceinline__ float epi_value(const GemmF32& g, Pow&& power, float carry, int m, int n, float v, float x) {
-  if (EPI == E_TRIL) v = n < m ? v : 0.0f;
   if (EPI == E_TRIL_DECAY) v = n < m ? (g.decay ? v * power(m, n) : v) : 0.0f;
   if ((EPI == E_ROWSCALE || EPI == E_ROWSCALE_ACC || EPI == E_ROWREV_ACC) && g.decay) v *= power(m, n);
   if (EPI == E_ROWSCALE_ACC || EPI == E_ROWREV_ACC) v += x;
@@ -788,7 +786,7 @@ hipError_t gemm(GemmF32 g, int64_t batch, hipStream_t st, float* part = nullptr,
   g.batch = batch;
   if (g.niv > 1) batch *= g.niv;
   if (batch > kMaxBatch) return hipErrorInvalidValue;
-  g.tri = (EPI == E_TRIL || EPI == E_TRIL_DECAY || EPI == E_SYM_DECAY) && g.M == g.N;
+  g.tri = (EPI == E_TRIL_DECAY || EPI == E_SYM_DECAY) && g.M == g.N;
   if (EPI == E_SYM_DECAY && (!g.tri || part)) return hipErrorInvalidValue;
   const size_t per = (size_t)batch * (size_t)g.M * (size_t)g.N;
   const int64_t tiles = tile_count(g.M, g.N, 128, g.tri) * batch;

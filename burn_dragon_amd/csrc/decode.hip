@@ -8,9 +8,9 @@
 // Sparse step (rho updated in place, no decay): only the rows in A change,
 // so only they are read and written.  G workgroups per (batch, head) stream
 // (1024 threads, 512 for ranges of up to 256 rows) each own a range of N / G
-// rows (G grows while the grid stays within one workgroup per CU).  A workgroup compacts its range's active rows
-// (8 rows per thread, wavefront prefix scan, workgroup offsets through LDS)
-// into an LDS list (ascending), then its waves stream exactly those rho
+// rows (G grows while the grid stays within one workgroup per CU).  A workgroup
+// compacts its range's active rows (8 rows per thread, wavefront prefix scan,
+// workgroup offsets through LDS) into an LDS list (ascending), then its waves stream exactly those rho
 // rows: a whole 1 KiB row per wave per load at D = 256 (float4 per lane), 8
 // rows in flight per wave.
 //
@@ -23,10 +23,11 @@
 //
 // Readouts are reduced across waves in LDS in a fixed order; with G > 1 the
 // range partials go to a range buffer, and the last of a stream's workgroups
-// to finish sums them in range order, so the result is deterministic.  Where
-// streams have at most 4 ranges (and no LayerNorm follows), the active lists are asked for, the step is dense, or the buffers are a
-// caller's (which overlapping calls may share), a finalize kernel sums the
-// partials (and concatenates the lists) instead.  At C3's shape with B = 1
+// to finish sums them in range order, so the result is deterministic.  A
+// finalize kernel sums the partials (and concatenates the lists) instead where
+// streams have at most 4 ranges (and no LayerNorm follows), where the active
+// lists are asked for, in the dense step, and in a caller's buffers (which
+// overlapping calls may share).  At C3's shape with B = 1
 // (4 streams of 32 ranges) a kernel of 8.1 us and a finalize launch of 4.4 are
 // one of 11.2.
 #include <type_traits>

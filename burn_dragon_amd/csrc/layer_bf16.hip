@@ -566,16 +566,16 @@ __global__ __launch_bounds__(64 * (XR_MW + XR_DW + XR_SW), 1) void layer_x_roles
 // CU) owns a 128-token tile of one sequence (the last one's missing rows are
 // fetched and multiplied, not stored) and a
 // range of 128-latent chunks of H N, and per chunk
-//   Y^T  = Ev_chunk a_h^T        [128 latents x 256 tokens], K = D
+//   Y^T  = Ev_chunk a_h^T        [128 latents x 128 tokens], K = D
 //   y    = act(Y) * x            bf16, into LDS as the next product's A operand
-//   z   += y Dec_chunk^T         [256 tokens x D], K = 128
+//   z   += y Dec_chunk^T         [128 tokens x D], K = 128
 // with z in the accumulators across the chunks, written at the end as the
 // split-K partial [kp, M, D] that the residual kernel sums in order.  Y is
 // computed transposed so that each accumulator register of a lane holds 4
 // consecutive latents of one token: one 8-byte read of x and one 8-byte
 // write of y.  y is rounded to bf16 exactly as GEMM Y stores it.
 // Operands stream through a 3-slot direct-load ring two steps ahead (a step
-// is 32 deep: a Y step loads 256 a_h rows and 128 Ev rows, a z step 256
+// is 32 deep: a Y step loads 128 a_h rows and 128 Ev rows, a z step 256
 // decoder rows); x lands in the y buffer itself, in pairs of 32-latent
 // blocks as soon as the previous chunk's z steps have read them.  (A 4-slot ring, three
 // steps ahead in all 160 KiB of LDS, was slower: C5 1.08 against 0.98 ms
@@ -850,9 +850,10 @@ constexpr int SK_CHUNK = 8;  // 32-deep steps loaded at once per wave
 
 // MB = 16-row blocks: 1, 2 or 4.  F32 (X, logits): the rows are f32 and
 // rounded here, as to_bf16_kernel does, where that would be a launch for this
-// product alone (the decode step and the logits); its loads are half as many
-// steps deep, so X of a B1 T47 prompt, whose attention needs the bf16 rows
-// anyway, takes 12.2 us from those and 14.4 from the f32 ones.
+// product alone (the decode step and the logits); its loads are
+// SK_CHUNK / MB steps deep (the f32 rows take the registers), so X of a B1 T47
+// prompt (MB = 4, two steps), whose attention needs the bf16 rows anyway, takes
+// 12.2 us from those and 14.4 from the f32 ones.
 template <int KIND, int MB, bool F32>
 __global__ __launch_bounds__(256) void skinny_gemm_kernel(LayerGemmArgs g) {
   // X, Y (K = D, H N columns): each wave owns a 16-column block and all of
@@ -1117,10 +1118,13 @@ hipError_t launch_skinny(const LayerGemmArgs& g, hipStream_t st) {
 template <int KIND>
 hipError_t launch_gemm(const LayerGemmArgs& g, hipStream_t st) {
   if (g.M <= SK_MAXM) {
-    if constexpr (KIND == G_L) return launch_skinny<KIND, true>(g, st);
-    if constexpr (KIND == G_X)
-      if (g.af) return launch_skinny<KIND, true>(g, st);
-    return launch_skinny<KIND, false>(g, st);
+    if constexpr (KIND == G_L) {
+      return launch_skinny<KIND, true>(g, st);
+    } else {
+      if constexpr (KIND == G_X)
+        if (g.af) return launch_skinny<KIND, true>(g, st);
+      return launch_skinny<KIND, false>(g, st);
+    }
   }
   const int64_t total = (int64_t)g.mt * g.ct * (KIND == G_Z ? g.ks : 1);
   const int64_t slots = 2 * (int64_t)device_cus();  // two workgroups per CU
