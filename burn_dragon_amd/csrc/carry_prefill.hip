@@ -27,6 +27,8 @@
 // the rotation's VALU and LDS work.  The loading waves issue loads only, so
 // their waits can count DMAs in flight (loads complete in order; a store
 // issued later may complete before them).
+#include <type_traits>
+
 #include "bdh_mfma.h"
 
 namespace bdh {
@@ -64,7 +66,7 @@ __device__ __forceinline__ void lds_dma_wait_barrier() {
 __device__ __forceinline__ void plain_barrier() { asm volatile("s_barrier" ::: "memory"); }
 
 // The loading waves (rw = wave - 4).
-template <bool ROPE, bool QOUT, bool DECAY>
+template <bool ROPE, bool QOUT, bool DECAY, bool DIRECT>
 __device__ __forceinline__ void carry_loader(const CarryArgs& a, char* lds, int64_t s, int64_t n0, int64_t d0,
                                              int rw, int lane) {
   const int rtid = rw * 64 + lane;
@@ -115,11 +117,11 @@ __device__ __forceinline__ void carry_loader(const CarryArgs& a, char* lds, int6
   // (cos, sin) of the lane's 4 pairs at its two tokens of the step rotated
   // next: from frac(pos f) for step 0 (positions clamped to T - 1 as the
   // rows are), then advanced by e(32 f) a step, one complex multiply a pair
-  // instead of a phase, a cosine and a sine (the steps run in order).  A call
-  // of one interval computes every step's words from their phases, as the
+  // instead of a phase, a cosine and a sine (the steps run in order).  DIRECT,
+  // a call of one interval: every step's words come from their phases, as the
   // state units of a call without a carried state do: a sequence split in
-  // such calls then carries the state of the whole.
-  const bool direct = a.T <= a.L;
+  // such calls then carries the state of the whole.  (As a template: a branch
+  // in the loop cost the calls of several intervals 0.5-2 %.)
   float ca[4], sa[4], cb[4], sb[4], ec[4], es[4];
   if (ROPE) {
     const int64_t ta = 2 * tp < a.T ? 2 * tp : a.T - 1, tb = 2 * tp + 1 < a.T ? 2 * tp + 1 : a.T - 1;
@@ -168,7 +170,7 @@ __device__ __forceinline__ void carry_loader(const CarryArgs& a, char* lds, int6
       const float pn = (float)(a.fixed ? a.pos0 : a.pos0 + t + BK);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        if (direct) {
+        if (DIRECT) {
           const float fa = rope_frac(pn, fq[j]), fb = rope_frac(a.fixed ? pn : pn + 1.0f, fq[j]);
           ca[j] = __builtin_amdgcn_cosf(fa);
           sa[j] = __builtin_amdgcn_sinf(fa);
@@ -348,14 +350,14 @@ __device__ __forceinline__ void carry_mma(const CarryArgs& a, char* lds, int64_t
   });
 }
 
-template <bool ROPE, bool QOUT, bool DECAY>
+template <bool ROPE, bool QOUT, bool DECAY, bool DIRECT>
 __device__ __forceinline__ void carry_unit(const CarryArgs& a, char* lds, int64_t s, int64_t n0, int64_t d0) {
   const int lane = threadIdx.x & 63, w = wave_id();
-  if (w >= 4) carry_loader<ROPE, QOUT, DECAY>(a, lds, s, n0, d0, w - 4, lane);
+  if (w >= 4) carry_loader<ROPE, QOUT, DECAY, DIRECT>(a, lds, s, n0, d0, w - 4, lane);
   else carry_mma<QOUT, DECAY>(a, lds, s, n0, d0, w, lane);
 }
 
-template <bool ROPE, bool DECAY>
+template <bool ROPE, bool DECAY, bool DIRECT>
 __global__ __launch_bounds__(CARRY_NT, 1) void prefill_carry_kernel(CarryArgs a) {
   __shared__ __attribute__((aligned(16))) char lds[CARRY_LDS];
   const int nt = (int)(a.N / CARRY_N);
@@ -369,8 +371,8 @@ __global__ __launch_bounds__(CARRY_NT, 1) void prefill_carry_kernel(CarryArgs a)
   const int64_t s = u / (nt * dt);
   const int rem = u - (int)s * nt * dt;
   const int64_t n0 = (int64_t)(rem / dt) * CARRY_N, d0 = (int64_t)(rem % dt) * T256;
-  if (ROPE && d0 == 0) carry_unit<ROPE, true, DECAY>(a, lds, s, n0, d0);
-  else carry_unit<ROPE, false, DECAY>(a, lds, s, n0, d0);
+  if (ROPE && d0 == 0) carry_unit<ROPE, true, DECAY, DIRECT>(a, lds, s, n0, d0);
+  else carry_unit<ROPE, false, DECAY, DIRECT>(a, lds, s, n0, d0);
 }
 
 }  // namespace
@@ -379,13 +381,15 @@ int prefill_carry_units(int64_t S, int64_t N, int64_t Dp) { return (int)(S * (N 
 
 hipError_t launch_prefill_carry(const CarryArgs& a, hipStream_t st) {
   const unsigned grid = (unsigned)prefill_carry_units(a.S, a.N, a.Dp);
-  if (a.decay) {
-    if (a.freqs) hipLaunchKernelGGL((prefill_carry_kernel<true, true>), dim3(grid), dim3(CARRY_NT), 0, st, a);
-    else hipLaunchKernelGGL((prefill_carry_kernel<false, true>), dim3(grid), dim3(CARRY_NT), 0, st, a);
-  } else {
-    if (a.freqs) hipLaunchKernelGGL((prefill_carry_kernel<true, false>), dim3(grid), dim3(CARRY_NT), 0, st, a);
-    else hipLaunchKernelGGL((prefill_carry_kernel<false, false>), dim3(grid), dim3(CARRY_NT), 0, st, a);
-  }
+  auto launch = [&](auto decay) {
+    constexpr bool DECAY = decltype(decay)::value;
+    const dim3 blk(CARRY_NT);
+    if (!a.freqs) hipLaunchKernelGGL((prefill_carry_kernel<false, DECAY, false>), dim3(grid), blk, 0, st, a);
+    else if (a.T <= a.L) hipLaunchKernelGGL((prefill_carry_kernel<true, DECAY, true>), dim3(grid), blk, 0, st, a);
+    else hipLaunchKernelGGL((prefill_carry_kernel<true, DECAY, false>), dim3(grid), blk, 0, st, a);
+  };
+  if (a.decay) launch(std::true_type{});
+  else launch(std::false_type{});
   return hipGetLastError();
 }
 
