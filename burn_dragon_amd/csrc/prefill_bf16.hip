@@ -697,7 +697,7 @@ bdh_status run_bf16_path(const Bf16Args& a, hipStream_t st, uint64_t* launches) 
   bool carried1 = a.rho_in != nullptr && a.T > T256 && a.D > T256 / 2 && x_m >= 48;
   if (carried1 && a.rho_out != a.rho_in) {
     if (a.decay != nullptr) carried1 = a.T > 400 ? x_m >= 72 || S > 16 : a.D <= 192 && x_m >= 72;
-    else if (a.freqs != nullptr && a.T > 320) carried1 = x_m >= 56 || S <= 16;
+    else if (a.freqs != nullptr && a.T > 320) carried1 = x_m >= 56 || S <= 24;
   }
   if (a.state && (n_iv >= 2 || carried1) && a.D * a.N * 2 < ((int64_t)1 << 31) &&
       (size_t)(n_iv * S * a.N * a.D) * sizeof(bf16_t) <= kCarrySnapMax) {

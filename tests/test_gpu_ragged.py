@@ -79,7 +79,7 @@ def test_layer_tiles_match_oracle(oracle, B, H, T, N, D, carried, yz):
     (2, 390, 8192, 64, None, [0.99, 0.98, 0.97, 0.96], False, False),
     (8, 390, 4096, 192, 5, None, False, False),                  # many, out of place: not enough beyond 320 tokens
     (8, 310, 5120, 192, 5, None, False, True),                   # enough below: the state-carry form
-    (4, 390, 8192, 192, 5, None, False, True),                   # of 16 streams
+    (6, 390, 5632, 192, 5, None, False, True),                   # of 24 streams
     (4, 390, 8192, 192, 5, None, True, True),                    # in place
     (4, 390, 8192, 192, None, None, False, True),                # no rotation
     (4, 390, 8192, 192, None, [0.99, 0.98, 0.97, 0.96], False, False),
