@@ -37,6 +37,13 @@
 // bits could show (kLost), computes its block again with the fp32 MFMA.  (What
 // stays lost: an operand below 2^-134 has no parts, so a sum of products of
 // such operands alone is 0.)
+// A product with an operand scaled by decay powers multiplies both operands by
+// 2^16 instead, which keeps the last part of every fp32 number above bf16's
+// smallest: its sums may be as small as the decay makes them.  (Looked at as
+// the others, they sent the state of neurons silent while a strong decay
+// forgets them to the fp32 MFMA: B1 nh4 T4096 N8192 D128, 1 % active, ALiBi
+// decays from 0.78, 3095 us against 1180.  The factor in every product took the
+// f32 C2 shape from 1.04 to 1.11 ms: one more instruction for two values.)
 #pragma once
 
 #include <type_traits>
@@ -98,6 +105,7 @@ constexpr int DSCALE = 1024;         // KSCALE: most k of one workgroup (LDS tab
 // to sqrt(K) 2^-134 of the largest operand (2^-127.5 at K = 8192), and that
 // has to stay below its own 2^-24.
 constexpr float kLost = 0x1p-104f;
+constexpr float kUp = 0x1p16f;  // KSCALE: the operands' factor
 
 __device__ __forceinline__ float dpowf(float d, int e) { return powf(d, (float)e); }
 
@@ -335,9 +343,9 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
   constexpr bool SNAP = EPI == E_CARRY_SNAP;
   if (KSCALE) {
     if (SNAP) {
-      for (int k = t; k <= g.len; k += 256) sct[k] = dpowf(d, k);
+      for (int k = t; k <= g.len; k += 256) sct[k] = dpowf(d, k) * kUp;
     } else {
-      for (int k = t; k < (nks + 2) * GK; k += 256) sct[k] = k < Kt ? dpowf(d, g.kpow - (k_lo + k)) : 0.0f;
+      for (int k = t; k < (nks + 2) * GK; k += 256) sct[k] = k < Kt ? dpowf(d, g.kpow - (k_lo + k)) * kUp : 0.0f;
     }
     __syncthreads();
   }
@@ -371,10 +379,14 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
       for (int e = 0; e < E; ++e) mx = fmaxf(fmaxf(mx, fabsf(a[e])), fabsf(bv[e]));
       asm volatile("" : "+v"(mx));  // here, not where copies of the values would have to live to
     };
-    if (!(AKC && BKC)) largest();
+    if (KSCALE) {
+#pragma unroll
+      for (int e = 0; e < E; ++e) bv[e] *= kUp;
+    }
+    if (!KSCALE && !(AKC && BKC)) largest();
     split_store(o, la, a);
     split_store(o + 3 * PA, lb, bv);
-    if (AKC && BKC) largest();
+    if (!KSCALE && AKC && BKC) largest();
   };
 
   floatx16 big[NB][NB], small[NB][NB];
@@ -422,8 +434,9 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
   uint32_t least = ~0u;
   auto look = [&](float v, float& nan) {
     nan = fmaf(v, 0.0f, nan);
-    least = min(least, (__builtin_bit_cast(uint32_t, v) << 1) - 1);
+    if (!KSCALE) least = min(least, (__builtin_bit_cast(uint32_t, v) << 1) - 1);
   };
+  float down = KSCALE ? 1.0f / (kUp * kUp) : 1.0f;
   auto snapshot = [&](int i) {
     float* o = g.snap + i * g.sSnap + c0;
     // (The block's addresses are not kept through the step loop: 64 of them
@@ -446,8 +459,9 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
         }
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const float v = big[i2][j][r] + small[i2][j][r];
+          float v = big[i2][j][r] + small[i2][j][r];
           look(v, nan);
+          if (KSCALE) v *= down;
           if (mo + 32 * i2 + acc_row(0, r) < M && n < N)
             o[off + acc_row(0, r) * g.sCm] = X != nullptr ? v + x[r] * dl : v;
         }
@@ -504,13 +518,14 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
         big[i][j][r] += small[i][j][r];
         small[i][j][r] = 0.0f;
         look(big[i][j][r], nan);
+        if (KSCALE) big[i][j][r] *= down;
       }
   bad |= nan != 0.0f;
   // A sum below kLost of the largest operand of the workgroup asks for the
   // block again; the largest operand is looked for where one is above kLarge
   // or a sum below its share.
   constexpr float kLarge = 0x1p40f;
-  const bool ask = __any(mx >= kLarge || least < (__builtin_bit_cast(uint32_t, kLarge * kLost) << 1) - 1);
+  const bool ask = !KSCALE && __any(mx >= kLarge || least < (__builtin_bit_cast(uint32_t, kLarge * kLost) << 1) - 1);
   if (lane == 0) wask[w] = ask;
   __syncthreads();  // also: every wave has read its last fragments
   if (wask[0] || wask[1] || wask[2] || wask[3]) {
@@ -524,6 +539,7 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
   if (__any(bad)) {
     // The block again on v_mfma_f32_32x32x2_f32, straight from memory.
     if (SNAP) X = epi_addend<EPI>(g, c0);
+    down = 1.0f;
 #pragma unroll
     for (int i = 0; i < NB; ++i)
 #pragma unroll
@@ -536,7 +552,7 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmF32 g, int ntx, 
 #pragma unroll
       for (int i = 0; i < NB; ++i) {
         av[i] = A0[(int64_t)min(mw + 32 * i + (lane & 31), M - 1) * g.sAm + (int64_t)ka * g.sAk];
-        if (KSCALE) av[i] *= sct[SNAP ? max(0, len_of(i0) - (kk - i0 * g.len)) : min(kk, Kt - 1)];
+        if (KSCALE) av[i] *= dpowf(d, SNAP ? max(0, len_of(i0) - (kk - i0 * g.len)) : g.kpow - ka);
         bv[i] = B0[(int64_t)min(nw + 32 * i + (lane & 31), N - 1) * g.sBn + (int64_t)ka * g.sBk];
         if (kk >= Kt) av[i] = bv[i] = 0.0f;
       }

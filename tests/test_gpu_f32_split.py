@@ -205,3 +205,45 @@ def test_captured_in_the_scratch_of_another_length(warm, T):
         assert rel_l2(host(out.rho), host(want.rho)) <= TOL
     del graph
     bd.release_stream_scratch(st)
+
+
+@pytest.mark.parametrize("T", [300, 700])
+@pytest.mark.parametrize("decay", [[0.7788, 0.5], [-0.7, 1.0], [1.02, 0.6]])
+def test_state_of_neurons_long_silent(oracle, T, decay):
+    # Neurons active at one token each: their rows of the state decay with the
+    # tokens since, down to fp32's smallest normal number and beyond.  Every
+    # value but the denormal ones keeps fp32's accuracy.
+    torch = need_gpu()
+    import burn_dragon_amd as bd
+    N, D = 160, 70
+    rng = np.random.default_rng(T)
+    q = np.zeros((1, 2, T, N), np.float32)
+    at = rng.integers(0, T, N)
+    q[:, :, at, np.arange(N)] = rng.uniform(0.5, 2.0, (1, 2, N))
+    v = rng.standard_normal((1, 1, T, D)).astype(np.float32)
+    d = np.asarray(decay, np.float32)
+    announce("f32 split, long silent neurons", T, decay)
+    out = bd.try_fused_recurrent_attention(dev(torch, q), dev(torch, v), None, dev(torch, d))
+    torch.cuda.synchronize()
+    want = q.astype(np.float64).transpose(0, 1, 3, 2) * d.astype(np.float64)[:, None, None] ** (T - np.arange(T)) @ v
+    got = out.rho.cpu().numpy()
+    ok = np.abs(want) >= 2.0 ** -125
+    # (Two powers of d, two products and a sum in fp32: 8 roundings of at most an ulp or so.)
+    np.testing.assert_allclose(got[ok], want[ok], rtol=8 * 2.0 ** -23)
+    assert np.all(np.abs(got[~ok]) <= 2.0 ** -124)
+
+
+def test_decayed_sums_past_the_scaled_range(oracle):
+    # The decayed operand is multiplied by 2^40: sums above 2^88 leave fp32's
+    # range so scaled, and are computed again.
+    torch = need_gpu()
+    import burn_dragon_amd as bd
+    B, H, T, N, D = 1, 2, 600, 96, 70
+    rng = np.random.default_rng(5)
+    q = rng.standard_normal((B, H, T, N)).astype(np.float32) * np.float32(2.0 ** 50)
+    v = rng.standard_normal((B, 1, T, D)).astype(np.float32) * np.float32(2.0 ** 50)
+    d = np.array([0.99, 0.9], np.float32)
+    announce("f32 split, decayed sums past the scaled range")
+    rho = bd.try_fused_recurrent_attention(dev(torch, q), dev(torch, v), None, dev(torch, d)).rho
+    torch.cuda.synchronize()
+    assert rel_l2(host(rho), oracle.recurrent_f64(q, v, None, d)[1]) <= TOL
